@@ -1070,8 +1070,8 @@ def main():
             "unit": "GB/s",
             "frac": achieved / profiling.L2_PEAK_GBS,
             "traffic": traffic,
-            "kernel": {"stream512_chunked": "k_knn_stream512", "stream512": "k_knn_stream512",
-                       "inner": "k_knn_stream512", "stream1024": "k_knn_stream1024",
+            "kernel": {"stream512_chunked": "k_knn_stream<512>", "stream512": "k_knn_stream<512>",
+                       "inner": "k_knn_stream<512>", "stream1024": "k_knn_stream<1024>",
                        "two_pass": "k_knn_two_pass"}.get(vname, vname)
                       + f" (variant {vname}, cell {frac:.3f}r; fused gather + radiance, cell-ordered queries)",
             "kernel_ms": gather_ms,

@@ -62,6 +62,14 @@ struct KnnParams {
     float* rgb;  // 3 planes of nq (radiance only)
     int remap;
     int h;  // inner box half-width in cells (0: walk the whole box at once)
+    // Streaming gathers: wave u of n_waves takes the queries at u,
+    // u + n_waves, ... (at most gq) of the processing order. nr > 0: the first walked box (the inner one, or the
+    // whole) has at most nr = (2 w + 1)^2 rows, gq nr <= 64, and one lane
+    // works out each row of all the wave's queries; nr = 0 (Morton, or more
+    // than 64 rows): gq = 1 and the rows are taken 64 at a time.
+    int nr, w, gq;
+    uint32_t n_waves;
+    uint32_t xcd_shift;  // log2 of the workgroups in an XCD's chunk (remap 2)
     // (nullable) the query count on the device, at most nq: positions past
     // it are skipped; nq stays the planes' stride
     const uint32_t* nq_dev;
@@ -145,45 +153,53 @@ __device__ __forceinline__ void small_divmod(int s, int d, float rd, int& q, int
     r = s - q * d;
 }
 
+// The run of one (y, z) row (linear layout) over the cells [xlo, xhi] that
+// can hold a photon within the bound T.
+__device__ __forceinline__ bool row_cells(const GridGeom& G, const uint32_t* __restrict__ starts,
+                                          const uint32_t* __restrict__ sizes, int y, int z, int xlo, int xhi, float qx,
+                                          float qy, float qz, float T, uint32_t& b, uint32_t& len) {
+    const float thr = T * 1.001f;
+    const float gy = axis_gap(qy, y, G.g[1], G.mn[1], G.cell), gz = axis_gap(qz, z, G.g[2], G.mn[2], G.cell);
+    const float dyz2 = gy * gy + gz * gz;
+    if (!(dyz2 <= thr)) return false;
+    // (the hardware square root: its ulp is far inside the margins)
+    const float dx = __builtin_amdgcn_sqrtf(thr - dyz2 + 1e-3f * T);
+    const float e = (fabsf(qx) + dx) * 1e-6f;
+    int xl, xh;
+    cell_bounds(qx - dx - e, qx + dx + e, G.mn[0], __builtin_amdgcn_rcpf(G.cell), G.g[0], xl, xh);
+    xl = max(xlo, xl);
+    xh = min(xhi, xh);
+    if (xl > xh) return false;
+    const uint32_t c0 = pmd::cell_index(G, xl, y, z);
+    const uint32_t c1 = c0 + (uint32_t)(xh - xl);
+    b = starts[c0];
+    len = starts[c1] + sizes[c1] - b;
+    return true;
+}
+
 __device__ __forceinline__ bool row_span(const GridGeom& G, const uint32_t* __restrict__ starts,
                                          const uint32_t* __restrict__ sizes, const Box& B, int s, float qx, float qy,
                                          float qz, float T, uint32_t& b, uint32_t& len) {
-    const int nx = B.hi[0] - B.lo[0] + 1, ny = B.hi[1] - B.lo[1] + 1, nz = B.hi[2] - B.lo[2] + 1;
-    const float thr = T * 1.001f;
+    const int nx = B.hi[0] - B.lo[0] + 1, ny = B.hi[1] - B.lo[1] + 1;
     b = 0;
     len = 0;
     if (G.layout == PM_LAYOUT_LINEAR) {
+        const int nz = B.hi[2] - B.lo[2] + 1;
         int zi, yi;
         if (ny * nz < (1 << 20))
             small_divmod(s, ny, __builtin_amdgcn_rcpf((float)ny), zi, yi);
         else
             zi = s / ny, yi = s % ny;
-        const int y = B.lo[1] + yi, z = B.lo[2] + zi;
-        const float gy = axis_gap(qy, y, G.g[1], G.mn[1], G.cell), gz = axis_gap(qz, z, G.g[2], G.mn[2], G.cell);
-        const float dyz2 = gy * gy + gz * gz;
-        if (!(dyz2 <= thr)) return false;
-        // (the hardware square root: its ulp is far inside the margins)
-        const float dx = __builtin_amdgcn_sqrtf(thr - dyz2 + 1e-3f * T);
-        const float e = (fabsf(qx) + dx) * 1e-6f;
-        int xl, xh;
-        cell_bounds(qx - dx - e, qx + dx + e, G.mn[0], __builtin_amdgcn_rcpf(G.cell), G.g[0], xl, xh);
-        xl = max(B.lo[0], xl);
-        xh = min(B.hi[0], xh);
-        if (xl > xh) return false;
-        const uint32_t c0 = pmd::cell_index(G, xl, y, z);
-        const uint32_t c1 = c0 + (uint32_t)(xh - xl);
-        b = starts[c0];
-        len = starts[c1] + sizes[c1] - b;
-    } else {
-        const int x = B.lo[0] + s % nx, t = s / nx;
-        const int y = B.lo[1] + t % ny, z = B.lo[2] + t / ny;
-        const float gx = axis_gap(qx, x, G.g[0], G.mn[0], G.cell), gy = axis_gap(qy, y, G.g[1], G.mn[1], G.cell),
-                    gz = axis_gap(qz, z, G.g[2], G.mn[2], G.cell);
-        if (!(gx * gx + gy * gy + gz * gz <= thr)) return false;
-        const uint32_t c = pmd::cell_index(G, x, y, z);
-        b = starts[c];
-        len = sizes[c];
+        return row_cells(G, starts, sizes, B.lo[1] + yi, B.lo[2] + zi, B.lo[0], B.hi[0], qx, qy, qz, T, b, len);
     }
+    const int x = B.lo[0] + s % nx, t = s / nx;
+    const int y = B.lo[1] + t % ny, z = B.lo[2] + t / ny;
+    const float gx = axis_gap(qx, x, G.g[0], G.mn[0], G.cell), gy = axis_gap(qy, y, G.g[1], G.mn[1], G.cell),
+                gz = axis_gap(qz, z, G.g[2], G.mn[2], G.cell);
+    if (!(gx * gx + gy * gy + gz * gz <= T * 1.001f)) return false;
+    const uint32_t c = pmd::cell_index(G, x, y, z);
+    b = starts[c];
+    len = sizes[c];
     return true;
 }
 
@@ -258,8 +274,66 @@ __device__ __forceinline__ void walk(const KnnParams& P, uint32_t lane, const Bo
 // step. The cursor (step start, next run, its start) is wave-uniform, in
 // SGPRs. f(am, sa, d2a, bm, sb, d2b): am / bm are the lane masks of the
 // lanes that hold a candidate (wave-uniform, SGPRs); d2 is computed on every
-// lane. Rows and their cells are pruned against Trow (T, or a smaller bound
-// when only keys below it can be kept).
+// lane.
+//
+// walk_runs: the runs held by the lanes in the mask `rows`, end = the run's
+// end in the stream (the next run's start) and d4 = 4 (b - its start)
+// (mod 2^32); total = the stream's length (> 0: at least one run).
+template <class F>
+__device__ __forceinline__ void walk_runs(__amdgpu_buffer_rsrc_t rx, __amdgpu_buffer_rsrc_t ry,
+                                          __amdgpu_buffer_rsrc_t rz, uint32_t lane, uint64_t rows, uint32_t d4,
+                                          uint32_t end, uint32_t total, float qx, float qy, float qz, F&& f) {
+    const int ilane = (int)lane;
+    const uint32_t lane4 = lane * 4u;
+    // the first non-empty run starts the stream at 0
+    uint32_t nstart = 0, cur = 0;
+    struct Step {
+        int left;  // stream positions left from the step's first
+        uint32_t oa, ob;
+        float xa, ya, za, xb, yb, zb;
+    };
+    // offsets and positions of the step at p; the runs starting before
+    // p + 128 are entered (lanes at or past a run's start take its offset)
+    auto load = [&](Step& w, uint32_t p) {
+        uint32_t da = cur, db = cur;
+        while (rows && nstart < p + 128u) {
+            const int j = __builtin_ctzll(rows);
+            rows &= rows - 1;
+            const uint32_t dj = __builtin_amdgcn_readlane(d4, j);
+            const int t0 = (int)(nstart - p);
+            da = ilane >= t0 ? dj : da;
+            db = ilane >= t0 - 64 ? dj : db;
+            cur = dj;
+            nstart = __builtin_amdgcn_readlane(end, j);
+        }
+        w.left = (int)(total - p);
+        w.oa = da + lane4 + p * 4u;
+        w.ob = db + lane4 + p * 4u + 256u;
+        w.xa = bload(rx, w.oa), w.ya = bload(ry, w.oa), w.za = bload(rz, w.oa);
+        w.xb = bload(rx, w.ob), w.yb = bload(ry, w.ob), w.zb = bload(rz, w.ob);
+    };
+    // Two register sets: each half of the loop body loads the next step
+    // into one set while the other is processed, so nothing is copied.
+    Step s0, s1;
+    uint32_t p = 0;
+    load(s0, 0);
+    auto half = [&](const Step& c, Step& nxt) -> bool {
+        const uint32_t pn = p + 128u;
+        const bool more = pn < total;
+        if (more) load(nxt, pn);
+        // (each mask is one lane compare's ballot)
+        f(wballot(ilane < c.left), c.oa >> 2, dist2(c.xa, c.ya, c.za, qx, qy, qz), wballot(ilane + 64 < c.left),
+          c.ob >> 2, dist2(c.xb, c.yb, c.zb, qx, qy, qz));
+        p = pn;
+        return more;
+    };
+    while (half(s0, s1) && half(s1, s0)) {
+    }
+}
+
+// walk_runs over the box B, 64 rows (Morton: cells) at a time; rows and
+// their cells are pruned against Trow (T, or a smaller bound when only keys
+// below it can be kept).
 template <class F>
 __device__ __forceinline__ void walk2(const KnnParams& P, uint32_t lane, const Box& B, float qx, float qy, float qz,
                                       float Trow, F&& f) {
@@ -267,62 +341,14 @@ __device__ __forceinline__ void walk2(const KnnParams& P, uint32_t lane, const B
     const bool linear = P.G.layout == PM_LAYOUT_LINEAR;
     const int nseg = linear ? ny * nz : nx * ny * nz;
     const __amdgpu_buffer_rsrc_t rx = plane_rsrc(P.px, P.n), ry = plane_rsrc(P.py, P.n), rz = plane_rsrc(P.pz, P.n);
-    const int ilane = (int)lane;
-    const uint32_t lane4 = lane * 4u;
     for (int sbase = 0; sbase < nseg; sbase += 64) {
-        const int s = sbase + ilane;
+        const int s = sbase + (int)lane;
         uint32_t b = 0, len = 0;
         if (s < nseg) row_span(P.G, P.starts, P.sizes, B, s, qx, qy, qz, Trow, b, len);
         const uint32_t incl = wave_incl_scan(len, lane);
         const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
         if (total == 0) continue;
-        const uint32_t pre = incl - len;
-        const uint32_t d4 = (b - pre) * 4u;  // mod 2^32: (d4 + 4 t) is 4 x slot
-        uint64_t rows = wballot(len > 0);
-        // the first non-empty run starts the stream at 0
-        uint32_t nstart = 0, cur = 0;
-        struct Step {
-            int left;  // stream positions left from the step's first
-            uint32_t oa, ob;
-            float xa, ya, za, xb, yb, zb;
-        };
-        // offsets and positions of the step at p; the runs starting before
-        // p + 128 are entered (lanes at or past a run's start take its offset)
-        auto load = [&](Step& w, uint32_t p) {
-            uint32_t da = cur, db = cur;
-            while (rows && nstart < p + 128u) {
-                const int j = __builtin_ctzll(rows);
-                rows &= rows - 1;
-                const uint32_t dj = __builtin_amdgcn_readlane(d4, j);
-                const int t0 = (int)(nstart - p);
-                da = ilane >= t0 ? dj : da;
-                db = ilane >= t0 - 64 ? dj : db;
-                cur = dj;
-                nstart = rows ? __builtin_amdgcn_readlane(pre, __builtin_ctzll(rows)) : 0xffffffffu;
-            }
-            w.left = (int)(total - p);
-            w.oa = da + lane4 + p * 4u;
-            w.ob = db + lane4 + p * 4u + 256u;
-            w.xa = bload(rx, w.oa), w.ya = bload(ry, w.oa), w.za = bload(rz, w.oa);
-            w.xb = bload(rx, w.ob), w.yb = bload(ry, w.ob), w.zb = bload(rz, w.ob);
-        };
-        // Two register sets: each half of the loop body loads the next step
-        // into one set while the other is processed, so nothing is copied.
-        Step s0, s1;
-        uint32_t p = 0;
-        load(s0, 0);
-        auto half = [&](const Step& c, Step& nxt) -> bool {
-            const uint32_t pn = p + 128u;
-            const bool more = pn < total;
-            if (more) load(nxt, pn);
-            // (each mask is one lane compare's ballot)
-            f(wballot(ilane < c.left), c.oa >> 2, dist2(c.xa, c.ya, c.za, qx, qy, qz), wballot(ilane + 64 < c.left),
-              c.ob >> 2, dist2(c.xb, c.yb, c.zb, qx, qy, qz));
-            p = pn;
-            return more;
-        };
-        while (half(s0, s1) && half(s1, s0)) {
-        }
+        walk_runs(rx, ry, rz, lane, wballot(len > 0), (b + len - incl) * 4u, incl, total, qx, qy, qz, f);
     }
 }
 
@@ -406,9 +432,18 @@ __device__ __forceinline__ void sort_and_emit(const KnnParams& P, WaveLds<CAP>& 
     if (P.rgb) radiance_epilogue<R>(P, v, m, lane, q);
 }
 
+// Largest d2 of the m keys in the LDS buffer.
+template <int CAP>
+__device__ __forceinline__ float buffer_dmax(const WaveLds<CAP>& L, uint32_t lane, uint32_t m) {
+    float d = 0.f;
+    for (uint32_t e = lane; e < m; e += 64) d = fmaxf(d, __uint_as_float((uint32_t)(L.buf[e] >> 32)));
+    return wave_max_nonneg_f32(d);
+}
+
 // Radiance estimate (Raytracer.cuh:110-138) over the m kept keys left in
-// the LDS buffer, unsorted: the filter radius is their largest distance and
-// the sum runs in buffer order (lane-strided, then a wave reduction).
+// the LDS buffer, unsorted: the filter radius is their largest distance
+// (dmax = its square) and the sum runs in buffer order (lane-strided, then a
+// wave reduction of the three channels together).
 //
 // The filter weight w = alpha (1 - (1 - e^{-beta d^2 / (2 r^2)}) / (1 - e^{-beta}))
 // is evaluated as A + B e^{x} with x = d^2 (-beta / (2 r^2)) from the squared
@@ -417,89 +452,88 @@ __device__ __forceinline__ void sort_and_emit(const KnnParams& P, WaveLds<CAP>& 
 // from the hardware square root and reciprocal; against the reference's FP32
 // sequence of square roots, divisions and expf this moves the estimate by a
 // few 1e-7 relative, inside its 1e-5 bound. The cos > 0 test keeps the
-// reference's rounding.
+// reference's rounding. The six power and direction planes are read as raw
+// buffers with one 32-bit offset per lane.
 template <int CAP>
 __device__ __forceinline__ void radiance_buffer(const KnnParams& P, const WaveLds<CAP>& L, uint32_t lane, uint32_t q,
-                                                uint32_t m) {
+                                                uint32_t m, float dmax) {
     const float alpha = 1.818f, beta = 1.953f;
     const float pi_f = 3.141592654f;
     // 1 / (1 - e^{-beta}) and log2(e), rounded to FP32
     const float inv_denom = 1.16529458f, log2e = 1.44269504f;
-    float dmax = 0.f;
-    for (uint32_t e = lane; e < m; e += 64) dmax = fmaxf(dmax, __uint_as_float((uint32_t)(L.buf[e] >> 32)));
-    dmax = wave_max_nonneg_f32(dmax);
     // hardware square root and reciprocals (a few 1e-7 relative on the
     // estimate, inside its 1e-5 bound)
     const float rmax = __builtin_amdgcn_sqrtf(dmax);
+    const float filter_r = __fmul_rn(rmax, rmax);
     float res0 = 0.f, res1 = 0.f, res2 = 0.f;
     if (m > 0) {
-        const float filter_r = __fmul_rn(rmax, rmax);
         // x log2(e) = d^2 * s
         const float s = -beta * __builtin_amdgcn_rcpf(2.f * filter_r) * log2e;
         const float wa = alpha * (1.f - inv_denom), wb = alpha * inv_denom;
         const float nx = P.nrm[q], ny = P.nrm[P.nq + q], nz = P.nrm[2 * (size_t)P.nq + q];
-        for (uint32_t e = lane; e < m; e += 64) {
-            const uint64_t v = L.buf[e];
-            const uint32_t idx = (uint32_t)v;
-            // power is read with the direction (one memory round trip),
-            // and used only where the photon faces the surface
-            const float dx = P.dir[idx], dy = P.dir[P.n + idx], dz = P.dir[2 * (size_t)P.n + idx];
-            const float p0 = P.power[idx], p1 = P.power[P.n + idx], p2 = P.power[2 * (size_t)P.n + idx];
-            const float cosNL = __fadd_rn(__fadd_rn(__fmul_rn(nx, -dx), __fmul_rn(ny, -dy)), __fmul_rn(nz, -dz));
-            if (cosNL > 0.f) {
-                const float w = wa + wb * __builtin_amdgcn_exp2f(__uint_as_float((uint32_t)(v >> 32)) * s);
-                res0 += p0 * w;
-                res1 += p1 * w;
-                res2 += p2 * w;
+        const __amdgpu_buffer_rsrc_t rd0 = plane_rsrc(P.dir, P.n), rd1 = plane_rsrc(P.dir + P.n, P.n),
+                                     rd2 = plane_rsrc(P.dir + 2 * (size_t)P.n, P.n);
+        const __amdgpu_buffer_rsrc_t rp0 = plane_rsrc(P.power, P.n), rp1 = plane_rsrc(P.power + P.n, P.n),
+                                     rp2 = plane_rsrc(P.power + 2 * (size_t)P.n, P.n);
+        for (uint32_t base = 0; base < m; base += 64) {
+            const uint32_t e = base + lane;
+            if (e < m) {
+                const uint64_t v = L.buf[e];
+                const uint32_t off = (uint32_t)v * 4u;
+                // power is read with the direction (one memory round trip),
+                // and used only where the photon faces the surface
+                const float dx = bload(rd0, off), dy = bload(rd1, off), dz = bload(rd2, off);
+                const float p0 = bload(rp0, off), p1 = bload(rp1, off), p2 = bload(rp2, off);
+                const float cosNL = __fadd_rn(__fadd_rn(__fmul_rn(nx, -dx), __fmul_rn(ny, -dy)), __fmul_rn(nz, -dz));
+                if (cosNL > 0.f) {
+                    const float w = wa + wb * __builtin_amdgcn_exp2f(__uint_as_float((uint32_t)(v >> 32)) * s);
+                    res0 += p0 * w;
+                    res1 += p1 * w;
+                    res2 += p2 * w;
+                }
             }
         }
     }
-    res0 = wave_sum_f32(res0);
-    res1 = wave_sum_f32(res1);
-    res2 = wave_sum_f32(res2);
-    if (lane == 0) {
-        float coef = 1.f;
-        if (m > 0) coef = __builtin_amdgcn_rcpf(__fmul_rn(pi_f, __fmul_rn(rmax, rmax)));
-        P.rgb[q] = m > 0 ? res0 * coef : 0.f;
-        P.rgb[P.nq + q] = m > 0 ? res1 * coef : 0.f;
-        P.rgb[2 * (size_t)P.nq + q] = m > 0 ? res2 * coef : 0.f;
+    // channel 0 in lane 15, 2 in lane 31, 1 in lane 47
+    const float tot = wave_sum3_f32(res0, res1, res2);
+    if ((lane & 15) == 15 && lane < 63) {
+        const float coef = __builtin_amdgcn_rcpf(__fmul_rn(pi_f, __fmul_rn(rmax, rmax)));
+        const uint32_t plane = lane == 15 ? 0u : lane == 31 ? 2u : 1u;
+        P.rgb[(size_t)plane * P.nq + q] = m > 0 ? tot * coef : 0.f;
     }
 }
 
-template <int CAP>
+// The end of a query: cnt keys in the buffer, all of them with d2 bits below
+// hi, hold the k nearest (or everything within the radius).
+template <int CAP, bool kLists>
 __device__ __forceinline__ void finish(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, uint32_t q, uint32_t cnt,
-                                       uint32_t found, uint64_t khi) {
+                                       uint32_t hi) {
     const uint32_t k = (uint32_t)P.k;
-    const uint32_t m = found < k ? found : k;
-    if (!P.out_idx) {
-        // no neighbour lists: narrow to exactly the k smallest and estimate
-        // from the buffer without sorting (up to 256 keys: selected from
-        // registers, the keys read once)
-        if (cnt <= 256) {
-            uint64_t v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t e = (uint32_t)j * 64 + lane;
-                v[j] = e < cnt ? L.buf[e] : ~0ull;
-            }
-            cnt = reg_select<4, CAP>(L, lane, v, cnt, k, P.bT, khi);
-        } else {
-            cnt = buf_select<CAP>(L, lane, cnt, k, k, P.bT, khi);
-        }
+    const uint32_t m = cnt < k ? cnt : k;
+    if (kLists && P.out_idx) {
+        // narrowed to the smallest sort that holds k keys (64, 128 or 256)
+        uint64_t khi = (uint64_t)hi << 32;
+        cnt = buf_select<CAP>(L, lane, cnt, k, k <= 64 ? 64u : k <= 128 ? 128u : 256u, P.bT, khi);
         wave_sync();
-        if (P.out_count && lane == 0) P.out_count[q] = m;
-        if (P.rgb) radiance_buffer<CAP>(P, L, lane, q, m);
+        if (cnt <= 64)
+            sort_and_emit<1, CAP>(P, L, lane, q, cnt, m);
+        else if (cnt <= 128)
+            sort_and_emit<2, CAP>(P, L, lane, q, cnt, m);
+        else
+            sort_and_emit<4, CAP>(P, L, lane, q, cnt, m);
         return;
     }
-    // narrowed to the smallest sort that holds k keys (64, 128 or 256)
-    cnt = buf_select<CAP>(L, lane, cnt, k, k <= 64 ? 64u : k <= 128 ? 128u : 256u, P.bT, khi);
-    wave_sync();
-    if (cnt <= 64)
-        sort_and_emit<1, CAP>(P, L, lane, q, cnt, m);
-    else if (cnt <= 128)
-        sort_and_emit<2, CAP>(P, L, lane, q, cnt, m);
+    // no neighbour lists: narrow to exactly the k smallest and estimate
+    // from the buffer without sorting
+    if (P.out_count && lane == 0) P.out_count[q] = m;
+    if (!P.rgb) return;
+    float dmax;
+    if (cnt > k)
+        dmax = lin_select<CAP>(L, lane, cnt, k, hi, P.bT);
     else
-        sort_and_emit<4, CAP>(P, L, lane, q, cnt, m);
+        dmax = buffer_dmax<CAP>(L, lane, m);
+    wave_sync();
+    radiance_buffer<CAP>(P, L, lane, q, m, dmax);
 }
 
 // The candidate box of query q: its cell +- rc, clamped (PhotonGrid.cu:262-272).
@@ -520,19 +554,28 @@ __device__ __forceinline__ void box_of(const KnnParams& P, uint32_t q, Box& B, f
     }
 }
 
-// XCD-chunked order: XCD x takes chunks x, x + 8, ... of kXcdChunk
-// consecutive workgroups (the grid is rounded up to a multiple of 8 chunks).
-constexpr uint32_t kXcdChunk = 256;
-__device__ __forceinline__ uint32_t xcd_chunked(uint32_t b) {
+// XCD-chunked order: XCD x takes chunks x, x + 8, ... of 2^shift consecutive
+// workgroups (the grid is rounded up to a multiple of 8 chunks).
+constexpr uint32_t kXcdChunk = 256;  // queries / 4 in a chunk, at most
+__device__ __forceinline__ uint32_t xcd_chunked(uint32_t b, uint32_t shift) {
     const uint32_t x = b % 8, i = b / 8;
-    return ((i / kXcdChunk) * 8 + x) * kXcdChunk + (i % kXcdChunk);
+    return ((((i >> shift) * 8 + x)) << shift) + (i & ((1u << shift) - 1u));
 }
+// The chunk of a launch of nblk workgroups of gq queries a wave: about
+// kXcdChunk x 4 queries, and no more than leaves every XCD one (a small
+// launch is not padded by more than 8 workgroups a chunk).
+inline uint32_t xcd_shift_for(uint32_t nblk, uint32_t gq) {
+    uint32_t s = 0;
+    while ((2u << s) * gq <= kXcdChunk && (uint64_t)(16u << s) <= nblk) ++s;
+    return s;
+}
+inline uint32_t xcd_round(uint32_t nblk, uint32_t shift) { return pm::div_up(nblk, 8u << shift) * (8u << shift); }
 
 // Query of this wave in a one-wave-per-query launch (XCD-aware block order,
 // optional processing order); false past the end (wave-uniform).
 __device__ __forceinline__ bool query_of_wave(const KnnParams& P, uint32_t& q) {
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t blk = P.remap == 2 ? xcd_chunked(blockIdx.x)
+    const uint32_t blk = P.remap == 2 ? xcd_chunked(blockIdx.x, P.xcd_shift)
                          : P.remap   ? pmd::xcd_remap(blockIdx.x, gridDim.x)
                                      : blockIdx.x;
     const uint32_t ql = blk * kWaves + wave;
@@ -541,98 +584,28 @@ __device__ __forceinline__ bool query_of_wave(const KnnParams& P, uint32_t& q) {
     return true;
 }
 
-// One step of the streaming selection over two candidates per lane (index
-// sa / sb, squared distance d2a / d2b, lanes holding one: masks am / bm):
-// appends the keys below the acceptance bound khi to the LDS buffer, and
-// narrows the buffer first when the step would overflow it. khi never
-// exceeds (bits(T) + 1) << 32, so a key below it is within the radius (d2
-// >= 0: its bits order as its value; a NaN d2 is above every bound). Every
-// predicate is a ballot of a plain compare combined in SGPRs; the writing
-// lanes come back from their mask.
-template <int CAP>
-__device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, uint32_t k, uint32_t bT, uint64_t am,
-                                      uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b, uint32_t& cnt,
-                                      uint64_t& khi) {
-    const uint64_t ka = make_key(d2a, sa), kb = make_key(d2b, sb);
-    uint64_t bala = am & wballot(ka < khi), balb = bm & wballot(kb < khi);
-    uint32_t na = (uint32_t)__popcll(bala), nb = (uint32_t)__popcll(balb);
-    if (cnt + na + nb > (uint32_t)CAP) {
-        // leaves at most CAP / 2 keys, room for this step's 128
-        wave_sync();
-        cnt = buf_select<CAP>(L, lane, cnt, k, CAP / 2, bT, khi);
-        bala = am & wballot(ka < khi);
-        balb = bm & wballot(kb < khi);
-        na = (uint32_t)__popcll(bala);
-        nb = (uint32_t)__popcll(balb);
-    }
-    if (__builtin_amdgcn_inverse_ballot_w64(bala)) L.buf[cnt + mbcnt(bala)] = ka;
-    if (__builtin_amdgcn_inverse_ballot_w64(balb)) L.buf[cnt + na + mbcnt(balb)] = kb;
-    cnt += na + nb;
+// A kernel parameter record read by scalar loads where it is used: from the
+// launch's own argument segment, or a batch's job table. `opaque` keeps a
+// use's loads from being hoisted (and held in SGPRs) across what is before
+// it.
+typedef const __attribute__((address_space(4))) KnnParams* ParamsPtr;
+__device__ __forceinline__ ParamsPtr opaque(ParamsPtr p) {
+    asm volatile("" : "+s"(p));
+    return p;
 }
-
-// Per-query set-up of the streaming gather: the query's position (x, y,
-// z: set by the caller, wave-uniform), its cell, and with the inner box the
-// d2 bits below which a key is closer than every photon outside it (less a
-// few ulps of rounding: every such photon has d2 >= gap^2). The three axes
-// are worked side by side in lanes 0..2 (the cell hash's division and the
-// inner box's two face gaps, each axis by the same formulas as one at a
-// time) and read back; the gap is the exact minimum over the axes.
-struct QSetup {
-    uint32_t q;
-    float x, y, z;
-    int c[3];
-    uint32_t gbits;
-};
-__device__ __forceinline__ void query_setup(const KnnParams& P, QSetup& S, uint32_t lane) {
-    // (the query's coordinates and the per-axis grid values are taken as
-    // wave-uniform values first, so the lane selects below stay selects and
-    // never become an indexed load from memory)
-    const float mn0 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.G.mn[0])));
-    const float mn1 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.G.mn[1])));
-    const float mn2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.G.mn[2])));
-    const int g0 = __builtin_amdgcn_readfirstlane(P.G.g[0]), g1 = __builtin_amdgcn_readfirstlane(P.G.g[1]),
-              g2 = __builtin_amdgcn_readfirstlane(P.G.g[2]);
-    const float x = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S.x)));
-    const float y = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S.y)));
-    const float z = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(S.z)));
-    const int a = lane < 3u ? (int)lane : 0;
-    const float v = a == 0 ? x : a == 1 ? y : z;
-    const float mn = a == 0 ? mn0 : a == 1 ? mn1 : mn2;
-    const int g = a == 0 ? g0 : a == 1 ? g1 : g2;
-    const int c = pmd::cell_coord(v, mn, P.G.cell, g);
+__device__ __forceinline__ GridGeom geom_of(ParamsPtr kp) {
+    GridGeom G;
 #pragma unroll
-    for (int i = 0; i < 3; ++i) S.c[i] = __builtin_amdgcn_readlane(c, i);
-    S.gbits = 0u;
-    if (P.h > 0) {
-        const int lo = max(0, c - P.h), hi = min(g - 1, c + P.h);
-        const uint32_t gb = __float_as_uint(inner_gap(v, lo, hi, g, mn, P.G.cell));
-        const float gap = fminf(fminf(__uint_as_float(__builtin_amdgcn_readlane(gb, 0)),
-                                      __uint_as_float(__builtin_amdgcn_readlane(gb, 1))),
-                                __uint_as_float(__builtin_amdgcn_readlane(gb, 2)));
-        S.gbits = min(__float_as_uint(gap * gap * 0.999f), __float_as_uint(P.T) + 1u);
+    for (int a = 0; a < 3; ++a) {
+        G.mn[a] = kp->G.mn[a];
+        G.g[a] = kp->G.g[a];
     }
+    G.cell = kp->G.cell;
+    G.layout = kp->G.layout;
+    return G;
 }
-
-// Single pass: in-radius keys stream into an LDS buffer of CAP keys; when it
-// would overflow, buf_select keeps only the smallest bin range holding >= k
-// keys and tightens the acceptance bound. Exact: a dropped key has >= k kept
-// keys below it.
-//
-// With P.h > 0 the walk first covers only the inner box (the query's cell
-// +- h). If that finds at least k keys within the radius and the k-th
-// smallest of them is closer than every photon outside the inner box can
-// be, those k keys are the answer (m = k); otherwise the query walks the
-// whole box again from an empty buffer. Both outcomes are exact.
-// The finish's parameters, re-read where P came from (scalar loads) instead
-// of kept in SGPRs across the walk: kFrom = kFromArgs when P is the launch's
-// own kernel argument (at offset 0 of the argument segment), kFromRecord
-// when P was loaded from the record src; kFromNone uses P.
-constexpr int kFromNone = 0, kFromArgs = 1, kFromRecord = 2;
-template <class Ptr>
-__device__ __forceinline__ void finish_params(KnnParams& Pf, Ptr kp) {
-    // (a pointer the compiler cannot see through, so the loads stay here;
-    // every field the finish reads is taken from it)
-    asm volatile("" : "+s"(kp));
+// the finish's parameters (every field it reads)
+__device__ __forceinline__ void finish_params(KnnParams& Pf, ParamsPtr kp) {
     Pf.k = kp->k;
     Pf.n = kp->n;
     Pf.nq = kp->nq;
@@ -646,104 +619,218 @@ __device__ __forceinline__ void finish_params(KnnParams& Pf, Ptr kp) {
     Pf.out_count = kp->out_count;
 }
 
-template <int CAP, int kFrom = kFromNone>
-__device__ __forceinline__ void stream_core(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, const QSetup& S,
-                                            const KnnParams* src = nullptr) {
-    const uint32_t q = S.q;
-    const float qx = S.x, qy = S.y, qz = S.z;
-    const float T = P.T;
-    const uint32_t k = (uint32_t)P.k;
-    // the candidate box: the query's cell +- rc, clamped (PhotonGrid.cu:262-272)
-    Box B;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        B.lo[a] = max(0, S.c[a] - P.rc);
-        B.hi[a] = min(P.G.g[a] - 1, S.c[a] + P.rc);
+// One step of the streaming selection over two candidates per lane (index
+// sa / sb, squared distance d2a / d2b, lanes holding one: masks am / bm):
+// appends the keys whose d2 bits lie below the acceptance bound hi to the
+// LDS buffer, and narrows the buffer first when the step would overflow it.
+// hi never exceeds bits(T) + 1, so an accepted key is within the radius (d2
+// >= 0: its bits order as its value; a NaN d2 is above every bound). A
+// narrowing's bound on whole keys is rounded up to d2 bits: the keys this
+// lets in besides lie above k kept ones, and are dropped by the finish.
+// Every predicate is a ballot of a plain compare combined in SGPRs; the
+// writing lanes come back from their mask.
+template <int CAP>
+__device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr kp0, uint64_t am, uint32_t sa,
+                                      float d2a, uint64_t bm, uint32_t sb, float d2b, uint32_t& cnt, uint32_t& hi) {
+    uint64_t bala = am & wballot(__float_as_uint(d2a) < hi), balb = bm & wballot(__float_as_uint(d2b) < hi);
+    uint32_t na = (uint32_t)__popcll(bala), nb = (uint32_t)__popcll(balb);
+    if (cnt + na + nb > (uint32_t)CAP) {
+        // leaves at most CAP / 2 keys, room for this step's 128
+        wave_sync();
+        ParamsPtr kp = opaque(kp0);
+        uint64_t khi = (uint64_t)hi << 32;
+        cnt = buf_select<CAP>(L, lane, cnt, (uint32_t)kp->k, CAP / 2, kp->bT, khi);
+        hi = (uint32_t)((khi + 0xffffffffull) >> 32);
+        bala = am & wballot(__float_as_uint(d2a) < hi);
+        balb = bm & wballot(__float_as_uint(d2b) < hi);
+        na = (uint32_t)__popcll(bala);
+        nb = (uint32_t)__popcll(balb);
     }
-    // the inner box (the query's cell +- h) first when asked for
-    Box W = B;
-    const uint32_t gbits = S.gbits;
-    bool inner = P.h > 0;
-    if (inner) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            W.lo[a] = max(0, S.c[a] - P.h);
-            W.hi[a] = min(P.G.g[a] - 1, S.c[a] + P.h);
+    // (the sum is pinned ahead of the lane branches: computed in both arms of
+    // one it would come back as a per-lane value, and the count, the branch
+    // above and the whole loop with it)
+    const uint32_t cb = __builtin_amdgcn_readfirstlane(cnt + na);
+    if (__builtin_amdgcn_inverse_ballot_w64(bala)) L.buf[cnt + mbcnt(bala)] = make_key(d2a, sa);
+    if (__builtin_amdgcn_inverse_ballot_w64(balb)) L.buf[cb + mbcnt(balb)] = make_key(d2b, sb);
+    cnt = cb + nb;
+}
+
+// Single pass: in-radius keys stream into an LDS buffer of CAP keys; when it
+// would overflow, buf_select keeps only the smallest bin range holding >= k
+// keys and tightens the acceptance bound. Exact: a dropped key has >= k kept
+// keys below it.
+//
+// With h > 0 the walk first covers only the inner box (the query's cell
+// +- h), and only keys closer than every photon outside it are kept (its
+// squared face gap less a few ulps of rounding). If that finds at least k
+// keys, the k smallest are the answer; otherwise the query walks the whole
+// box again from an empty buffer. Both outcomes are exact.
+//
+// One wave, the nqw <= gq queries at positions p0, p0 + stride, ... of
+// `order` (entries less qb; null: the positions themselves). The set-up
+// (cell, box, face gap, and the photon run of every row) is worked for all of
+// them at once, lane i nr + s taking row s of query i: it is about 230 VALU
+// instructions whatever the lanes in use, as many as one query's walk and
+// finish on a dense map. Each query then walks its rows from those lanes.
+// The stride is the launch's wave count: waves that run side by side are at
+// neighbouring queries (their cells' lines are shared in L1 and L2), and a
+// run of queries with crowded boxes (a caustic's focus) is spread over as
+// many waves as one query a wave would give it. With consecutive queries per
+// wave instead, L2 reads doubled and a frame's gathers took 2.9 ms, not 1.9.
+template <int CAP, bool kLists>
+__device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint32_t lane,
+                                            const uint32_t* __restrict__ order, uint32_t p0, uint32_t stride,
+                                            uint32_t qb, uint32_t nqw) {
+    uint32_t q, hib, d4 = 0, end = 0;
+    float x, y, z;
+    uint64_t rows_all = 0;
+    {
+        ParamsPtr kp = opaque(kp0);
+        const GridGeom G = geom_of(kp);
+        const int nr = kp->nr;
+        int i = 0, s = 0;
+        if (nr > 0) small_divmod((int)lane, nr, __builtin_amdgcn_rcpf((float)nr), i, s);
+        const bool mine = nr > 0 && (uint32_t)i < nqw;
+        const uint32_t pos = p0 + min((uint32_t)i, nqw - 1u) * stride;
+        q = (order ? order[pos] : pos) - qb;
+        x = kp->qx[q];
+        y = kp->qy[q];
+        z = kp->qz[q];
+        const int cx = pmd::cell_coord(x, G.mn[0], G.cell, G.g[0]), cy = pmd::cell_coord(y, G.mn[1], G.cell, G.g[1]),
+                  cz = pmd::cell_coord(z, G.mn[2], G.cell, G.g[2]);
+        const float T = kp->T;
+        hib = __float_as_uint(T) + 1u;
+        float Trow = T;
+        const int h = kp->h;
+        if (h > 0) {
+            const float gx = inner_gap(x, max(0, cx - h), min(G.g[0] - 1, cx + h), G.g[0], G.mn[0], G.cell),
+                        gy = inner_gap(y, max(0, cy - h), min(G.g[1] - 1, cy + h), G.g[1], G.mn[1], G.cell),
+                        gz = inner_gap(z, max(0, cz - h), min(G.g[2] - 1, cz + h), G.g[2], G.mn[2], G.cell);
+            const float gap = fminf(fminf(gx, gy), gz);
+            hib = min(__float_as_uint(gap * gap * 0.999f), hib);
+            // (only keys below the bound are kept: the rows are pruned with it)
+            Trow = fminf(T, __uint_as_float(hib));
+        }
+        if (nr > 0) {
+            const int w = kp->w, side = 2 * w + 1;
+            int zi, yi;
+            small_divmod(s, side, __builtin_amdgcn_rcpf((float)side), zi, yi);
+            const int yy = cy - w + yi, zz = cz - w + zi;
+            uint32_t b = 0, len = 0;
+            if (mine && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2])
+                row_cells(G, kp->starts, kp->sizes, yy, zz, max(0, cx - w), min(G.g[0] - 1, cx + w), x, y, z, Trow, b,
+                          len);
+            const uint32_t incl = wave_incl_scan(len, lane);
+            // each query's stream starts at 0: less the lanes before its first
+            const uint32_t before = __shfl(incl, i > 0 ? i * nr - 1 : 0, 64);
+            end = incl - (i > 0 ? before : 0u);
+            d4 = (b + len - end) * 4u;
+            rows_all = wballot(len > 0);
         }
     }
-    uint32_t cnt;
-    uint64_t khi;
-    for (;;) {
-        // the acceptance bound starts at the radius (d2 <= T), and in the
-        // inner box at gbits: only keys closer than every photon outside it
-        // are buffered there
-        cnt = 0;
-        khi = inner ? (uint64_t)gbits << 32 : (uint64_t)(__float_as_uint(T) + 1u) << 32;
-        // (the inner walk keeps only keys below gbits: its rows are pruned
-        // against that bound)
-        const float Trow = inner ? fminf(T, __uint_as_float(gbits)) : T;
-        walk2(P, lane, W, qx, qy, qz, Trow,
-              [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
-                  push2<CAP>(L, lane, k, P.bT, am, sa, d2a, bm, sb, d2b, cnt, khi);
-              });
-        wave_sync();
-        // with at least k such keys, the k smallest keys overall are among
-        // them (the buffer holds every in-radius key below its bound, or at
-        // least k of them once narrowed)
-        if (!inner || cnt >= k) break;
-        // otherwise the whole box from an empty buffer
-        W = B;
-        inner = false;
-        wave_sync();
+    for (uint32_t i = 0; i < nqw; ++i) {
+        uint32_t cnt, hi, qi;
+        {
+            ParamsPtr kp = opaque(kp0);
+            const int nr = kp->nr;
+            const uint32_t lb = i * (uint32_t)nr;
+            const float qx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lb));
+            const float qy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(y), lb));
+            const float qz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(z), lb));
+            const uint32_t n = kp->n;
+            const __amdgpu_buffer_rsrc_t rx = plane_rsrc(kp->px, n), ry = plane_rsrc(kp->py, n),
+                                         rz = plane_rsrc(kp->pz, n);
+            hi = __builtin_amdgcn_readlane(hib, lb);
+            bool batch = nr > 0, inner = kp->h > 0;
+            for (;;) {
+                cnt = 0;
+                for (int sbase = 0;; sbase += 64) {
+                    uint32_t cd4 = d4, cend = end, total;
+                    uint64_t rows;
+                    bool last = true;
+                    if (batch) {
+                        rows = rows_all & ((~0ull >> (64 - nr)) << lb);
+                        total = __builtin_amdgcn_readlane(end, lb + (uint32_t)nr - 1u);
+                    } else {
+                        // 64 rows (Morton: cells) of the box, one per lane
+                        ParamsPtr kc = opaque(kp0);
+                        const GridGeom G = geom_of(kc);
+                        const int w = inner ? kc->h : kc->rc;
+                        const float qv[3] = {qx, qy, qz};
+                        Box B;
+#pragma unroll
+                        for (int a = 0; a < 3; ++a) {
+                            const int c = __builtin_amdgcn_readfirstlane(
+                                pmd::cell_coord(qv[a], G.mn[a], G.cell, G.g[a]));
+                            B.lo[a] = max(0, c - w);
+                            B.hi[a] = min(G.g[a] - 1, c + w);
+                        }
+                        const int nx = B.hi[0] - B.lo[0] + 1, nyz = (B.hi[1] - B.lo[1] + 1) * (B.hi[2] - B.lo[2] + 1);
+                        const int nseg = G.layout == PM_LAYOUT_LINEAR ? nyz : nx * nyz;
+                        const int sr = sbase + (int)lane;
+                        const float Trow = inner ? fminf(kc->T, __uint_as_float(hi)) : kc->T;
+                        uint32_t b = 0, len = 0;
+                        if (sr < nseg) row_span(G, kc->starts, kc->sizes, B, sr, qx, qy, qz, Trow, b, len);
+                        cend = wave_incl_scan(len, lane);
+                        cd4 = (b + len - cend) * 4u;
+                        rows = wballot(len > 0);
+                        total = __builtin_amdgcn_readlane(cend, 63);
+                        last = sbase + 64 >= nseg;
+                    }
+                    if (total > 0)
+                        walk_runs(rx, ry, rz, lane, rows, cd4, cend, total, qx, qy, qz,
+                                  [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
+                                      push2<CAP>(L, lane, kp0, am, sa, d2a, bm, sb, d2b, cnt, hi);
+                                  });
+                    if (last) break;
+                }
+                wave_sync();
+                // with at least k such keys, the k smallest keys overall are
+                // among them (the buffer holds every in-radius key below its
+                // bound, or at least k of them once narrowed)
+                if (!inner) break;
+                kp = opaque(kp0);
+                if (cnt >= (uint32_t)kp->k) break;
+                // otherwise the whole box from an empty buffer
+                inner = false;
+                batch = false;
+                hi = __float_as_uint(kp->T) + 1u;
+                wave_sync();
+            }
+            qi = __builtin_amdgcn_readlane(q, lb);
+        }
+        // The count within the radius that the finish needs is min(found, k),
+        // and that is min(cnt, k): without a narrowing the buffer holds every
+        // key within the radius (cnt = found), and a narrowing keeps at least
+        // k (it starts above CAP - 128 >= k keys), so cnt >= k after one.
+        KnnParams Pf;
+        finish_params(Pf, opaque(kp0));
+        finish<CAP, kLists>(Pf, L, lane, qi, cnt, hi);
+        wave_sync();  // the buffer is read before the next query's keys
     }
-    // The count within the radius that the finish needs is min(found, k),
-    // and that is min(cnt, k): without a narrowing the buffer holds every
-    // key within the radius (cnt = found), and a narrowing keeps at least k
-    // (it starts above CAP - 128 >= k keys), so cnt >= k after one.
-    const uint32_t found = cnt;
-    if constexpr (kFrom == kFromArgs) {
-        KnnParams Pf = P;
-        finish_params(Pf, (const __attribute__((address_space(4))) KnnParams*)__builtin_amdgcn_kernarg_segment_ptr());
-        finish<CAP>(Pf, L, lane, q, cnt, found, khi);
-    } else if constexpr (kFrom == kFromRecord) {
-        KnnParams Pf = P;
-        finish_params(Pf, src);
-        finish<CAP>(Pf, L, lane, q, cnt, found, khi);
-    } else {
-        finish<CAP>(P, L, lane, q, cnt, found, khi);
-    }
 }
 
-// One query on the wave (its set-up wave-uniform).
-template <int CAP, int kFrom = kFromNone>
-__device__ __forceinline__ void stream_one(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, uint32_t q,
-                                           const KnnParams* src = nullptr) {
-    // the query is the wave's: its coordinates (and so the box, the row
-    // count and the cursor of walk) are wave-uniform, held in SGPRs
-    QSetup S;
-    S.q = q;
-    S.x = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.qx[q])));
-    S.y = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.qy[q])));
-    S.z = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.qz[q])));
-    query_setup(P, S, lane);
-    stream_core<CAP, kFrom>(P, L, lane, S, src);
+// The queries of wave u among n_waves: u, u + n_waves, ...
+__device__ __forceinline__ uint32_t wave_queries(uint32_t u, uint32_t n_waves, uint32_t gq, uint32_t nq) {
+    return min(gq, (nq - u - 1u) / n_waves + 1u);  // u < nq
 }
 
-// 512-key buffer: 17 KB of LDS per workgroup, so 7 waves per SIMD fit when
-// the registers do (68 VGPRs under this occupancy target, no spills).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_knn_stream512(KnnParams P) {
-    __shared__ WaveLds<512> lds[kWaves];
-    uint32_t q;
-    if (!query_of_wave(P, q)) return;  // wave-uniform; no workgroup barriers below
-    stream_one<512, kFromArgs>(P, lds[threadIdx.x >> 6], threadIdx.x & 63, q);
-}
-
-// 1024-key buffer: fewer refinements per query, LDS-limited to 4 waves per SIMD.
-__global__ __launch_bounds__(256) void k_knn_stream1024(KnnParams P) {
-    __shared__ WaveLds<1024> lds[kWaves];
-    uint32_t q;
-    if (!query_of_wave(P, q)) return;
-    stream_one<1024, kFromArgs>(P, lds[threadIdx.x >> 6], threadIdx.x & 63, q);
+// The single-map launch, waves in the XCD-aware order. CAP = 512: 17 KB of
+// LDS per workgroup; CAP = 1024 (fewer narrowings, k up to 512) is
+// LDS-limited to 4 waves per SIMD.
+template <int CAP, bool kLists>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : 4))) void k_knn_stream(
+    KnnParams P) {
+    __shared__ WaveLds<CAP> lds[kWaves];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t blk = P.remap == 2 ? xcd_chunked(blockIdx.x, P.xcd_shift)
+                         : P.remap   ? pmd::xcd_remap(blockIdx.x, gridDim.x)
+                                     : blockIdx.x;
+    const uint32_t nq = P.nq_dev ? min(P.nq, *P.nq_dev) : P.nq;
+    const uint32_t u = blk * kWaves + wave;
+    if (u >= nq || u >= P.n_waves) return;  // wave-uniform; no workgroup barriers below
+    stream_wave<CAP, kLists>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), lds[wave], threadIdx.x & 63, P.order,
+                             u, P.n_waves, 0u, wave_queries(u, P.n_waves, (uint32_t)P.gq, nq));
 }
 
 // Large k (257..2048, e.g. the shipped renderer's k = 2000 / 400): one wave
@@ -786,7 +873,7 @@ __device__ __forceinline__ void large_one(const KnnParams& P, WaveLds<CAP>& L, u
     wave_sync();
     if (!P.out_idx) {  // radiance / counts only: no sort needed
         if (P.out_count && lane == 0) P.out_count[q] = m;
-        if (P.rgb) radiance_buffer<CAP>(P, L, lane, q, m);
+        if (P.rgb) radiance_buffer<CAP>(P, L, lane, q, m, buffer_dmax<CAP>(L, lane, m));
         return;
     }
     uint32_t n2 = 64;
@@ -1085,13 +1172,14 @@ __global__ __launch_bounds__(256) void k_gather_wide(KnnParams P, uint32_t* __re
 }
 
 // Batched forms: the queries of many jobs (grids, radii, k) in one launch.
-// A position p maps to a flattened query index g (through the batch's
-// processing order, if any), whose job is the last one with qbase <= g.
-__device__ __forceinline__ uint32_t job_of(const uint32_t* __restrict__ qbase, uint32_t n_jobs, uint32_t g) {
+// The launch's waves are numbered job by job: job j's are wbase[j] ... ,
+// gq_j queries each, so a wave's queries are all of one job (positions
+// qbase[j] + ... of the flattened order, which is sorted by job).
+__device__ __forceinline__ uint32_t job_of(const uint32_t* __restrict__ base, uint32_t n_jobs, uint32_t g) {
     uint32_t lo = 0, hi = n_jobs;
     while (hi - lo > 1) {
         uint32_t mid = (lo + hi) >> 1;
-        if (qbase[mid] <= g)
+        if (base[mid] <= g)
             lo = mid;
         else
             hi = mid;
@@ -1099,53 +1187,54 @@ __device__ __forceinline__ uint32_t job_of(const uint32_t* __restrict__ qbase, u
     return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// One wave per position. Workgroups go to the 8 XCDs round-robin; the
-// linear workgroup id is remapped so that XCD x takes chunks x, x + 8, ...
-// of kXcdChunk consecutive workgroups: each XCD's L2 still sees runs of
-// neighbouring cells, while at any moment all XCDs work inside the same
-// region of the (job, cell) order and share the photon blocks in the MALL
-// (a contiguous eighth per XCD would put eight different jobs in flight).
-// The 2-D grid keeps every dimension's work-item count below 2^32; the
-// workgroups past the rounded-up count exit at once.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_knn_batch_grid(
-    const KnnParams* __restrict__ jobs, const uint32_t* __restrict__ qbase, uint32_t n_jobs,
-    const uint32_t* __restrict__ order, uint32_t total, uint32_t n_blocks) {
-    __shared__ WaveLds<512> lds[kWaves];
-    const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
-    if (b >= n_blocks) return;  // n_blocks is a multiple of 8 * kXcdChunk
-    const uint32_t p = xcd_chunked(b) * kWaves + (threadIdx.x >> 6);
-    if (p >= total) return;  // wave-uniform
-    const uint32_t g = order ? order[p] : p;
-    const uint32_t j = job_of(qbase, n_jobs, g);
-    const KnnParams P = jobs[j];
-    stream_one<512, kFromRecord>(P, lds[threadIdx.x >> 6], threadIdx.x & 63,
-                                 __builtin_amdgcn_readfirstlane(g - qbase[j]), jobs + j);
+template <bool kLists>
+__device__ __forceinline__ void batch_wave(const KnnParams* __restrict__ jobs, const uint32_t* __restrict__ qbase,
+                                           const uint32_t* __restrict__ wbase, uint32_t n_jobs,
+                                           const uint32_t* __restrict__ order, uint32_t u, WaveLds<512>& L) {
+    const uint32_t j = job_of(wbase, n_jobs, u);
+    ParamsPtr kp = (ParamsPtr)(jobs + j);
+    const uint32_t n_waves = kp->n_waves;
+    const uint32_t qb = __builtin_amdgcn_readfirstlane(qbase[j]);
+    const uint32_t first = __builtin_amdgcn_readfirstlane(u - wbase[j]);
+    stream_wave<512, kLists>(kp, L, threadIdx.x & 63, order, qb + first, n_waves, qb,
+                             wave_queries(first, n_waves, (uint32_t)kp->gq, kp->nq));
 }
 
-// Persistent form: workgroups stay resident and their waves take tiles of
-// kBatchTile positions from a device work counter until it passes the total.
-constexpr uint32_t kBatchTile = 4;
+// Workgroups go to the 8 XCDs round-robin; the linear workgroup id is
+// remapped so that XCD x takes chunks x, x + 8, ... of 2^shift consecutive
+// workgroups: each XCD's L2 still sees runs of neighbouring cells, while at
+// any moment all XCDs work inside the same region of the (job, cell) order
+// and share the photon blocks in the MALL (a contiguous eighth per XCD would
+// put eight different jobs in flight). The 2-D grid keeps every dimension's
+// work-item count below 2^32; the workgroups past the rounded-up count exit
+// at once.
+template <bool kLists>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(7))) void k_knn_batch_grid(
+    const KnnParams* __restrict__ jobs, const uint32_t* __restrict__ qbase, const uint32_t* __restrict__ wbase,
+    uint32_t n_jobs, const uint32_t* __restrict__ order, uint32_t n_waves, uint32_t n_blocks, uint32_t shift) {
+    __shared__ WaveLds<512> lds[kWaves];
+    const uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+    if (b >= n_blocks) return;  // n_blocks is a multiple of 8 << shift
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t u = xcd_chunked(b, shift) * kWaves + wave;
+    if (u >= n_waves) return;  // wave-uniform
+    batch_wave<kLists>(jobs, qbase, wbase, n_jobs, order, u, lds[wave]);
+}
 
-template <int CAP>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_knn_batch(const KnnParams* __restrict__ jobs, const uint32_t* __restrict__ qbase,
-                                                   uint32_t n_jobs, const uint32_t* __restrict__ order, uint32_t total,
-                                                   uint32_t* __restrict__ counter) {
-    __shared__ WaveLds<CAP> lds[kWaves];
-    const uint32_t lane = threadIdx.x & 63;
-    WaveLds<CAP>& L = lds[threadIdx.x >> 6];
+// Persistent form: workgroups stay resident and their waves take wave units
+// from a device work counter until it passes the total.
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_knn_batch(
+    const KnnParams* __restrict__ jobs, const uint32_t* __restrict__ qbase, const uint32_t* __restrict__ wbase,
+    uint32_t n_jobs, const uint32_t* __restrict__ order, uint32_t n_waves, uint32_t* __restrict__ counter) {
+    __shared__ WaveLds<512> lds[kWaves];
+    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     for (;;) {
-        uint32_t pos = 0;
-        if (lane == 0) pos = atomicAdd(counter, kBatchTile);
-        pos = __builtin_amdgcn_readfirstlane(pos);
-        if (pos >= total) break;
-        const uint32_t end = min(total, pos + kBatchTile);
-        for (uint32_t p = pos; p < end; ++p) {
-            const uint32_t g = order ? order[p] : p;
-            const uint32_t j = job_of(qbase, n_jobs, g);
-            const KnnParams P = jobs[j];
-            stream_one<CAP>(P, L, lane, __builtin_amdgcn_readfirstlane(g - qbase[j]));
-            wave_sync();
-        }
+        uint32_t u = 0;
+        if (lane == 0) u = atomicAdd(counter, 1u);
+        u = __builtin_amdgcn_readfirstlane(u);
+        if (u >= n_waves) break;
+        batch_wave<true>(jobs, qbase, wbase, n_jobs, order, u, lds[wave]);
+        wave_sync();
     }
 }
 
@@ -1197,7 +1286,10 @@ __global__ __launch_bounds__(256) void k_knn_two_pass(KnnParams P) {
         cnt += na;
     });
     wave_sync();
-    finish<CAP>(P, L, lane, q, cnt, found, khi);
+    // (khi <= (bits(T) + 1) << 32 once narrowed, else every key is within T)
+    const uint32_t top = __float_as_uint(T) + 1u;
+    const uint64_t up = khi >= (uint64_t)top << 32 ? top : (khi + 0xffffffffull) >> 32;
+    finish<CAP, true>(P, L, lane, q, cnt, (uint32_t)up);
 }
 
 // Radiance from a stored kNN result (pm_radiance): one wave per query.
@@ -1376,7 +1468,22 @@ pm_status setup(pm_ctx* ctx, const pm_grid* grid, const float* d_q, uint32_t nq,
     P.k = k;
     P.remap = (flags & PM_KNN_NO_XCD_REMAP) ? 0 : (flags & PM_KNN_XCD_CONTIGUOUS) ? 1 : 2;
     P.h = (flags & PM_KNN_INNER_BOX) ? P.rc / 2 : 0;
+    P.gq = 1;
     return PM_OK;
+}
+
+// The streaming gather's queries per wave, for a launch of `total` queries:
+// as many as their rows fit the wave's 64 lanes, while at least kFillWaves
+// waves remain (16 a SIMD's worth: below that the chip is not full and a
+// wave's queries would only run one after the other).
+constexpr uint32_t kFillWaves = 16384;
+void split_waves(KnnParams& P, uint64_t total) {
+    P.w = P.h > 0 ? P.h : P.rc;
+    const int64_t side = 2 * (int64_t)P.w + 1, rows = side * side;
+    P.nr = P.G.layout == PM_LAYOUT_LINEAR && rows <= 64 ? (int)rows : 0;
+    const uint64_t fit = P.nr > 0 ? 64 / (uint64_t)P.nr : 1;
+    P.gq = (int)std::max<uint64_t>(1, std::min<uint64_t>(fit, total / kFillWaves));
+    P.n_waves = pm::div_up(P.nq, (uint32_t)P.gq);
 }
 
 pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint32_t* order_out) {
@@ -1436,7 +1543,8 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
         pm_status st = pm::fill_u32(ctx, ovf_count, 0u, 1);
         if (st != PM_OK) return st;
         uint32_t nblk = pm::div_up(P.nq, kWaves);
-        if (P.remap == 2) nblk = pm::div_up(nblk, 8 * kXcdChunk) * 8 * kXcdChunk;
+        P.xcd_shift = xcd_shift_for(nblk, 1);
+        if (P.remap == 2) nblk = xcd_round(nblk, P.xcd_shift);
         hipLaunchKernelGGL(k_gather_wide, dim3(nblk), dim3(256), 0, ctx->stream, P, ovf_list, ovf_count);
         PM_CHECK_LAUNCH(ctx, "k_gather_wide");
         const uint32_t lblocks = std::min<uint32_t>(P.nq, (uint32_t)std::max(ctx->cu_count, 1) * 8u);
@@ -1447,32 +1555,33 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
         PM_CHECK_LAUNCH(ctx, "k_knn_large_list");
         return PM_OK;
     }
-    if (mid) {
-        uint32_t nblk = pm::div_up(P.nq, kWaves);
-        if (P.remap == 2) nblk = pm::div_up(nblk, 8 * kXcdChunk) * 8 * kXcdChunk;
-        hipLaunchKernelGGL(k_knn_stream1024, dim3(nblk), dim3(256), 0, ctx->stream, P);
-        PM_CHECK_LAUNCH(ctx, "k_knn_stream1024");
-        return PM_OK;
-    }
     if (P.k > 1024) {
         hipLaunchKernelGGL(k_knn_large<4096>, dim3(P.nq), dim3(64), 0, ctx->stream, P);
         PM_CHECK_LAUNCH(ctx, "k_knn_large");
         return PM_OK;
     }
-    if (P.k > 256) {
+    if (P.k > 256 && !mid) {
         hipLaunchKernelGGL(k_knn_large<2048>, dim3(P.nq), dim3(64), 0, ctx->stream, P);
         PM_CHECK_LAUNCH(ctx, "k_knn_large");
         return PM_OK;
     }
-    uint32_t nblk = pm::div_up(P.nq, kWaves);
-    if (P.remap == 2) nblk = pm::div_up(nblk, 8 * kXcdChunk) * 8 * kXcdChunk;
+    const bool two_pass = !mid && (flags & PM_KNN_TWO_PASS);
+    if (!two_pass) split_waves(P, P.nq);
+    uint32_t nblk = pm::div_up(two_pass ? P.nq : P.n_waves, kWaves);
+    P.xcd_shift = xcd_shift_for(nblk, (uint32_t)P.gq);
+    if (P.remap == 2) nblk = xcd_round(nblk, P.xcd_shift);
     const dim3 grid_dim(nblk), block(256);
-    if (flags & PM_KNN_TWO_PASS)
+    const bool lists = P.out_idx != nullptr;
+    if (two_pass)
         hipLaunchKernelGGL(k_knn_two_pass, grid_dim, block, 0, ctx->stream, P);
+    else if (mid || ((flags & PM_KNN_LARGE_BUFFER) && !lists))
+        hipLaunchKernelGGL((k_knn_stream<1024, false>), grid_dim, block, 0, ctx->stream, P);
     else if (flags & PM_KNN_LARGE_BUFFER)
-        hipLaunchKernelGGL(k_knn_stream1024, grid_dim, block, 0, ctx->stream, P);
+        hipLaunchKernelGGL((k_knn_stream<1024, true>), grid_dim, block, 0, ctx->stream, P);
+    else if (lists)
+        hipLaunchKernelGGL((k_knn_stream<512, true>), grid_dim, block, 0, ctx->stream, P);
     else
-        hipLaunchKernelGGL(k_knn_stream512, grid_dim, block, 0, ctx->stream, P);
+        hipLaunchKernelGGL((k_knn_stream<512, false>), grid_dim, block, 0, ctx->stream, P);
     PM_CHECK_LAUNCH(ctx, "k_knn");
     return PM_OK;
 }
@@ -1592,7 +1701,7 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     // launches of the single-map kernel, first, on the same stream.
     std::vector<KnnParams> hp;
     std::vector<std::pair<const pm_grid*, KnnParams>> large;
-    std::vector<uint32_t> qbase, cell_base;
+    std::vector<uint32_t> qbase, cell_base, wbase;
     hp.reserve(n_jobs);
     uint64_t total = 0, cells = 0;
     for (uint32_t j = 0; j < n_jobs; ++j) {
@@ -1633,11 +1742,20 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     }
     if (total == 0) return PM_OK;
     n_jobs = (uint32_t)hp.size();
+    uint64_t waves = 0;
+    bool lists = false;
+    for (KnnParams& P : hp) {
+        split_waves(P, total);
+        wbase.push_back((uint32_t)waves);
+        waves += P.n_waves;
+        lists |= P.out_idx != nullptr;
+    }
+    const uint32_t n_waves = (uint32_t)waves;  // (at most total)
     const bool sorted = (flags & PM_KNN_SORT_QUERIES) && cells <= 0xFFFFFFFFull;
     const uint32_t nt = (uint32_t)total;
     const size_t rs = sorted ? pm::radix_sort_scratch_bytes(nt) : 0;
     const size_t bytes = pm::carve_size({(size_t)n_jobs * sizeof(KnnParams), (size_t)n_jobs * 4, (size_t)n_jobs * 4,
-                                         64, sorted ? (size_t)nt * 4 : 0, sorted ? (size_t)nt * 4 : 0,
+                                         (size_t)n_jobs * 4, 64, sorted ? (size_t)nt * 4 : 0, sorted ? (size_t)nt * 4 : 0,
                                          sorted ? (size_t)nt * 4 : 0, rs});
     void* work = nullptr;
     pm_status st = pm::scratch_reserve(ctx, bytes, &work);
@@ -1646,10 +1764,12 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     KnnParams* d_jobs = cv.take<KnnParams>(n_jobs);
     uint32_t* d_qbase = cv.take<uint32_t>(n_jobs);
     uint32_t* d_cbase = cv.take<uint32_t>(n_jobs);
+    uint32_t* d_wbase = cv.take<uint32_t>(n_jobs);
     uint32_t* d_counter = cv.take<uint32_t>(16);
     PM_HIP(ctx, hipMemcpyAsync(d_jobs, hp.data(), hp.size() * sizeof(KnnParams), hipMemcpyHostToDevice, ctx->stream));
     PM_HIP(ctx, hipMemcpyAsync(d_qbase, qbase.data(), qbase.size() * 4, hipMemcpyHostToDevice, ctx->stream));
     PM_HIP(ctx, hipMemcpyAsync(d_cbase, cell_base.data(), cell_base.size() * 4, hipMemcpyHostToDevice, ctx->stream));
+    PM_HIP(ctx, hipMemcpyAsync(d_wbase, wbase.data(), wbase.size() * 4, hipMemcpyHostToDevice, ctx->stream));
     // the tables are copied from pageable host vectors: wait before they go
     PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const uint32_t* order = nullptr;
@@ -1668,16 +1788,22 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     }
     if (flags & PM_KNN_BATCH_QUEUE) {
         if ((st = pm::fill_u32(ctx, d_counter, 0u, 1)) != PM_OK) return st;
-        const uint32_t blocks = std::min<uint32_t>(pm::div_up(pm::div_up(nt, kBatchTile), kWaves),
-                                                   (uint32_t)std::max(ctx->cu_count, 1) * 8u);
-        hipLaunchKernelGGL(k_knn_batch<512>, dim3(blocks), dim3(256), 0, ctx->stream, d_jobs, d_qbase, n_jobs, order,
-                           nt, d_counter);
+        const uint32_t blocks =
+            std::min<uint32_t>(pm::div_up(n_waves, kWaves), (uint32_t)std::max(ctx->cu_count, 1) * 8u);
+        hipLaunchKernelGGL(k_knn_batch, dim3(blocks), dim3(256), 0, ctx->stream, d_jobs, d_qbase, d_wbase, n_jobs,
+                           order, n_waves, d_counter);
     } else {
-        const uint32_t step = 8 * kXcdChunk;
-        const uint32_t blocks = pm::div_up(pm::div_up(nt, kWaves), step) * step;
+        const uint32_t nblk = pm::div_up(n_waves, kWaves);
+        const uint32_t shift = xcd_shift_for(nblk, std::max(1u, nt / n_waves));
+        const uint32_t blocks = xcd_round(nblk, shift);
         const uint32_t gx = std::min<uint32_t>(blocks, 65536u);
-        hipLaunchKernelGGL(k_knn_batch_grid, dim3(gx, pm::div_up(blocks, gx)), dim3(256), 0, ctx->stream, d_jobs,
-                           d_qbase, n_jobs, order, nt, blocks);
+        const dim3 gd(gx, pm::div_up(blocks, gx));
+        if (lists)
+            hipLaunchKernelGGL(k_knn_batch_grid<true>, gd, dim3(256), 0, ctx->stream, d_jobs, d_qbase, d_wbase, n_jobs,
+                               order, n_waves, blocks, shift);
+        else
+            hipLaunchKernelGGL(k_knn_batch_grid<false>, gd, dim3(256), 0, ctx->stream, d_jobs, d_qbase, d_wbase,
+                               n_jobs, order, n_waves, blocks, shift);
     }
     PM_CHECK_LAUNCH(ctx, "k_knn_batch");
     return PM_OK;

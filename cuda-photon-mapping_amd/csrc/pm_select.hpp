@@ -27,7 +27,10 @@ inline float radius_threshold(float r) {
 
 template <int CAP>
 struct WaveLds {
-    uint32_t hist[64];
+    union {
+        uint32_t hist[64];
+        uint64_t list[32];
+    };
     uint64_t buf[CAP];
 };
 
@@ -79,6 +82,27 @@ __device__ __forceinline__ float wave_max_nonneg_f32(float v) {
     v = fmaxf(v, dpp_src<0x142, 0xa>(v));
     v = fmaxf(v, dpp_src<0x143, 0xc>(v));
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Three sums at once (no LDS): the halves of two values trade places so that
+// one add folds both (v_permlane32_swap, then v_permlane16_swap), and the
+// last four steps run on all rows of 16 lanes together. Row 0's lane 15 holds
+// the sum of a, row 1's of c, row 2's of b: 8 adds and 3 swaps against 18
+// adds for the sums one by one.
+__device__ __forceinline__ float wave_sum3_f32(float a, float b, float c) {
+    const auto u = [](float v) { return __float_as_uint(v); };
+    const auto f = [](uint32_t v) { return __uint_as_float(v); };
+    // lanes 0-31: a, lanes 32-63: b
+    const auto ab = __builtin_amdgcn_permlane32_swap(u(a), u(b), false, false);
+    const auto cc = __builtin_amdgcn_permlane32_swap(u(c), 0u, false, false);
+    const float x = f(ab[0]) + f(ab[1]), y = f(cc[0]) + f(cc[1]);
+    const auto r = __builtin_amdgcn_permlane16_swap(u(x), u(y), false, false);
+    float v = f(r[0]) + f(r[1]);
+    v += dpp_src<0x111, 0xf>(v);
+    v += dpp_src<0x112, 0xf>(v);
+    v += dpp_src<0x114, 0xf>(v);
+    v += dpp_src<0x118, 0xf>(v);
+    return v;
 }
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m) {
@@ -174,76 +198,61 @@ __device__ uint32_t buf_select(WaveLds<CAP>& L, uint32_t lane, uint32_t cnt, uin
     return out;
 }
 
-// buf_select to exactly the k smallest keys, for at most 64 R buffered keys
-// read into registers once (v[j] = entry 64 j + lane, ~0 past cnt): rounds
-// of bins like buf_select's (finer in the first), counted from the
-// registers instead of re-reading the buffer; the kept set is the same (the
-// k smallest keys, which are unique). The kept
-// keys are then written back to the buffer's front in buffer order (one
-// pass, every read already done). Returns the count kept (min(cnt, k)).
-template <int R, int CAP>
-__device__ uint32_t reg_select(WaveLds<CAP>& L, uint32_t lane, const uint64_t (&v)[R], uint32_t cnt, uint32_t k,
-                               uint32_t bT, uint64_t& khi_io) {
-    if (cnt <= k) return cnt;
-    // the first round bins four per octave (the top two mantissa bits of
-    // d2; 2 bT + 1 bounds bits(T) >> 21), so the crossing bin holds fewer
-    // keys for the rounds that split it
-    const uint32_t bT2 = (bT << 1) | 1u;
+// buf_select to exactly the k smallest of the cnt > k keys, whose d2 bits all
+// lie below hi; returns the k-th smallest's d2. One histogram of 64 bins
+// linear in d2 (photons on surfaces fall evenly in d2, so the bin of the
+// k-th holds a few keys: the mapping is monotone however it rounds), one
+// in-place compaction of the keys in the bins below, and the crossing bin's
+// keys ranked against each other. A crossing bin of more than 32 keys
+// (duplicates, extreme clusters) is left to buf_select. The kept set is the
+// same as buf_select's (the k smallest keys, which are unique).
+template <int CAP>
+__device__ __forceinline__ float lin_select(WaveLds<CAP>& L, uint32_t lane, uint32_t cnt, uint32_t k, uint32_t hi,
+                                            uint32_t bT) {
+    const float scale = 64.f * __builtin_amdgcn_rcpf(__uint_as_float(hi));
+    // (a NaN product, when hi is 0 or denormal, gives bin 63)
+    auto bin = [&](uint32_t d2) { return (uint32_t)fminf(__uint_as_float(d2) * scale, 63.f); };
     L.hist[lane] = 0;
     wave_sync();
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if ((uint32_t)j * 64 + lane < cnt) {
-            const uint32_t h = bT2 - (uint32_t)(v[j] >> 53);
-            atomicAdd(&L.hist[h < 63u ? h : 63u], 1u);
-        }
-    }
+    for (uint32_t base = 0; base < cnt; base += 64)
+        if (base + lane < cnt) atomicAdd(&L.hist[bin((uint32_t)(L.buf[base + lane] >> 32))], 1u);
     wave_sync();
-    const uint32_t cum = wave_incl_scan(L.hist[63 - lane], lane);
-    const int ls = __builtin_ctzll(wballot(cum >= k));
-    const uint32_t hstar = 63u - (uint32_t)ls;
-    uint32_t A = __builtin_amdgcn_readlane(cum, ls);
-    const uint32_t prev = __builtin_amdgcn_readlane(cum, ls > 0 ? ls - 1 : 0);
-    uint64_t khi = (uint64_t)(bT2 - hstar + 1u) << 53, klo = 0;
-    uint32_t below = 0;
-    if (hstar < 63u) {
-        klo = (uint64_t)(bT2 - hstar) << 53;
-        below = ls > 0 ? prev : 0u;
-    }
-    if (khi > khi_io) khi = khi_io;
-    while (A > k) {
-        const uint64_t width = khi - klo;
-        const int s = width <= 64 ? 0 : 64 - __builtin_clzll(width - 1) - 6;
-        L.hist[lane] = 0;
+    const uint32_t h = L.hist[lane];
+    const uint32_t incl = wave_incl_scan(h, lane);
+    const uint32_t bs = (uint32_t)__builtin_ctzll(wballot(incl >= k));
+    const uint32_t c = __builtin_amdgcn_readlane(h, bs), need = k - (__builtin_amdgcn_readlane(incl, bs) - c);
+    wave_sync();  // the bins are read before the list (same LDS) is written
+    if (c > 32u) {
+        uint64_t khi = (uint64_t)hi << 32;
+        buf_select<CAP>(L, lane, cnt, k, k, bT, khi);
         wave_sync();
-#pragma unroll
-        for (int j = 0; j < R; ++j)
-            if (v[j] >= klo && v[j] < khi) atomicAdd(&L.hist[(uint32_t)((v[j] - klo) >> s)], 1u);
+        float d = 0.f;
+        for (uint32_t e = lane; e < k; e += 64) d = fmaxf(d, __uint_as_float((uint32_t)(L.buf[e] >> 32)));
+        return wave_max_nonneg_f32(d);
+    }
+    // (a row's writes never pass its reads: the LDS is in order for a wave)
+    uint32_t out = 0, lc = 0;
+    for (uint32_t base = 0; base < cnt; base += 64) {
+        const uint64_t key = base + lane < cnt ? L.buf[base + lane] : ~0ull;
         wave_sync();
-        const uint32_t cu = wave_incl_scan(L.hist[lane], lane);
-        const uint32_t need = k - below;
-        const int js = __builtin_ctzll(wballot(cu >= need));
-        const uint32_t pv = __builtin_amdgcn_readlane(cu, js > 0 ? js - 1 : 0);
-        const uint32_t at = __builtin_amdgcn_readlane(cu, js);
-        const uint64_t nlo = klo + ((uint64_t)js << s);
-        uint64_t nhi = klo + ((uint64_t)(js + 1) << s);
-        if (nhi > khi) nhi = khi;
-        A = below + at;
-        below += js > 0 ? pv : 0u;
-        klo = nlo;
-        khi = nhi;
+        const uint32_t b = base + lane < cnt ? bin((uint32_t)(key >> 32)) : 64u;
+        const uint64_t lt = wballot(b < bs), eq = wballot(b == bs);
+        if (b < bs) L.buf[out + mbcnt(lt)] = key;
+        if (b == bs) L.list[lc + mbcnt(eq)] = key;
+        out += (uint32_t)__popcll(lt);
+        lc += (uint32_t)__popcll(eq);
+        wave_sync();
     }
-    // the kept keys (invalid entries are ~0, never below the bound), in order
-    uint32_t out = 0;
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        const bool keep = v[j] < khi;
-        const uint64_t bal = wballot(keep);
-        if (keep) L.buf[out + mbcnt(bal)] = v[j];
-        out += (uint32_t)__popcll(bal);
+    const uint64_t kk = lane < c ? L.list[lane & 31u] : ~0ull;
+    uint32_t rank = 0;
+    for (uint32_t j = 0; j < c; ++j) {
+        const uint64_t kj = ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(kk >> 32), j) << 32) |
+                            (uint32_t)__builtin_amdgcn_readlane((uint32_t)kk, j);
+        rank += kj < kk ? 1u : 0u;
     }
-    khi_io = khi;
-    return out;
+    if (lane < c && rank < need) L.buf[out + rank] = kk;
+    const int at = __builtin_ctzll(wballot(lane < c && rank == need - 1u));
+    return __uint_as_float(__builtin_amdgcn_readlane((uint32_t)(kk >> 32), at));
 }
 
 // Ascending bitonic sort of buf[0, n) in LDS by one wave; n is a power of two.

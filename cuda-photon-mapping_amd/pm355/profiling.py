@@ -8,7 +8,7 @@ bench.py reads. Each summary records a hash of the HIP sources it was
 measured on; bench.py flags the numbers as stale when the sources have
 changed since.
 
-    python -m pm355.profiling summarize --kernel k_knn_stream512 \
+    python -m pm355.profiling summarize --kernel k_knn_stream \
         --pmc DIR [DIR ...] --copy DIR [DIR ...] --meta sources=gather key=value ... --out FILE
     python -m pm355.profiling valu --pmc DIR --traces 2 --out FILE
 
