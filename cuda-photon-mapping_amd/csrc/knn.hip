@@ -69,6 +69,7 @@ struct KnnParams {
     // than 64 rows): gq = 1 and the rows are taken 64 at a time.
     int nr, w, gq;
     uint32_t n_waves;
+    float guess;         // candidates that the guessed bound aims at (stream_wave)
     uint32_t xcd_shift;  // log2 of the workgroups in an XCD's chunk (remap 2)
     // (nullable) the query count on the device, at most nq: positions past
     // it are skipped; nq stays the planes' stride
@@ -662,9 +663,15 @@ __device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr 
 //
 // With h > 0 the walk first covers only the inner box (the query's cell
 // +- h), and only keys closer than every photon outside it are kept (its
-// squared face gap less a few ulps of rounding). If that finds at least k
-// keys, the k smallest are the answer; otherwise the query walks the whole
-// box again from an empty buffer. Both outcomes are exact.
+// squared face gap less a few ulps of rounding). Where the first walk's rows
+// hold many more candidates N than k, its bound b is lowered to the squared
+// radius expected to hold somewhat more than k of them, and the rows and
+// cells are pruned to that: on surfaces the photons within b are about
+// N / (1 + 0.6 cell / sqrt(b))^2 (the walked cells against the disc), evenly
+// in d2; `guess` = 1.2 (k + 3 sqrt(k) + 2) leaves three standard deviations
+// and a fifth for an uneven map. If the first walk finds at least k keys, the
+// k smallest are the answer; otherwise the query walks the whole box again
+// from an empty buffer. Both outcomes are exact.
 //
 // One wave, the nqw <= gq queries at positions p0, p0 + stride, ... of
 // `order` (entries less qb; null: the positions themselves). The set-up
@@ -716,15 +723,32 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
             int zi, yi;
             small_divmod(s, side, __builtin_amdgcn_rcpf((float)side), zi, yi);
             const int yy = cy - w + yi, zz = cz - w + zi;
-            uint32_t b = 0, len = 0;
-            if (mine && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2])
-                row_cells(G, kp->starts, kp->sizes, yy, zz, max(0, cx - w), min(G.g[0] - 1, cx + w), x, y, z, Trow, b,
-                          len);
-            const uint32_t incl = wave_incl_scan(len, lane);
-            // each query's stream starts at 0: less the lanes before its first
-            const uint32_t before = __shfl(incl, i > 0 ? i * nr - 1 : 0, 64);
-            end = incl - (i > 0 ? before : 0u);
-            d4 = (b + len - end) * 4u;
+            const bool row = mine && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2];
+            const int xlo = max(0, cx - w), xhi = min(G.g[0] - 1, cx + w);
+            const float cr = 1.f + 0.6f * G.cell * __builtin_amdgcn_rsqf(Trow);
+            const float aim = kp->guess * cr * cr;
+            uint32_t len;
+            for (bool first = true;; first = false) {
+                uint32_t b = 0;
+                len = 0;
+                if (row) row_cells(G, kp->starts, kp->sizes, yy, zz, xlo, xhi, x, y, z, Trow, b, len);
+                const uint32_t incl = wave_incl_scan(len, lane);
+                // each query's stream starts at 0: less the lanes before its first
+                const uint32_t before = __shfl(incl, i > 0 ? i * nr - 1 : 0, 64);
+                end = incl - (i > 0 ? before : 0u);
+                d4 = (b + len - end) * 4u;
+                if (!first) break;
+                // many more candidates than k: a smaller bound first, when
+                // that is so for most of the wave's queries or far so for one
+                const uint32_t all = __shfl(end, min(i * nr + nr - 1, 63), 64);
+                const bool crowded = mine && aim < 0.7f * (float)all;
+                const int nc = __builtin_popcountll(wballot(crowded));
+                if (2 * nc < (int)nqw * nr && !wballot(mine && aim < 0.2f * (float)all)) break;
+                if (crowded) {
+                    Trow = Trow * aim * __builtin_amdgcn_rcpf((float)all);
+                    hib = min(hib, __float_as_uint(Trow));
+                }
+            }
             rows_all = wballot(len > 0);
         }
     }
@@ -741,7 +765,10 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
             const __amdgpu_buffer_rsrc_t rx = plane_rsrc(kp->px, n), ry = plane_rsrc(kp->py, n),
                                          rz = plane_rsrc(kp->pz, n);
             hi = __builtin_amdgcn_readlane(hib, lb);
-            bool batch = nr > 0, inner = kp->h > 0;
+            // (a first walk below the radius is of the inner box when there
+            // is one)
+            const uint32_t hit = __float_as_uint(kp->T) + 1u;
+            bool batch = nr > 0, inner = kp->h > 0 && nr == 0, part = hi < hit;
             for (;;) {
                 cnt = 0;
                 for (int sbase = 0;; sbase += 64) {
@@ -788,12 +815,11 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
                 // with at least k such keys, the k smallest keys overall are
                 // among them (the buffer holds every in-radius key below its
                 // bound, or at least k of them once narrowed)
-                if (!inner) break;
+                if (!part) break;
                 kp = opaque(kp0);
                 if (cnt >= (uint32_t)kp->k) break;
                 // otherwise the whole box from an empty buffer
-                inner = false;
-                batch = false;
+                inner = part = batch = false;
                 hi = __float_as_uint(kp->T) + 1u;
                 wave_sync();
             }
@@ -1484,6 +1510,9 @@ void split_waves(KnnParams& P, uint64_t total) {
     const uint64_t fit = P.nr > 0 ? 64 / (uint64_t)P.nr : 1;
     P.gq = (int)std::max<uint64_t>(1, std::min<uint64_t>(fit, total / kFillWaves));
     P.n_waves = pm::div_up(P.nq, (uint32_t)P.gq);
+    // (a single query's wave would only wait for the second look-up of its
+    // rows, and the inner box is about the guess already)
+    P.guess = P.gq > 1 && P.h == 0 ? 1.2f * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
 }
 
 pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint32_t* order_out) {

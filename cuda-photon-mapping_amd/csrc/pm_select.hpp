@@ -201,11 +201,13 @@ __device__ uint32_t buf_select(WaveLds<CAP>& L, uint32_t lane, uint32_t cnt, uin
 // buf_select to exactly the k smallest of the cnt > k keys, whose d2 bits all
 // lie below hi; returns the k-th smallest's d2. One histogram of 64 bins
 // linear in d2 (photons on surfaces fall evenly in d2, so the bin of the
-// k-th holds a few keys: the mapping is monotone however it rounds), one
-// in-place compaction of the keys in the bins below, and the crossing bin's
-// keys ranked against each other. A crossing bin of more than 32 keys
-// (duplicates, extreme clusters) is left to buf_select. The kept set is the
-// same as buf_select's (the k smallest keys, which are unique).
+// k-th holds a few keys: the mapping is monotone however it rounds), the
+// crossing bin's keys ranked against each other, and one in-place compaction.
+// A crossing bin of more than 32 keys (duplicates, extreme clusters) is left
+// to buf_select. The kept set is the same as buf_select's (the k smallest
+// keys, which are unique), in buffer order, which is the order of the walk
+// whatever bounds were tried on the way: a query's estimate does not depend
+// on the queries that its wave or launch holds besides.
 template <int CAP>
 __device__ __forceinline__ float lin_select(WaveLds<CAP>& L, uint32_t lane, uint32_t cnt, uint32_t k, uint32_t hi,
                                             uint32_t bT) {
@@ -230,19 +232,17 @@ __device__ __forceinline__ float lin_select(WaveLds<CAP>& L, uint32_t lane, uint
         for (uint32_t e = lane; e < k; e += 64) d = fmaxf(d, __uint_as_float((uint32_t)(L.buf[e] >> 32)));
         return wave_max_nonneg_f32(d);
     }
-    // (a row's writes never pass its reads: the LDS is in order for a wave)
-    uint32_t out = 0, lc = 0;
+    // the crossing bin's keys, ranked against each other: the k-th smallest
+    uint32_t lc = 0;
     for (uint32_t base = 0; base < cnt; base += 64) {
-        const uint64_t key = base + lane < cnt ? L.buf[base + lane] : ~0ull;
-        wave_sync();
-        const uint32_t b = base + lane < cnt ? bin((uint32_t)(key >> 32)) : 64u;
-        const uint64_t lt = wballot(b < bs), eq = wballot(b == bs);
-        if (b < bs) L.buf[out + mbcnt(lt)] = key;
-        if (b == bs) L.list[lc + mbcnt(eq)] = key;
-        out += (uint32_t)__popcll(lt);
-        lc += (uint32_t)__popcll(eq);
-        wave_sync();
+        const bool in = base + lane < cnt;
+        const uint64_t key = in ? L.buf[base + lane] : ~0ull;
+        const bool eq = in && bin((uint32_t)(key >> 32)) == bs;
+        const uint64_t bal = wballot(eq);
+        if (eq) L.list[lc + mbcnt(bal)] = key;
+        lc += (uint32_t)__popcll(bal);
     }
+    wave_sync();
     const uint64_t kk = lane < c ? L.list[lane & 31u] : ~0ull;
     uint32_t rank = 0;
     for (uint32_t j = 0; j < c; ++j) {
@@ -250,9 +250,22 @@ __device__ __forceinline__ float lin_select(WaveLds<CAP>& L, uint32_t lane, uint
                             (uint32_t)__builtin_amdgcn_readlane((uint32_t)kk, j);
         rank += kj < kk ? 1u : 0u;
     }
-    if (lane < c && rank < need) L.buf[out + rank] = kk;
     const int at = __builtin_ctzll(wballot(lane < c && rank == need - 1u));
-    return __uint_as_float(__builtin_amdgcn_readlane((uint32_t)(kk >> 32), at));
+    const uint32_t khi = __builtin_amdgcn_readlane((uint32_t)(kk >> 32), at);
+    const uint64_t kth = ((uint64_t)khi << 32) | (uint32_t)__builtin_amdgcn_readlane((uint32_t)kk, at);
+    // in-place compaction in buffer order, one row of 64 at a time (a row's
+    // writes never pass its reads: the LDS is in order for a wave)
+    uint32_t out = 0;
+    for (uint32_t base = 0; base < cnt; base += 64) {
+        const uint64_t key = base + lane < cnt ? L.buf[base + lane] : ~0ull;
+        wave_sync();
+        const bool keep = key <= kth;
+        const uint64_t bal = wballot(keep);
+        if (keep) L.buf[out + mbcnt(bal)] = key;
+        out += (uint32_t)__popcll(bal);
+        wave_sync();
+    }
+    return __uint_as_float(khi);
 }
 
 // Ascending bitonic sort of buf[0, n) in LDS by one wave; n is a power of two.

@@ -59,7 +59,10 @@ def test_lists_and_estimate(ctx, inputs, cell, layout, flags, nq, k):
     rgb, rcnt = ctx.gather_radiance(g, q, qn, R, k, flags, want_count=True)
     both = ctx.gather_batch([(g, q, qn, R, k), (g, q[:, :777].copy(), qn[:, :777].copy(), R, k)], flags,
                             want_knn=True)
+    few = ctx.gather_radiance(g, q[:, :777].copy(), qn[:, :777].copy(), R, k, flags)
     ctx.sync()
+    # a query's estimate does not depend on the launch it is part of
+    assert np.array_equal(few.cpu().numpy().view(np.uint32), rgb[:, :777].cpu().numpy().view(np.uint32))
     for i, d, c in ((idx, dist, cnt), (both[0]["idx"], both[0]["dist"], both[0]["count"])):
         assert np.array_equal(c.cpu().numpy().view(np.uint32), oc)
         assert np.array_equal(i.cpu().numpy().view(np.uint32), oi)
