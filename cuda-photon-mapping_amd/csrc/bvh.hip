@@ -96,7 +96,8 @@ __global__ __launch_bounds__(256) void k_bvh_nodes(const uint32_t* __restrict__ 
         parent_int[g + 1] = i;
     }
     if (i == 0) parent_int[0] = -1;
-    nodes[4 * (size_t)(base + i) + 3] = make_float4(__int_as_float(c0), __int_as_float(c1), 0.f, 0.f);
+    nodes[4 * (size_t)(base + i) + 3] =
+        make_float4(__int_as_float(c0), __int_as_float(c1), __int_as_float((int)t0 + lo), __int_as_float(hi - lo + 1));
 }
 
 // Boxes pass between threads of different blocks (and XCDs): device-scope
@@ -145,6 +146,65 @@ __global__ __launch_bounds__(256) void k_bvh_boxes(const float* __restrict__ t9,
         child = base + node;
         node = up;
     }
+}
+
+// Triangle records: slot t0 + j holds triangle t0 + (vals ? vals[j] : j). A
+// model with a BVH has its records in the tree's leaf order.
+__global__ __launch_bounds__(256) void k_tri_recs(const float* __restrict__ t9, const uint32_t* __restrict__ vals,
+                                                 uint32_t t0, uint32_t n, float4* __restrict__ recs) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j >= n) return;
+    const uint32_t t = t0 + (vals ? vals[j] : j);
+    pmg::store_rec(recs, t0 + j, t,
+                   pmg::make_rec(pmg::load_v(t9, t, 0), pmg::load_v(t9, t, 1), pmg::load_v(t9, t, 2)));
+}
+
+// The four-wide node of each binary node: its two children, a child of more
+// than four triangles replaced by its own two; one of at most four becomes a
+// leaf (its record slots are consecutive).
+__global__ __launch_bounds__(256) void k_bvh_wide(const float4* __restrict__ nodes, int base, int n,
+                                                 float4* __restrict__ wide) {
+    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n) return;
+    int k = 0;
+    float4* w = wide + 8 * (size_t)(base + i);
+    auto put = [&](const float* box, int code) {
+        w[2 * k] = make_float4(box[0], box[1], box[2], box[3]);
+        w[2 * k + 1] = make_float4(box[4], box[5], __int_as_float(code), 0.f);
+        ++k;
+    };
+    // child c of binary node p: its box, and its code in the wide tree
+    auto child = [&](int p, int c, float (&box)[6], int& first, int& count) -> int {
+        const float4* nd = nodes + 4 * (size_t)p;
+        const float f[12] = {nd[0].x, nd[0].y, nd[0].z, nd[0].w, nd[1].x, nd[1].y,
+                             nd[1].z, nd[1].w, nd[2].x, nd[2].y, nd[2].z, nd[2].w};
+        for (int d = 0; d < 6; ++d) box[d] = c == 0 ? f[d] : f[6 + d];
+        const int code = __float_as_int(c == 0 ? nd[3].x : nd[3].y);
+        const int lo = __float_as_int(nd[3].z), cnt = __float_as_int(nd[3].w);
+        if (code < 0) {
+            first = c == 0 ? lo : lo + cnt - 1;
+            count = 1;
+        } else {
+            first = __float_as_int(nodes[4 * (size_t)code + 3].z);
+            count = __float_as_int(nodes[4 * (size_t)code + 3].w);
+        }
+        return code;
+    };
+    for (int c = 0; c < 2; ++c) {
+        float box[6];
+        int first, count;
+        const int code = child(base + i, c, box, first, count);
+        if (count <= 4) {
+            put(box, pmg::wide_leaf(first, count));
+            continue;
+        }
+        for (int g = 0; g < 2; ++g) {
+            const int gc = child(code, g, box, first, count);
+            put(box, count <= 4 ? pmg::wide_leaf(first, count) : gc);
+        }
+    }
+    const float none[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    while (k < 4) put(none, pmg::kWideNone);
 }
 
 }  // namespace
@@ -210,6 +270,22 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
             return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %llu nodes", (unsigned long long)n_nodes));
         }
     }
+    // (a wide leaf's code holds its first record slot in 29 bits)
+    if (scene->n_tris && scene->n_tris < (1u << 29)) {
+        hipError_t e = hipMalloc(&a->recs, (size_t)scene->n_tris * 80);
+        if (e != hipSuccess) {
+            a->recs = nullptr;
+            return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %u triangles", scene->n_tris));
+        }
+        if (n_nodes && (e = hipMalloc(&a->wide, n_nodes * 128)) != hipSuccess) {
+            a->wide = nullptr;
+            return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %llu nodes", (unsigned long long)n_nodes));
+        }
+        hipLaunchKernelGGL(k_tri_recs, dim3(pm::div_up(scene->n_tris, 256)), dim3(256), 0, ctx->stream,
+                           scene->d_tris9, (const uint32_t*)nullptr, 0u, scene->n_tris, a->recs);
+        hipError_t le = hipGetLastError();
+        if (le != hipSuccess) return bail(pm::hip_fail(ctx, le, "k_tri_recs"));
+    }
     // exact model AABBs (the reference's create_kd_tree result)
     hipError_t e = hipMemcpyAsync(d_tb, ranges.data(), ranges.size() * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e != hipSuccess) return bail(pm::hip_fail(ctx, e, "pm_accel_build: upload"));
@@ -244,6 +320,13 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
         hipLaunchKernelGGL(k_bvh_boxes, dim3(pm::div_up(n, 256)), dim3(256), 0, ctx->stream, scene->d_tris9, vals_s,
                            (int)n, t0, base, margin, a->nodes, parent_int, parent_leaf, arrive);
         PM_CHECK_LAUNCH(ctx, "k_bvh_boxes");
+        if (a->recs) {
+            hipLaunchKernelGGL(k_tri_recs, dim3(pm::div_up(n, 256)), dim3(256), 0, ctx->stream, scene->d_tris9,
+                               vals_s, t0, n, a->recs);
+            hipLaunchKernelGGL(k_bvh_wide, dim3(pm::div_up(n - 1, 256)), dim3(256), 0, ctx->stream, a->nodes, base,
+                               (int)(n - 1), a->wide);
+            PM_CHECK_LAUNCH(ctx, "k_bvh_wide");
+        }
         a->roots[i] = base;
         base += (int)(n - 1);
     }
@@ -254,6 +337,8 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
 extern "C" pm_status pm_accel_destroy(pm_accel* accel) {
     if (!accel) return PM_OK;
     if (accel->nodes) (void)hipFree(accel->nodes);
+    if (accel->recs) (void)hipFree(accel->recs);
+    if (accel->wide) (void)hipFree(accel->wide);
     delete accel;
     return PM_OK;
 }

@@ -44,11 +44,7 @@ struct Cam {
 };
 
 struct RaysParams {
-    const float* tris;
-    const float* nrms;
-    const DevModel* models;
-    int n_models;
-    const float4* bvh;
+    SceneGeo geo;
     float def_ior;
     Cam cam;
     int max_depth;
@@ -72,8 +68,8 @@ struct Plan {
 };
 
 __global__ __launch_bounds__(256) void k_render_rays(RaysParams P) {
-    __shared__ uint2 s_stack[kLdsStack * kStackLanes];
-    const BvhStack S{s_stack + threadIdx.x};
+    __shared__ RayLds s_ray[kRayWaves];
+    RayLds& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
     // 8x8 pixel tile per wave: coherent rays share model AABB outcomes
     const uint32_t lane = threadIdx.x & 63, wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int W = P.cam.w, H = P.cam.h;
@@ -131,17 +127,13 @@ __global__ __launch_bounds__(256) void k_render_rays(RaysParams P) {
         float th = 0.f;
         V3 n = v3(0, 0, 0);
         int hmod = -1;
-        // all lanes join the (wave-uniform) triangle loops; dead lanes shoot a
-        // null ray that hits nothing
-        Ray rr = ray;
-        if (!alive) rr.d = v3(0, 0, 0);
-        bool hit = scene_hit(P.models, P.n_models, P.tris, P.nrms, P.bvh, rr, th, n, hmod, S) && alive;
+        const bool hit = find_hit<false>(P.geo, alive, ray, th, n, hmod, S);
         if (!hit) continue;
         // Raytracer::find_intersection: point = dir*t + origin; normal turned
         // toward the ray only inside objects
         V3 ip = add(mul(ray.d, th), ray.o);
         if (in_obj && dot(ray.d, n) > 0) n = mul(n, -1.f);
-        const DevModel& mat = P.models[hmod];
+        const DevModel& mat = P.geo.models[hmod];
         if (nh < (uint32_t)P.hmax) {
             size_t s = (size_t)nh * P.npix + pix, plane = (size_t)P.hmax * P.npix;
             P.hp[s] = ip.x;
@@ -401,11 +393,7 @@ extern "C" pm_status pm_frame_rays(pm_ctx* ctx, pm_frame* F, const pm_scene* sce
     if ((st = upload_models(ctx, scene, F->d_models, tmp, host_models)) != PM_OK) return st;
 
     RaysParams P{};
-    P.tris = scene->d_tris9;
-    P.nrms = scene->d_normals9;
-    P.models = F->d_models;
-    P.n_models = F->nm;
-    P.bvh = bvh_nodes(scene);
+    P.geo = scene_geo(scene, F->d_models);
     P.def_ior = scene->default_refr_index;
     std::memcpy(&P.cam, camera, sizeof(Cam));
     P.max_depth = R.max_depth;
@@ -635,11 +623,7 @@ pm_status frame_plan_create(pm_ctx* ctx, const pm_scene* scene, const pm_camera*
         return st;
     }
     RaysParams& P = F->P;
-    P.tris = scene->d_tris9;
-    P.nrms = scene->d_normals9;
-    P.models = F->d_models;
-    P.n_models = F->nm;
-    P.bvh = bvh_nodes(scene);
+    P.geo = scene_geo(scene, F->d_models);
     P.def_ior = scene->default_refr_index;
     std::memcpy(&P.cam, camera, sizeof(Cam));
     P.max_depth = R.max_depth;

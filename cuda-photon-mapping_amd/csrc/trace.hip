@@ -31,11 +31,7 @@ struct CaEntry {
 };
 
 struct TraceParams {
-    const float* tris;
-    const float* nrms;
-    const DevModel* models;
-    int n_models;
-    const float4* bvh;
+    SceneGeo geo;
     int light;
     float pp[3];
     float def_ior;
@@ -55,7 +51,12 @@ struct TraceParams {
     // opaque < 1), as a bit mask; valid when n_models <= 64
     uint64_t spec_mask;
     int spec_mask_valid;
-    uint32_t n_segs;  // caustic phase: emission blocks (queue segments) of this batch
+    // The batch's paths are emitted in segments of `seg` consecutive paths, a
+    // wave each: segment k's kept paths are entries k seg ... of the queue,
+    // seg_len[k] of them. List l, a tracing block's work, is the segments l,
+    // l + n_lists, ...
+    uint32_t seg, n_segs, n_lists;
+    uint32_t* seg_len;
     // Planned traces (a fixed batch schedule enqueued without host
     // synchronisation): the maps' fill counts so far, on the device, decide
     // each batch's phase; null for the host-driven loop.
@@ -114,49 +115,73 @@ __device__ __forceinline__ bool ca_lookup(const TraceParams& P, float n1, float 
 
 // Emission (PhotonTracing.cu:345-370) with gpu_get_random_point_with_normal
 // (Model.cuh:202-243): roundf triangle pick, barycentrics x = u,
-// y = u' (1 - x), origin offset 1e-4 along the (unnormalised) normal.
-__device__ __forceinline__ Ray emit(const TraceParams& P, Stream& rng) {
-    const DevModel& L = P.models[P.light];
+// y = u' (1 - x), origin offset 1e-4 along the (unnormalised) normal. The
+// point takes the first three words of the path's block 0, and every trial
+// of a direction four: the word left of the block before, and the first three
+// of the next one.
+__device__ __forceinline__ void emit_point(const TraceParams& P, uint32_t path, V3& o, V3& lnrm, uint32_t& word) {
+    const DevModel& L = P.geo.models[P.light];
     const uint32_t lt = L.t1 - L.t0;
-    int tsel = (int)roundf(0 + rng.next() * (float)((3 * (int)lt - 3) / 3));
+    uint32_t w[4];
+    philox4x32_10((uint32_t)P.seed, (uint32_t)(P.seed >> 32), path, 0u, 0u, w);
+    int tsel = (int)roundf(0 + uniform01(w[0]) * (float)((3 * (int)lt - 3) / 3));
     uint32_t t = L.t0 + (uint32_t)tsel;
-    float ux = rng.next();
-    float uy = 0.f + rng.next() * ((1.f - ux) - 0.f);
+    float ux = uniform01(w[1]);
+    float uy = 0.f + uniform01(w[2]) * ((1.f - ux) - 0.f);
     float uz = 1.f - ux - uy;
-    V3 point = add(add(mul(load_v(P.tris, t, 0), ux), mul(load_v(P.tris, t, 1), uy)), mul(load_v(P.tris, t, 2), uz));
-    V3 lnrm = add(add(mul(load_v(P.nrms, t, 0), ux), mul(load_v(P.nrms, t, 1), uy)), mul(load_v(P.nrms, t, 2), uz));
-    Ray ray;
-    ray.o = add(point, mul(lnrm, 0.0001f));
-    float prob, dt;
-    do {
-        ray.d.x = -1.f + rng.next() * (1.f - -1.f);
-        ray.d.y = -1.f + rng.next() * (1.f - -1.f);
-        ray.d.z = -1.f + rng.next() * (1.f - -1.f);
-        ray.d = normalize_rcp(ray.d);
-        prob = rng.next();
-        dt = dot(ray.d, lnrm);
-        if (dt < 0) {
-            dt = -dt;
-            ray.d = mul(ray.d, -1.f);
-        }
-    } while (prob > dt);
-    return ray;
+    V3 point = add(add(mul(load_v(P.geo.tris, t, 0), ux), mul(load_v(P.geo.tris, t, 1), uy)),
+                   mul(load_v(P.geo.tris, t, 2), uz));
+    lnrm = add(add(mul(load_v(P.geo.nrms, t, 0), ux), mul(load_v(P.geo.nrms, t, 1), uy)),
+               mul(load_v(P.geo.nrms, t, 2), uz));
+    o = add(point, mul(lnrm, 0.0001f));
+    word = w[3];
+}
+// One trial of the direction from block blk; false: rejected, the next trial
+// follows.
+__device__ __forceinline__ bool emit_trial(const TraceParams& P, uint32_t path, uint32_t blk, uint32_t& word, V3 lnrm,
+                                           V3& d) {
+    uint32_t w[4];
+    philox4x32_10((uint32_t)P.seed, (uint32_t)(P.seed >> 32), path, blk, 0u, w);
+    d.x = -1.f + uniform01(word) * (1.f - -1.f);
+    d.y = -1.f + uniform01(w[0]) * (1.f - -1.f);
+    d.z = -1.f + uniform01(w[1]) * (1.f - -1.f);
+    d = normalize_rcp(d);
+    const float prob = uniform01(w[2]);
+    word = w[3];
+    float dt = dot(d, lnrm);
+    if (dt < 0) {
+        dt = -dt;
+        d = mul(d, -1.f);
+    }
+    return !(prob > dt);
 }
 
 // With the global map full, a path whose first ray reaches no specular or
 // refractive model's AABB (the test scene_hit gates every model with) first
 // hits a diffuse surface or nothing: it can store no caustic photon.
 __device__ __forceinline__ bool may_store_caustic(const TraceParams& P, const Ray& ray) {
-    bool any = false;
-    for (uint64_t msk = P.spec_mask; msk; msk &= msk - 1) any |= box_hit(P.models[__builtin_ctzll(msk)].box, ray);
+    const RayInv R = ray_inv(ray);
+    bool any = false, doubt = !R.safe;
+    for (uint64_t msk = P.spec_mask; msk; msk &= msk - 1) {
+        bool hit, miss;
+        box_quick(P.geo.models[__builtin_ctzll(msk)].box, ray, R.inv, hit, miss);
+        any |= hit;
+        doubt |= !hit && !miss;
+    }
+    any = any && R.safe;
+    if (!any && doubt)
+        for (uint64_t msk = P.spec_mask; msk; msk &= msk - 1) any |= box_hit(P.geo.models[__builtin_ctzll(msk)].box, ray);
     return any;
 }
 
-// A caustic-phase path that survived emission: its ray and generator state.
+// An emitted path: its ray, its number in the batch, and its generator's
+// state after emission (the next block, and the word left of the one before).
 struct PathState {
-    float o[3], d[3];
-    uint32_t i, blk, pos;
-    uint32_t buf[4];
+    float o[3];
+    uint32_t i;
+    float d[3];
+    uint32_t blk;
+    uint32_t word;
 };
 
 // The state of one light path between bounces.
@@ -181,10 +206,11 @@ struct Live {
     }
 };
 
-// One bounce of a path (trace / destiny, PhotonTracing.cu:127-326), staging
-// its photon at path slot L.i. Returns false once the path has ended; the
-// caller then stores the path's photon counts.
-__device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, BvhStack S) {
+// One bounce of a path at its ray's hit (trace / destiny,
+// PhotonTracing.cu:127-326), staging its photon at path slot L.i. Returns
+// false once the path has ended; the caller then stores the path's photon
+// counts.
+__device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, float th, V3 n, int hm) {
     const V3 pp = v3(P.pp[0], P.pp[1], P.pp[2]);
     Ray& ray = L.ray;
     Stream& rng = L.rng;
@@ -192,28 +218,25 @@ __device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, BvhSt
     const uint32_t i = L.i;
     {
         // trace (PhotonTracing.cu:278-326)
-        float th;
-        V3 n;
-        int hm;
-        if (!scene_hit(P.models, P.n_models, P.tris, P.nrms, P.bvh, ray, th, n, hm, S)) return false;
         V3 ip = add(mul(ray.d, th), ray.o);
         if (dot(ray.d, n) > 0) n = mul(n, -1.f);
-        const DevModel& mo = P.models[hm];
+        const DevModel& mo = P.geo.models[hm];
         const float cosNL = dot(neg(ray.d), n);
         const float ior = mo.ior;
         const int mid = mo.id;
         uint8_t dest = 0xFF;
+        rng.ensure(2);
         // refract_destity (PhotonTracing.cu:220-243) with get_refraction_pair
         if (mo.opaque != 1.f) {
             float n1, n2;
             if (ms.size == 0) {
                 n1 = P.def_ior;
                 n2 = ior;
-            } else if (P.models[ms.top()].id == mid) {
-                n1 = P.models[ms.top()].ior;
-                n2 = ms.size == 1 ? P.def_ior : P.models[ms.second()].ior;
+            } else if (P.geo.models[ms.top()].id == mid) {
+                n1 = P.geo.models[ms.top()].ior;
+                n2 = ms.size == 1 ? P.def_ior : P.geo.models[ms.second()].ior;
             } else {
-                n1 = P.models[ms.top()].ior;
+                n1 = P.geo.models[ms.top()].ior;
                 n2 = ior;
             }
             float ca;
@@ -247,12 +270,12 @@ __device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, BvhSt
         if (dest == REFR) {
             // get_update_refraction_pair (PhotonTracing.cu:127-151)
             float n1, n2;
-            if (ms.size != 0 && P.models[ms.top()].id == mid) {
-                n1 = P.models[ms.top()].ior;
-                n2 = ms.size == 1 ? P.def_ior : P.models[ms.second()].ior;
+            if (ms.size != 0 && P.geo.models[ms.top()].id == mid) {
+                n1 = P.geo.models[ms.top()].ior;
+                n2 = ms.size == 1 ? P.def_ior : P.geo.models[ms.second()].ior;
                 ms.pop();
             } else {
-                n1 = ms.size == 0 ? P.def_ior : P.models[ms.top()].ior;
+                n1 = ms.size == 0 ? P.def_ior : P.geo.models[ms.top()].ior;
                 n2 = ior;
                 if (ms.size < P.max_b) ms.push((uint32_t)hm);
             }
@@ -295,6 +318,7 @@ __device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, BvhSt
                 do {
                     float x1, x2, s1, s2;
                     do {
+                        rng.ensure(2);
                         x1 = -1.f + rng.next() * (1.f - -1.f);
                         x2 = -1.f + rng.next() * (1.f - -1.f);
                         s1 = x1 * x1;
@@ -318,107 +342,136 @@ __device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, BvhSt
     return ++L.b < P.max_b;
 }
 
-// Caustic phase, step 1: emission only. Most paths end here; each block of
-// kEmitBlock paths packs its survivors, in path order, at the front of its
-// own queue segment and records how many there are, so the bounce loop
-// (k_trace_continue) runs in dense waves without any global atomic.
-constexpr int kEmitBlock = 1024;
+// Emission of a segment by one wave. The direction is drawn by rejection: half
+// the trials fail, and the most trials of 64 paths are seven or eight. So the
+// wave tries until three quarters of its lanes have a direction; those store
+// theirs and take the segment's next paths, and the trials go on with the
+// others' where they are. A path a lane, to the last, took half as many
+// instructions again; refilling as soon as a few lanes were free took as
+// many (storing and setting up cost the wave as much as three trials). In
+// the caustic phase most paths end here: only those that may store a photon
+// are kept.
+constexpr uint32_t kSegPaths = 256;
 
-__global__ __launch_bounds__(kEmitBlock) void k_trace_emit(TraceParams P, PathState* __restrict__ queue,
-                                                          uint32_t* __restrict__ seg_len) {
-    __shared__ uint32_t s_wave[kEmitBlock / 64];
-    const uint32_t i = blockIdx.x * kEmitBlock + threadIdx.x;
-    const uint32_t lane = __lane_id(), wave = threadIdx.x >> 6;
-    if (P.got && batch_phase(P) != 1) {
-        // a planned batch outside the caustic phase: no survivors here
-        if (threadIdx.x == 0) seg_len[blockIdx.x] = 0;
-        return;
+__global__ __launch_bounds__(64) void k_trace_emit(TraceParams P, PathState* __restrict__ queue) {
+    const int ph = batch_phase(P);
+    if (ph == 2) return;
+    // (a scene of more than 64 models keeps every path)
+    const bool all = ph == 0 || !P.spec_mask_valid;
+    const uint32_t lo = blockIdx.x * P.seg, hi = min(lo + P.seg, P.n_paths);
+    PathState* out = queue + (size_t)blockIdx.x * P.seg;
+    uint32_t next = lo, kept = 0;  // (wave-uniform)
+    bool have = false;             // a path in trial
+    bool full = false;             // a direction found
+    uint32_t i = 0, blk = 0, word = 0;
+    Ray ray{v3(0, 0, 0), v3(0, 0, 0)};
+    V3 lnrm = v3(0, 0, 0);
+    for (;;) {
+        // lanes with a direction store their path
+        bool keep = false;
+        if (full) {
+            if (ph == 1) P.cnt_c[i] = 0;  // (the global counts are not read in this phase)
+            keep = all || may_store_caustic(P, ray);
+            full = false;
+        }
+        const uint64_t mk = __ballot(keep);
+        if (keep) {
+            PathState st;
+            st.o[0] = ray.o.x, st.o[1] = ray.o.y, st.o[2] = ray.o.z;
+            st.d[0] = ray.d.x, st.d[1] = ray.d.y, st.d[2] = ray.d.z;
+            st.i = i;
+            st.blk = blk;
+            st.word = word;
+            out[kept + __builtin_amdgcn_mbcnt_hi((uint32_t)(mk >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mk, 0u))] = st;
+        }
+        kept += (uint32_t)__popcll(mk);
+        // lanes without a path take the next ones
+        const uint64_t mn = __ballot(!have);
+        if (!have) {
+            i = next + __builtin_amdgcn_mbcnt_hi((uint32_t)(mn >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mn, 0u));
+            if (i < hi) {
+                emit_point(P, (uint32_t)(P.path_base + i), ray.o, lnrm, word);
+                blk = 1;
+                have = true;
+            }
+        }
+        next += (uint32_t)__popcll(mn);
+        if (!__ballot(have)) break;
+        do {
+            if (have) {
+                full = emit_trial(P, (uint32_t)(P.path_base + i), blk, word, lnrm, ray.d);
+                have = !full;
+                ++blk;
+            }
+        } while (__popcll(__ballot(have)) > (next < hi ? 16 : 0));
     }
-    bool keep = false;
-    Ray ray;
-    Stream rng;
-    if (i < P.n_paths) {
-        rng.init(P.seed, 0u, (uint32_t)(P.path_base + i));
-        ray = emit(P, rng);
-        P.cnt_c[i] = 0;  // (the global counts are not read in this phase)
-        keep = may_store_caustic(P, ray);
-    }
-    const uint64_t m = __ballot(keep);
-    if (lane == 0) s_wave[wave] = (uint32_t)__popcll(m);
-    __syncthreads();
-    uint32_t before = 0, total = 0;
-#pragma unroll
-    for (int w = 0; w < kEmitBlock / 64; ++w) {
-        const uint32_t c = s_wave[w];
-        before += (uint32_t)w < wave ? c : 0u;
-        total += c;
-    }
-    if (threadIdx.x == 0) seg_len[blockIdx.x] = total;
-    if (!keep) return;
-    const uint32_t slot = blockIdx.x * kEmitBlock + before + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-    PathState st;
-    st.o[0] = ray.o.x, st.o[1] = ray.o.y, st.o[2] = ray.o.z;
-    st.d[0] = ray.d.x, st.d[1] = ray.d.y, st.d[2] = ray.d.z;
-    st.i = i;
-    st.blk = rng.blk;
-    st.pos = rng.pos;
-    for (int c = 0; c < 4; ++c) st.buf[c] = rng.buf[c];
-    queue[slot] = st;
+    if (threadIdx.x == 0) P.seg_len[blockIdx.x] = kept;
 }
 
-// Path r of the caustic-phase survivor list (in path order): entry
-// r - seg_off[s] of queue segment s, the last segment whose exclusive offset
-// is <= r.
-__device__ __forceinline__ void queued_path(const TraceParams& P, const PathState* __restrict__ queue,
-                                            const uint32_t* __restrict__ seg_off, uint32_t r, Live& L) {
-    uint32_t lo = 0, hi = P.n_segs - 1;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (seg_off[mid] <= r)
-            lo = mid;
+// Path e of the block's list: entry e - pre[k] of its segment k, the last
+// one with pre[k] <= e (pre: the exclusive scan of the segments' lengths).
+__device__ __forceinline__ void take_path(const TraceParams& P, const PathState* __restrict__ queue,
+                                          const uint32_t* pre, uint32_t mine, uint32_t e, Live& L) {
+    uint32_t a = 0, b = mine - 1;
+    while (a < b) {
+        const uint32_t mid = (a + b + 1) >> 1;
+        if (pre[mid] <= e)
+            a = mid;
         else
-            hi = mid - 1;
+            b = mid - 1;
     }
-    const PathState st = queue[lo * kEmitBlock + (r - seg_off[lo])];
+    const PathState st = queue[(size_t)(blockIdx.x + a * P.n_lists) * P.seg + (e - pre[a])];
     Stream rng;
     rng.init(P.seed, 0u, (uint32_t)(P.path_base + st.i));
-    rng.blk = st.blk;
-    rng.pos = st.pos;
-    for (int c = 0; c < 4; ++c) rng.buf[c] = st.buf[c];
+    rng.resume(st.blk, st.word);
     Ray ray;
     ray.o = v3(st.o[0], st.o[1], st.o[2]);
     ray.d = v3(st.d[0], st.d[1], st.d[2]);
     L.start(st.i, rng, ray);
 }
 
-// Persistent path tracing. Block b owns a contiguous range of the batch's
-// paths (global phase: path slots; caustic phase: survivor list entries).
+// Persistent path tracing. Block b works on list b of the emitted paths.
 // Each lane traces one path a bounce at a time and, when it ends, takes the
-// block's next path from an LDS counter, so a wave keeps its lanes busy
+// list's next path from an LDS counter, so a wave keeps its lanes busy
 // instead of waiting on its longest path. Which lane traces a path does not
-// change the photons it stores.
-template <bool kQueued>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_trace_pool(TraceParams P, const PathState* __restrict__ queue,
-                                                   const uint32_t* __restrict__ seg_off,
-                                                   const uint64_t* __restrict__ n_queued) {
-    __shared__ uint2 s_stack[kLdsStack * kStackLanes];
+// change the photons it stores. Bound by latency with four waves a SIMD (120
+// VGPRs; at five waves it spills and takes 1.5 times as long) and by the VALU:
+// the Cornell box's 2M + 500k photons take 0.65 + 0.87 ms here and 0.05 + 0.18
+// ms of emission, where the model-by-model walk with emission inside took
+// 1.42 + 1.09 + 0.31 ms.
+constexpr uint32_t kListSegs = 128;  // segments of a list, at most (the host sees to it)
+
+template <bool kRecs>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_trace_pool(
+    TraceParams P, const PathState* __restrict__ queue) {
+    __shared__ RayLds s_ray[kRayWaves];
+    __shared__ uint32_t s_pre[kListSegs + 1];
     __shared__ uint32_t s_next;
-    if (P.got) {
-        // planned batch: the queued kernels trace the caustic phase when the
-        // scene allows it, this one everything else; nothing once both maps
-        // are full
-        const int ph = batch_phase(P);
-        if (ph == 2 || (!kQueued && ph == 1 && P.spec_mask_valid) || (kQueued && ph != 1)) return;
-        P.caustic_only = ph;
+    const int ph = batch_phase(P);
+    if (ph == 2) return;  // (a planned batch with both maps full)
+    P.caustic_only = ph;
+    RayLds& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    const uint32_t mine = blockIdx.x < P.n_segs ? (P.n_segs - blockIdx.x - 1u) / P.n_lists + 1u : 0u;
+    if (threadIdx.x < 64) {
+        uint32_t sum = 0;
+        for (uint32_t k0 = 0; k0 < mine; k0 += 64) {
+            const uint32_t k = k0 + threadIdx.x;
+            uint32_t v = k < mine ? P.seg_len[blockIdx.x + k * P.n_lists] : 0u;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t y = __shfl_up(v, d, 64);
+                if (threadIdx.x >= (uint32_t)d) v += y;
+            }
+            if (k < mine) s_pre[k + 1] = sum + v;
+            sum += __shfl(v, 63, 64);
+        }
+        if (threadIdx.x == 0) s_pre[0] = 0;
     }
-    const BvhStack S{s_stack + threadIdx.x};
-    const uint32_t total = kQueued ? (uint32_t)*n_queued : P.n_paths;
-    const uint32_t per = (total + gridDim.x - 1) / gridDim.x;
-    const uint32_t lo = min(blockIdx.x * per, total), hi = min(lo + per, total);
-    if (threadIdx.x == 0) s_next = lo;
+    if (threadIdx.x == 0) s_next = 0;
     __syncthreads();
+    const uint32_t hi = mine ? s_pre[mine] : 0u;
     const uint32_t lane = __lane_id();
-    Live L;
+    Live L{};
     bool alive = false, done = false;
     for (;;) {
         const bool need = !alive && !done;
@@ -431,14 +484,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
             if (need) {
                 const uint32_t idx = base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
                 if (idx < hi) {
-                    if (kQueued) {
-                        queued_path(P, queue, seg_off, idx, L);
-                    } else {
-                        Stream rng;
-                        rng.init(P.seed, 0u, (uint32_t)(P.path_base + idx));
-                        const Ray ray = emit(P, rng);
-                        L.start(idx, rng, ray);
-                    }
+                    take_path(P, queue, s_pre, mine, idx, L);
                     alive = true;
                 } else {
                     done = true;
@@ -447,7 +493,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
         }
         // every lane is now tracing a path or out of work for good
         if (!__ballot(alive)) break;
-        if (alive && !bounce_step(P, L, S)) {
+        float th = 0.f;
+        V3 n = v3(0, 0, 0);
+        int hm = 0;
+        const bool hit = find_hit<kRecs>(P.geo, alive, L.ray, th, n, hm, S);
+        if (alive && !(hit && bounce_step(P, L, th, n, hm))) {
             P.cnt_g[L.i] = L.ng;
             P.cnt_c[L.i] = L.nc;
             alive = false;
@@ -550,16 +600,40 @@ pm_status trace_tables(pm_ctx* ctx, const pm_scene* scene, uint32_t n_global, in
     return PM_OK;
 }
 
+typedef void (*PoolKernel)(TraceParams, const PathState*);
+PoolKernel pool_kernel(const TraceParams& P) { return P.geo.recs ? k_trace_pool<true> : k_trace_pool<false>; }
+
+// Resident blocks of the persistent tracer (one full round over the CUs),
+// the number of lists.
+pm_status pool_lists(pm_ctx* ctx, const TraceParams& P, uint32_t* lists) {
+    int per_cu = 0;
+    PM_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pool_kernel(P), 256, 0));
+    *lists = (uint32_t)std::max(1, per_cu) * (uint32_t)std::max(1, ctx->cu_count);
+    return PM_OK;
+}
+
+// One batch's emission and tracing (P.n_paths, path_base and phase set).
+pm_status trace_batch(pm_ctx* ctx, TraceParams& P, PathState* queue) {
+    // (longer segments waste fewer trials at their ends; eight a list or more
+    // keep the lists even)
+    P.seg = kSegPaths;
+    while (P.seg < 1024u && (uint64_t)P.seg * 16 * P.n_lists <= P.n_paths) P.seg *= 2;
+    while ((uint64_t)P.seg * kListSegs * P.n_lists < P.n_paths) P.seg *= 2;
+    P.n_segs = pm::div_up(P.n_paths, P.seg);
+    P.n_lists = std::min(P.n_lists, P.n_segs);
+    hipLaunchKernelGGL(k_trace_emit, dim3(P.n_segs), dim3(64), 0, ctx->stream, P, queue);
+    PM_CHECK_LAUNCH(ctx, "k_trace_emit");
+    hipLaunchKernelGGL(pool_kernel(P), dim3(P.n_lists), dim3(256), 0, ctx->stream, P, queue);
+    PM_CHECK_LAUNCH(ctx, "k_trace_pool");
+    return PM_OK;
+}
+
 // The scene part of a trace's kernel parameters.
 void trace_params_base(const pm_scene* scene, const DevModel* d_models, const CaEntry* d_ca, int n_ca,
                        uint32_t n_global, int B, TraceParams& P) {
     const int nm = scene->n_models;
     P = TraceParams{};
-    P.tris = scene->d_tris9;
-    P.nrms = scene->d_normals9;
-    P.models = d_models;
-    P.n_models = nm;
-    P.bvh = bvh_nodes(scene);
+    P.geo = scene_geo(scene, d_models);
     P.spec_mask = 0;
     P.spec_mask_valid = nm <= 64 ? 1 : 0;
     for (int i = 0; i < nm && i < 64; ++i) {
@@ -603,14 +677,18 @@ extern "C" pm_status pm_trace_photons(pm_ctx* ctx, const pm_scene* scene, uint64
         std::min<uint64_t>(std::min<uint64_t>(kCausticBatch, std::max<uint64_t>(16 * want, 65536)), max_paths), 1);
     const uint32_t npath = std::max(batch_g, batch_c);
     const size_t slots = std::max((size_t)batch_g * B, (size_t)batch_c);
-    const uint32_t nseg = pm::div_up(batch_c, kEmitBlock);
+    TraceParams P;
+    trace_params_base(scene, nullptr, nullptr, 0, n_global, B, P);
+    uint32_t lists = 0;
+    pm_status st = pool_lists(ctx, P, &lists);
+    if (st != PM_OK) return st;
+    const size_t segs = pm::div_up(npath, kSegPaths);
     size_t rs_bytes = pm::carve_size({(size_t)nm * sizeof(DevModel), ca.size() * sizeof(CaEntry) + 16,
                                       (size_t)nm * 32, slots * 36, slots, (size_t)npath * 4, (size_t)npath * 4,
-                                      (size_t)npath * 4, (size_t)npath * 4, 3 * sizeof(uint64_t),
-                                      (size_t)nseg * kEmitBlock * sizeof(PathState), (size_t)nseg * 4,
-                                      (size_t)nseg * 4});
+                                      (size_t)npath * 4, (size_t)npath * 4, 2 * sizeof(uint64_t),
+                                      (size_t)npath * sizeof(PathState), segs * 4});
     void* work = nullptr;
-    pm_status st = pm::scratch_reserve(ctx, rs_bytes, &work);
+    st = pm::scratch_reserve(ctx, rs_bytes, &work);
     if (st != PM_OK) return st;
     pm::Carve cv{static_cast<char*>(work)};
     DevModel* d_models = cv.take<DevModel>(nm);
@@ -622,28 +700,22 @@ extern "C" pm_status pm_trace_photons(pm_ctx* ctx, const pm_scene* scene, uint64
     uint32_t* cnt_c = cv.take<uint32_t>(npath);
     uint32_t* off_g = cv.take<uint32_t>(npath);
     uint32_t* off_c = cv.take<uint32_t>(npath);
-    uint64_t* tot = cv.take<uint64_t>(3);
-    PathState* queue = cv.take<PathState>((size_t)nseg * kEmitBlock);
-    uint32_t* seg_len = cv.take<uint32_t>(nseg);
-    uint32_t* seg_off = cv.take<uint32_t>(nseg);
+    uint64_t* tot = cv.take<uint64_t>(2);
+    PathState* queue = cv.take<PathState>(npath);
+    uint32_t* seg_len = cv.take<uint32_t>(segs);
 
     // model records with their AABBs (the live effect of create_kd_tree)
     if ((st = upload_models(ctx, scene, d_models, d_tmp, hm)) != PM_OK) return st;
     if (!ca.empty())
         PM_HIP(ctx, hipMemcpyAsync(d_ca, ca.data(), ca.size() * sizeof(CaEntry), hipMemcpyHostToDevice, ctx->stream));
 
-    TraceParams P;
     trace_params_base(scene, d_models, d_ca, (int)ca.size(), n_global, B, P);
     P.seed = seed;
+    P.seg_len = seg_len;
     P.stage = stage;
     P.kind = kind;
     P.cnt_g = cnt_g;
     P.cnt_c = cnt_c;
-
-    // resident blocks of the persistent tracer: one full round over the CUs
-    int per_cu = 0;
-    PM_HIP(ctx, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace_pool<false>, 256, 0));
-    const uint32_t pool_blocks = (uint32_t)std::max(1, per_cu) * (uint32_t)ctx->cu_count;
 
     uint64_t paths = 0, got_g = 0, got_c = 0;
     uint32_t batch = batch_g;
@@ -657,22 +729,8 @@ extern "C" pm_status pm_trace_photons(pm_ctx* ctx, const pm_scene* scene, uint64
                                                          max_paths - paths);
         P.path_base = paths;
         P.n_paths = nb;
-        // In that phase most paths end at emission; the survivors go through
-        // a queue so that the bounce loop runs in dense waves.
-        const bool queued = P.caustic_only && P.spec_mask_valid;
-        if (queued) {
-            P.n_segs = pm::div_up(nb, kEmitBlock);
-            hipLaunchKernelGGL(k_trace_emit, dim3(P.n_segs), dim3(kEmitBlock), 0, ctx->stream, P, queue, seg_len);
-            PM_CHECK_LAUNCH(ctx, "k_trace_emit");
-            if ((st = pm::scan_u32(ctx, seg_len, seg_off, P.n_segs, false, tot + 2)) != PM_OK) return st;
-            hipLaunchKernelGGL(k_trace_pool<true>, dim3(std::min(pm::div_up(nb, 256), pool_blocks)), dim3(256), 0,
-                               ctx->stream, P, queue, seg_off, tot + 2);
-            PM_CHECK_LAUNCH(ctx, "k_trace_pool<queued>");
-        } else {
-            hipLaunchKernelGGL(k_trace_pool<false>, dim3(std::min(pm::div_up(nb, 256), pool_blocks)), dim3(256), 0,
-                               ctx->stream, P, nullptr, nullptr, nullptr);
-            PM_CHECK_LAUNCH(ctx, "k_trace_pool");
-        }
+        P.n_lists = lists;
+        if ((st = trace_batch(ctx, P, queue)) != PM_OK) return st;
         // (in the caustic phase no path stores a global photon)
         if (!P.caustic_only && (st = pm::scan_u32(ctx, cnt_g, off_g, nb, false, tot)) != PM_OK) return st;
         if ((st = pm::scan_u32(ctx, cnt_c, off_c, nb, false, tot + 1)) != PM_OK) return st;
@@ -719,17 +777,16 @@ struct TracePlan {
     TraceParams P{};
     uint64_t* got = nullptr;
     uint64_t paths = 0;
-    uint32_t batch = 0, n_batches = 0, pool_blocks = 0;
+    uint32_t batch = 0, n_batches = 0, lists = 0;
     uint32_t n_global = 0, n_caustic = 0;
     int B = 0;
 };
 
 size_t trace_plan_scratch_bytes(const TracePlan* T) {
     const size_t slots = (size_t)T->batch * T->B;
-    const uint32_t nseg = div_up(T->batch, kEmitBlock);
     const size_t per_path = (size_t)T->batch * 4;
-    return carve_size({slots * 36, slots, per_path, per_path, per_path, per_path, 3 * sizeof(uint64_t),
-                       (size_t)nseg * kEmitBlock * sizeof(PathState), (size_t)nseg * 4, (size_t)nseg * 4});
+    return carve_size({slots * 36, slots, per_path, per_path, per_path, per_path, 2 * sizeof(uint64_t),
+                       (size_t)T->batch * sizeof(PathState), (size_t)div_up(T->batch, kSegPaths) * 4});
 }
 
 pm_status trace_plan_create(pm_ctx* ctx, const pm_scene* scene, uint32_t n_global, uint32_t n_caustic,
@@ -775,9 +832,10 @@ pm_status trace_plan_create(pm_ctx* ctx, const pm_scene* scene, uint32_t n_globa
         return fail(ctx, PM_ERR_HIP, "trace plan: upload");
     }
     trace_params_base(scene, d_models, d_ca, (int)ca.size(), n_global, max_bounces, T->P);
-    int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_trace_pool<false>, 256, 0) != hipSuccess) per_cu = 1;
-    T->pool_blocks = (uint32_t)std::max(1, per_cu) * (uint32_t)ctx->cu_count;
+    if ((st = pool_lists(ctx, T->P, &T->lists)) != PM_OK) {
+        trace_plan_destroy(T);
+        return st;
+    }
     *out = T;
     return PM_OK;
 }
@@ -795,7 +853,6 @@ pm_status trace_plan_enqueue(pm_ctx* ctx, TracePlan* T, uint64_t seed, float* d_
     pm_status st = scratch_reserve(ctx, trace_plan_scratch_bytes(T), &work);
     if (st != PM_OK) return st;
     const size_t slots = (size_t)T->batch * T->B;
-    const uint32_t nseg_max = div_up(T->batch, kEmitBlock);
     Carve cv{static_cast<char*>(work)};
     float* stage = cv.take<float>(slots * 9);
     uint8_t* kind = cv.take<uint8_t>(slots);
@@ -803,10 +860,9 @@ pm_status trace_plan_enqueue(pm_ctx* ctx, TracePlan* T, uint64_t seed, float* d_
     uint32_t* cnt_c = cv.take<uint32_t>(T->batch);
     uint32_t* off_g = cv.take<uint32_t>(T->batch);
     uint32_t* off_c = cv.take<uint32_t>(T->batch);
-    uint64_t* tot = cv.take<uint64_t>(3);
-    PathState* queue = cv.take<PathState>((size_t)nseg_max * kEmitBlock);
-    uint32_t* seg_len = cv.take<uint32_t>(nseg_max);
-    uint32_t* seg_off = cv.take<uint32_t>(nseg_max);
+    uint64_t* tot = cv.take<uint64_t>(2);
+    PathState* queue = cv.take<PathState>(T->batch);
+    uint32_t* seg_len = cv.take<uint32_t>(div_up(T->batch, kSegPaths));
     if ((st = fill_u32(ctx, reinterpret_cast<uint32_t*>(T->got), 0u, 4)) != PM_OK) return st;
     TraceParams P = T->P;
     P.seed = seed;
@@ -816,6 +872,7 @@ pm_status trace_plan_enqueue(pm_ctx* ctx, TracePlan* T, uint64_t seed, float* d_
     P.cnt_c = cnt_c;
     P.stage_depth = T->B;
     P.caustic_only = 0;
+    P.seg_len = seg_len;
     P.got = T->got;
     P.need_g = T->n_global;
     P.need_c = T->n_caustic;
@@ -824,18 +881,8 @@ pm_status trace_plan_enqueue(pm_ctx* ctx, TracePlan* T, uint64_t seed, float* d_
         const uint32_t nb = (uint32_t)std::min<uint64_t>(T->batch, T->paths - base);
         P.path_base = base;
         P.n_paths = nb;
-        P.n_segs = div_up(nb, kEmitBlock);
-        hipLaunchKernelGGL(k_trace_pool<false>, dim3(std::min(div_up(nb, 256), T->pool_blocks)), dim3(256), 0,
-                           ctx->stream, P, nullptr, nullptr, nullptr);
-        PM_CHECK_LAUNCH(ctx, "k_trace_pool (plan)");
-        if (P.spec_mask_valid) {
-            hipLaunchKernelGGL(k_trace_emit, dim3(P.n_segs), dim3(kEmitBlock), 0, ctx->stream, P, queue, seg_len);
-            PM_CHECK_LAUNCH(ctx, "k_trace_emit (plan)");
-            if ((st = scan_u32(ctx, seg_len, seg_off, P.n_segs, false, tot + 2)) != PM_OK) return st;
-            hipLaunchKernelGGL(k_trace_pool<true>, dim3(std::min(div_up(nb, 256), T->pool_blocks)), dim3(256), 0,
-                               ctx->stream, P, queue, seg_off, tot + 2);
-            PM_CHECK_LAUNCH(ctx, "k_trace_pool<queued> (plan)");
-        }
+        P.n_lists = T->lists;
+        if ((st = trace_batch(ctx, P, queue)) != PM_OK) return st;
         if ((st = scan_u32(ctx, cnt_g, off_g, nb, false, tot)) != PM_OK) return st;
         if ((st = scan_u32(ctx, cnt_c, off_c, nb, false, tot + 1)) != PM_OK) return st;
         hipLaunchKernelGGL(k_trace_compact, dim3(div_up(nb, 256)), dim3(256), 0, ctx->stream, stage, kind, cnt_g, cnt_c,
