@@ -70,6 +70,7 @@ struct KnnParams {
     int nr, w, gq;
     uint32_t n_waves;
     float guess;         // candidates that the guessed bound aims at (stream_wave)
+    float within;        // share of a box's candidates expected within the radius
     uint32_t xcd_shift;  // log2 of the workgroups in an XCD's chunk (remap 2)
     // (nullable) the query count on the device, at most nq: positions past
     // it are skipped; nq stays the planes' stride
@@ -620,6 +621,11 @@ __device__ __forceinline__ void finish_params(KnnParams& Pf, ParamsPtr kp) {
     Pf.out_count = kp->out_count;
 }
 
+// Keys that a narrowing of a buffer of CAP leaves at most: at least the
+// largest k that the buffer serves (256, or 512), and room for a step.
+template <int CAP>
+constexpr uint32_t kNarrowTo = CAP == 512 ? 256 : 512;
+
 // One step of the streaming selection over two candidates per lane (index
 // sa / sb, squared distance d2a / d2b, lanes holding one: masks am / bm):
 // appends the keys whose d2 bits lie below the acceptance bound hi to the
@@ -636,11 +642,11 @@ __device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr 
     uint64_t bala = am & wballot(__float_as_uint(d2a) < hi), balb = bm & wballot(__float_as_uint(d2b) < hi);
     uint32_t na = (uint32_t)__popcll(bala), nb = (uint32_t)__popcll(balb);
     if (cnt + na + nb > (uint32_t)CAP) {
-        // leaves at most CAP / 2 keys, room for this step's 128
+        // leaves at most kNarrowTo keys, room for this step's 128
         wave_sync();
         ParamsPtr kp = opaque(kp0);
         uint64_t khi = (uint64_t)hi << 32;
-        cnt = buf_select<CAP>(L, lane, cnt, (uint32_t)kp->k, CAP / 2, kp->bT, khi);
+        cnt = buf_select<CAP>(L, lane, cnt, (uint32_t)kp->k, kNarrowTo<CAP>, kp->bT, khi);
         hi = (uint32_t)((khi + 0xffffffffull) >> 32);
         bala = am & wballot(__float_as_uint(d2a) < hi);
         balb = bm & wballot(__float_as_uint(d2b) < hi);
@@ -684,133 +690,157 @@ __device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr 
 // run of queries with crowded boxes (a caustic's focus) is spread over as
 // many waves as one query a wave would give it. With consecutive queries per
 // wave instead, L2 reads doubled and a frame's gathers took 2.9 ms, not 1.9.
+// A wave's queries after their set-up: per lane, the query's index, position
+// and first bound (d2 bits, exclusive), and the run of the lane's row (as
+// walk_runs takes it); rows: the lanes whose run is not empty.
+struct WaveQueries {
+    uint32_t q, hib, d4, end;
+    float x, y, z;
+    uint64_t rows;
+};
+__device__ __forceinline__ void setup_queries(ParamsPtr kp0, uint32_t lane, const uint32_t* __restrict__ order,
+                                              uint32_t p0, uint32_t stride, uint32_t qb, uint32_t nqw,
+                                              WaveQueries& W) {
+    ParamsPtr kp = opaque(kp0);
+    const GridGeom G = geom_of(kp);
+    const int nr = kp->nr;
+    int i = 0, s = 0;
+    if (nr > 0) small_divmod((int)lane, nr, __builtin_amdgcn_rcpf((float)nr), i, s);
+    const bool mine = nr > 0 && (uint32_t)i < nqw;
+    const uint32_t pos = p0 + min((uint32_t)i, nqw - 1u) * stride;
+    const uint32_t q = (order ? order[pos] : pos) - qb;
+    const float x = kp->qx[q], y = kp->qy[q], z = kp->qz[q];
+    const int cx = pmd::cell_coord(x, G.mn[0], G.cell, G.g[0]), cy = pmd::cell_coord(y, G.mn[1], G.cell, G.g[1]),
+              cz = pmd::cell_coord(z, G.mn[2], G.cell, G.g[2]);
+    const float T = kp->T;
+    uint32_t hib = __float_as_uint(T) + 1u, d4 = 0, end = 0;
+    uint64_t rows_all = 0;
+    float Trow = T;
+    const int h = kp->h;
+    if (h > 0) {
+        const float gx = inner_gap(x, max(0, cx - h), min(G.g[0] - 1, cx + h), G.g[0], G.mn[0], G.cell),
+                    gy = inner_gap(y, max(0, cy - h), min(G.g[1] - 1, cy + h), G.g[1], G.mn[1], G.cell),
+                    gz = inner_gap(z, max(0, cz - h), min(G.g[2] - 1, cz + h), G.g[2], G.mn[2], G.cell);
+        const float gap = fminf(fminf(gx, gy), gz);
+        hib = min(__float_as_uint(gap * gap * 0.999f), hib);
+        // (only keys below the bound are kept: the rows are pruned with it)
+        Trow = fminf(T, __uint_as_float(hib));
+    }
+    if (nr > 0) {
+        const int w = kp->w, side = 2 * w + 1;
+        int zi, yi;
+        small_divmod(s, side, __builtin_amdgcn_rcpf((float)side), zi, yi);
+        const int yy = cy - w + yi, zz = cz - w + zi;
+        const bool row = mine && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2];
+        const int xlo = max(0, cx - w), xhi = min(G.g[0] - 1, cx + w);
+        const float cr = 1.f + 0.6f * G.cell * __builtin_amdgcn_rsqf(Trow);
+        const float aim = kp->guess * cr * cr;
+        uint32_t len;
+        for (bool first = true;; first = false) {
+            uint32_t b = 0;
+            len = 0;
+            if (row) row_cells(G, kp->starts, kp->sizes, yy, zz, xlo, xhi, x, y, z, Trow, b, len);
+            const uint32_t incl = wave_incl_scan(len, lane);
+            // each query's stream starts at 0: less the lanes before its first
+            const uint32_t before = __shfl(incl, i > 0 ? i * nr - 1 : 0, 64);
+            end = incl - (i > 0 ? before : 0u);
+            d4 = (b + len - end) * 4u;
+            if (!first) break;
+            // many more candidates than k: a smaller bound first, when
+            // that is so for most of the wave's queries or far so for one
+            const uint32_t all = __shfl(end, min(i * nr + nr - 1, 63), 64);
+            const bool crowded = mine && aim < 0.7f * (float)all;
+            const int nc = __builtin_popcountll(wballot(crowded));
+            if (2 * nc < (int)nqw * nr && !wballot(mine && aim < 0.2f * (float)all)) break;
+            if (crowded) {
+                Trow = Trow * aim * __builtin_amdgcn_rcpf((float)all);
+                hib = min(hib, __float_as_uint(Trow));
+            }
+        }
+        rows_all = wballot(len > 0);
+    }
+    W.q = q;
+    W.hib = hib;
+    W.d4 = d4;
+    W.end = end;
+    W.x = x;
+    W.y = y;
+    W.z = z;
+    W.rows = rows_all;
+}
+
+// f (as walk_runs calls it) over the candidates of the query whose first
+// lane is lb: the rows set up for it (batch), or the whole box, or the inner
+// one, looked up now, with rows and cells pruned to the d2 bits below hi.
+template <class F>
+__device__ __forceinline__ void walk_query(ParamsPtr kp0, uint32_t lane, const WaveQueries& W, uint32_t lb, bool batch,
+                                           bool inner, uint32_t hi, F&& f) {
+    ParamsPtr kp = opaque(kp0);
+    const int nr = kp->nr;
+    const float qx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.x), lb));
+    const float qy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.y), lb));
+    const float qz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.z), lb));
+    const uint32_t n = kp->n;
+    const __amdgpu_buffer_rsrc_t rx = plane_rsrc(kp->px, n), ry = plane_rsrc(kp->py, n), rz = plane_rsrc(kp->pz, n);
+    for (int sbase = 0;; sbase += 64) {
+        uint32_t cd4 = W.d4, cend = W.end, total;
+        uint64_t rows;
+        bool last = true;
+        if (batch) {
+            rows = W.rows & ((~0ull >> (64 - nr)) << lb);
+            total = __builtin_amdgcn_readlane(W.end, lb + (uint32_t)nr - 1u);
+        } else {
+            // 64 rows (Morton: cells) of the box, one per lane
+            ParamsPtr kc = opaque(kp0);
+            const GridGeom G = geom_of(kc);
+            const int w = inner ? kc->h : kc->rc;
+            const float qv[3] = {qx, qy, qz};
+            Box B;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const int c = __builtin_amdgcn_readfirstlane(pmd::cell_coord(qv[a], G.mn[a], G.cell, G.g[a]));
+                B.lo[a] = max(0, c - w);
+                B.hi[a] = min(G.g[a] - 1, c + w);
+            }
+            const int nx = B.hi[0] - B.lo[0] + 1, nyz = (B.hi[1] - B.lo[1] + 1) * (B.hi[2] - B.lo[2] + 1);
+            const int nseg = G.layout == PM_LAYOUT_LINEAR ? nyz : nx * nyz;
+            const int sr = sbase + (int)lane;
+            const float Trow = inner ? fminf(kc->T, __uint_as_float(hi)) : kc->T;
+            uint32_t b = 0, len = 0;
+            if (sr < nseg) row_span(G, kc->starts, kc->sizes, B, sr, qx, qy, qz, Trow, b, len);
+            cend = wave_incl_scan(len, lane);
+            cd4 = (b + len - cend) * 4u;
+            rows = wballot(len > 0);
+            total = __builtin_amdgcn_readlane(cend, 63);
+            last = sbase + 64 >= nseg;
+        }
+        if (total > 0) walk_runs(rx, ry, rz, lane, rows, cd4, cend, total, qx, qy, qz, f);
+        if (last) break;
+    }
+}
+
 template <int CAP, bool kLists>
 __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint32_t lane,
                                             const uint32_t* __restrict__ order, uint32_t p0, uint32_t stride,
                                             uint32_t qb, uint32_t nqw) {
-    uint32_t q, hib, d4 = 0, end = 0;
-    float x, y, z;
-    uint64_t rows_all = 0;
-    {
-        ParamsPtr kp = opaque(kp0);
-        const GridGeom G = geom_of(kp);
-        const int nr = kp->nr;
-        int i = 0, s = 0;
-        if (nr > 0) small_divmod((int)lane, nr, __builtin_amdgcn_rcpf((float)nr), i, s);
-        const bool mine = nr > 0 && (uint32_t)i < nqw;
-        const uint32_t pos = p0 + min((uint32_t)i, nqw - 1u) * stride;
-        q = (order ? order[pos] : pos) - qb;
-        x = kp->qx[q];
-        y = kp->qy[q];
-        z = kp->qz[q];
-        const int cx = pmd::cell_coord(x, G.mn[0], G.cell, G.g[0]), cy = pmd::cell_coord(y, G.mn[1], G.cell, G.g[1]),
-                  cz = pmd::cell_coord(z, G.mn[2], G.cell, G.g[2]);
-        const float T = kp->T;
-        hib = __float_as_uint(T) + 1u;
-        float Trow = T;
-        const int h = kp->h;
-        if (h > 0) {
-            const float gx = inner_gap(x, max(0, cx - h), min(G.g[0] - 1, cx + h), G.g[0], G.mn[0], G.cell),
-                        gy = inner_gap(y, max(0, cy - h), min(G.g[1] - 1, cy + h), G.g[1], G.mn[1], G.cell),
-                        gz = inner_gap(z, max(0, cz - h), min(G.g[2] - 1, cz + h), G.g[2], G.mn[2], G.cell);
-            const float gap = fminf(fminf(gx, gy), gz);
-            hib = min(__float_as_uint(gap * gap * 0.999f), hib);
-            // (only keys below the bound are kept: the rows are pruned with it)
-            Trow = fminf(T, __uint_as_float(hib));
-        }
-        if (nr > 0) {
-            const int w = kp->w, side = 2 * w + 1;
-            int zi, yi;
-            small_divmod(s, side, __builtin_amdgcn_rcpf((float)side), zi, yi);
-            const int yy = cy - w + yi, zz = cz - w + zi;
-            const bool row = mine && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2];
-            const int xlo = max(0, cx - w), xhi = min(G.g[0] - 1, cx + w);
-            const float cr = 1.f + 0.6f * G.cell * __builtin_amdgcn_rsqf(Trow);
-            const float aim = kp->guess * cr * cr;
-            uint32_t len;
-            for (bool first = true;; first = false) {
-                uint32_t b = 0;
-                len = 0;
-                if (row) row_cells(G, kp->starts, kp->sizes, yy, zz, xlo, xhi, x, y, z, Trow, b, len);
-                const uint32_t incl = wave_incl_scan(len, lane);
-                // each query's stream starts at 0: less the lanes before its first
-                const uint32_t before = __shfl(incl, i > 0 ? i * nr - 1 : 0, 64);
-                end = incl - (i > 0 ? before : 0u);
-                d4 = (b + len - end) * 4u;
-                if (!first) break;
-                // many more candidates than k: a smaller bound first, when
-                // that is so for most of the wave's queries or far so for one
-                const uint32_t all = __shfl(end, min(i * nr + nr - 1, 63), 64);
-                const bool crowded = mine && aim < 0.7f * (float)all;
-                const int nc = __builtin_popcountll(wballot(crowded));
-                if (2 * nc < (int)nqw * nr && !wballot(mine && aim < 0.2f * (float)all)) break;
-                if (crowded) {
-                    Trow = Trow * aim * __builtin_amdgcn_rcpf((float)all);
-                    hib = min(hib, __float_as_uint(Trow));
-                }
-            }
-            rows_all = wballot(len > 0);
-        }
-    }
+    WaveQueries W;
+    setup_queries(kp0, lane, order, p0, stride, qb, nqw, W);
     for (uint32_t i = 0; i < nqw; ++i) {
-        uint32_t cnt, hi, qi;
+        uint32_t cnt, hi, lb;
         {
             ParamsPtr kp = opaque(kp0);
-            const int nr = kp->nr;
-            const uint32_t lb = i * (uint32_t)nr;
-            const float qx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), lb));
-            const float qy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(y), lb));
-            const float qz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(z), lb));
-            const uint32_t n = kp->n;
-            const __amdgpu_buffer_rsrc_t rx = plane_rsrc(kp->px, n), ry = plane_rsrc(kp->py, n),
-                                         rz = plane_rsrc(kp->pz, n);
-            hi = __builtin_amdgcn_readlane(hib, lb);
+            lb = i * (uint32_t)kp->nr;
+            hi = __builtin_amdgcn_readlane(W.hib, lb);
             // (a first walk below the radius is of the inner box when there
             // is one)
             const uint32_t hit = __float_as_uint(kp->T) + 1u;
-            bool batch = nr > 0, inner = kp->h > 0 && nr == 0, part = hi < hit;
+            bool batch = kp->nr > 0, inner = kp->h > 0 && kp->nr == 0, part = hi < hit;
             for (;;) {
                 cnt = 0;
-                for (int sbase = 0;; sbase += 64) {
-                    uint32_t cd4 = d4, cend = end, total;
-                    uint64_t rows;
-                    bool last = true;
-                    if (batch) {
-                        rows = rows_all & ((~0ull >> (64 - nr)) << lb);
-                        total = __builtin_amdgcn_readlane(end, lb + (uint32_t)nr - 1u);
-                    } else {
-                        // 64 rows (Morton: cells) of the box, one per lane
-                        ParamsPtr kc = opaque(kp0);
-                        const GridGeom G = geom_of(kc);
-                        const int w = inner ? kc->h : kc->rc;
-                        const float qv[3] = {qx, qy, qz};
-                        Box B;
-#pragma unroll
-                        for (int a = 0; a < 3; ++a) {
-                            const int c = __builtin_amdgcn_readfirstlane(
-                                pmd::cell_coord(qv[a], G.mn[a], G.cell, G.g[a]));
-                            B.lo[a] = max(0, c - w);
-                            B.hi[a] = min(G.g[a] - 1, c + w);
-                        }
-                        const int nx = B.hi[0] - B.lo[0] + 1, nyz = (B.hi[1] - B.lo[1] + 1) * (B.hi[2] - B.lo[2] + 1);
-                        const int nseg = G.layout == PM_LAYOUT_LINEAR ? nyz : nx * nyz;
-                        const int sr = sbase + (int)lane;
-                        const float Trow = inner ? fminf(kc->T, __uint_as_float(hi)) : kc->T;
-                        uint32_t b = 0, len = 0;
-                        if (sr < nseg) row_span(G, kc->starts, kc->sizes, B, sr, qx, qy, qz, Trow, b, len);
-                        cend = wave_incl_scan(len, lane);
-                        cd4 = (b + len - cend) * 4u;
-                        rows = wballot(len > 0);
-                        total = __builtin_amdgcn_readlane(cend, 63);
-                        last = sbase + 64 >= nseg;
-                    }
-                    if (total > 0)
-                        walk_runs(rx, ry, rz, lane, rows, cd4, cend, total, qx, qy, qz,
-                                  [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
-                                      push2<CAP>(L, lane, kp0, am, sa, d2a, bm, sb, d2b, cnt, hi);
-                                  });
-                    if (last) break;
-                }
+                walk_query(kp0, lane, W, lb, batch, inner, hi,
+                           [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
+                               push2<CAP>(L, lane, kp0, am, sa, d2a, bm, sb, d2b, cnt, hi);
+                           });
                 wave_sync();
                 // with at least k such keys, the k smallest keys overall are
                 // among them (the buffer holds every in-radius key below its
@@ -823,7 +853,6 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
                 hi = __float_as_uint(kp->T) + 1u;
                 wave_sync();
             }
-            qi = __builtin_amdgcn_readlane(q, lb);
         }
         // The count within the radius that the finish needs is min(found, k),
         // and that is min(cnt, k): without a narrowing the buffer holds every
@@ -831,7 +860,7 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
         // k (it starts above CAP - 128 >= k keys), so cnt >= k after one.
         KnnParams Pf;
         finish_params(Pf, opaque(kp0));
-        finish<CAP, kLists>(Pf, L, lane, qi, cnt, hi);
+        finish<CAP, kLists>(Pf, L, lane, __builtin_amdgcn_readlane(W.q, lb), cnt, hi);
         wave_sync();  // the buffer is read before the next query's keys
     }
 }
@@ -842,10 +871,11 @@ __device__ __forceinline__ uint32_t wave_queries(uint32_t u, uint32_t n_waves, u
 }
 
 // The single-map launch, waves in the XCD-aware order. CAP = 512: 17 KB of
-// LDS per workgroup; CAP = 1024 (fewer narrowings, k up to 512) is
-// LDS-limited to 4 waves per SIMD.
+// LDS per workgroup; CAP = 768 (256 < k <= 512, estimate only): 25 KB, 6 waves
+// per SIMD; CAP = 1024 (a tuning variant: fewer narrowings) is LDS-limited to
+// 4.
 template <int CAP, bool kLists>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : 4))) void k_knn_stream(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : CAP == 768 ? 6 : 4))) void k_knn_stream(
     KnnParams P) {
     __shared__ WaveLds<CAP> lds[kWaves];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -975,225 +1005,283 @@ __global__ __launch_bounds__(64) void k_knn_large_list(KnnParams P, const uint32
     }
 }
 
-// Radiance for 256 < k <= 2048 without a k-key buffer (the kernel behind the
-// reference frame's k = 2000 / 400 gathers). One wave per query, three walks
-// of the candidate box:
-//   1. count the photons within r and histogram their d2 into 256 bins (8
-//      per octave below the radius threshold, ascending in d2), keeping the
-//      largest d2;
-//   2. only if more than k are within r: collect the keys (d2, slot) of the
-//      bin holding the k-th smallest into a 512-key LDS buffer and sort it in
-//      registers; the (k - below)-th key there is the k-th key K* overall;
-//   3. sum the estimate over the photons within r with key <= K* (all of them
-//      when at most k are within r), the filter radius being the largest
-//      kept distance.
+// Radiance for 512 < k <= 2048 without a k-key buffer (the kernel behind the
+// reference frame's k = 2000 gather), set up and walked as the streaming
+// gather, over a query's candidates up to four times:
+//   1. when its rows hold few enough candidates that at most k are expected
+//      within the radius: count them and keep the largest d2. That is all
+//      when at most k are: they are all kept;
+//   2. otherwise count them into 256 bins linear in d2 (even on surfaces);
+//   3. collect the keys (d2, slot) of the bin holding the k-th smallest, at
+//      most 64 (a fuller bin is split 256 ways by a walk first), and rank them
+//      against each other: the (k - below)-th there is the k-th key K*;
+//   4. sum the estimate over the photons with key <= K* (or all of them), the
+//      filter radius being the largest kept distance.
 // The kept set is exactly the k smallest (d2, slot) keys, as in the buffered
-// kernels; only the order of the radiance sum differs (walk order). A query
-// whose crossing bin holds more than 512 keys is appended to `ovf_list` for
-// k_knn_large_list.
-constexpr uint32_t kWideCap = 512;
+// kernels; the radiance sum runs in walk order. A query whose split bin still
+// holds more than 64 keys is appended to `ovf_list` for k_knn_large_list.
+// Bound by the VALU (85% of its issue). The reference frame's ~740k queries
+// (1M photons, k = 2000, r = 0.05): 6.56 ms with a set-up and three walks a
+// query, a 512-key register sort and the reference's FP32 weights, 5.12 ms
+// now. Listing the slots in walk 1 for the sum to run over, instead of walking
+// again, saved 9% of the instructions and lost as much to the LDS (8 KB a
+// wave: 5 waves per SIMD).
+constexpr uint32_t kWideList = 64;
+constexpr uint32_t kWideRing = 256;
 struct WideLds {
     union {
         uint32_t hist[256];
-        uint64_t buf[kWideCap];
+        uint64_t list[kWideList];
+        uint64_t ring[kWideRing];  // kept keys waiting for their batch of 64
     };
 };
 
-__device__ __forceinline__ uint32_t wide_bin(float d2, uint32_t bT20) {
-    // d2 <= T, so bits(d2) >> 20 <= bT20; d2 <= T / 2^32 (and 0) share bin 0
-    const uint32_t h = bT20 - (__float_as_uint(d2) >> 20);
-    return 255u - (h < 255u ? h : 255u);
+// The crossing of the k-th count in L.hist (ascending bins): its bin, that
+// bin's count, and the count in the bins before it.
+__device__ __forceinline__ void wide_crossing(const WideLds& L, uint32_t lane, uint32_t k, uint32_t& bin,
+                                              uint32_t& c, uint32_t& below) {
+    // lane l holds bins 4 l .. 4 l + 3
+    const uint32_t h0 = L.hist[4 * lane], h1 = L.hist[4 * lane + 1], h2 = L.hist[4 * lane + 2],
+                   h3 = L.hist[4 * lane + 3];
+    const uint32_t incl = wave_incl_scan(h0 + h1 + h2 + h3, lane);
+    const int ls = __builtin_ctzll(wballot(incl >= k));
+    const uint32_t c0 = __builtin_amdgcn_readlane(h0, ls), c1 = __builtin_amdgcn_readlane(h1, ls),
+                   c2 = __builtin_amdgcn_readlane(h2, ls), c3 = __builtin_amdgcn_readlane(h3, ls);
+    below = __builtin_amdgcn_readlane(incl, ls) - (c0 + c1 + c2 + c3);
+    bin = 4u * (uint32_t)ls;
+    c = c0;
+    if (below + c < k) below += c, ++bin, c = c1;
+    if (below + c < k) below += c, ++bin, c = c2;
+    if (below + c < k) below += c, ++bin, c = c3;
 }
 
-__global__ __launch_bounds__(256) void k_gather_wide(KnnParams P, uint32_t* __restrict__ ovf_list,
-                                                     uint32_t* __restrict__ ovf_count) {
-    __shared__ WideLds lds[kWaves];
-    uint32_t q;
-    if (!query_of_wave(P, q)) return;  // wave-uniform; no workgroup barriers below
-    const uint32_t lane = threadIdx.x & 63;
-    WideLds& L = lds[threadIdx.x >> 6];
-    Box B;
-    float qx, qy, qz;
-    box_of(P, q, B, qx, qy, qz);
-    const float T = P.T;
-    const uint32_t k = (uint32_t)P.k;
-    const uint32_t bT20 = __float_as_uint(T) >> 20;
+constexpr float kBinTop = 0x1.fffffep+7f;  // the largest float below 256
 
-    for (uint32_t e = lane; e < 256; e += 64) L.hist[e] = 0;
-    wave_sync();
-    uint32_t found = 0;
-    float dmax = 0.f;
-    walk2(P, lane, B, qx, qy, qz, T, [&](uint64_t am, uint32_t, float d2a, uint64_t bm, uint32_t, float d2b) {
-        const bool va = __builtin_amdgcn_inverse_ballot_w64(am), vb = __builtin_amdgcn_inverse_ballot_w64(bm);
-        const bool ina = d2a <= (va ? T : -1.0f), inb = d2b <= (vb ? T : -1.0f);
-        found += (uint32_t)(__popcll(wballot(ina)) + __popcll(wballot(inb)));
-        if (ina) {
-            atomicAdd(&L.hist[wide_bin(d2a, bT20)], 1u);
-            dmax = fmaxf(dmax, d2a);
-        }
-        if (inb) {
-            atomicAdd(&L.hist[wide_bin(d2b, bT20)], 1u);
-            dmax = fmaxf(dmax, d2b);
-        }
-    });
-    wave_sync();
-    found = __builtin_amdgcn_readfirstlane(found);
-    const uint32_t m = found < k ? found : k;
+// One query (lb: its first lane); false: handed to the overflow list.
+__device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, uint32_t lb, uint32_t lane,
+                                           WideLds& L) {
+    uint32_t found, hi, m;
+    bool batch;
     uint64_t kstar = ~0ull;
     float rmax2;
-    if (found > k) {
-        // lane l holds bins 4l .. 4l+3; the crossing bin is the first whose
-        // inclusive count from the smallest d2 reaches k
-        const uint32_t h0 = L.hist[4 * lane], h1 = L.hist[4 * lane + 1], h2 = L.hist[4 * lane + 2],
-                       h3 = L.hist[4 * lane + 3];
-        const uint32_t incl = wave_incl_scan(h0 + h1 + h2 + h3, lane);
-        const int ls = __builtin_ctzll(wballot(incl >= k));
-        uint32_t below = __shfl(incl - (h0 + h1 + h2 + h3), ls, 64);
-        const uint32_t c0 = __shfl(h0, ls, 64), c1 = __shfl(h1, ls, 64), c2 = __shfl(h2, ls, 64);
-        uint32_t bstar = 4u * (uint32_t)ls, nb = c0;
-        if (below + c0 < k) {
-            below += c0;
-            ++bstar;
-            nb = c1;
-            if (below + c1 < k) {
-                below += c1;
-                ++bstar;
-                nb = c2;
-                if (below + c2 < k) {
-                    below += c2;
-                    ++bstar;
-                    nb = __shfl(h3, ls, 64);
-                }
+    {
+        ParamsPtr kp = opaque(kp0);
+        const uint32_t k = (uint32_t)kp->k, hit = __float_as_uint(kp->T) + 1u;
+        batch = kp->nr > 0;
+        hi = __builtin_amdgcn_readlane(W.hib, lb);
+        bool part = hi < hit, binned = true;
+        if (batch && !part) {
+            const uint32_t all = __builtin_amdgcn_readlane(W.end, lb + (uint32_t)kp->nr - 1u);
+            binned = (float)all * kp->within > 0.9f * (float)k;
+        }
+        float dmax = 0.f, scale = 0.f;
+        for (;;) {
+            found = 0;
+            dmax = 0.f;
+            if (!binned) {
+                walk_query(kp0, lane, W, lb, batch, false, hi,
+                           [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
+                               const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi),
+                                              bb = bm & wballot(__float_as_uint(d2b) < hi);
+                               found += (uint32_t)(__popcll(ba) + __popcll(bb));
+                               dmax = fmaxf(dmax, __builtin_amdgcn_inverse_ballot_w64(ba) ? d2a : 0.f);
+                               dmax = fmaxf(dmax, __builtin_amdgcn_inverse_ballot_w64(bb) ? d2b : 0.f);
+                           });
+                if (found <= k) break;
+                binned = true;
+                continue;
             }
+            for (uint32_t e = lane; e < 256; e += 64) L.hist[e] = 0;
+            wave_sync();
+            // (a NaN product, when hi is 0 or denormal, gives bin 255)
+            scale = 256.f * __builtin_amdgcn_rcpf(__uint_as_float(hi));
+            walk_query(kp0, lane, W, lb, batch, false, hi,
+                       [&](uint64_t am, uint32_t, float d2a, uint64_t bm, uint32_t, float d2b) {
+                           const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi),
+                                          bb = bm & wballot(__float_as_uint(d2b) < hi);
+                           found += (uint32_t)(__popcll(ba) + __popcll(bb));
+                           if (__builtin_amdgcn_inverse_ballot_w64(ba)) {
+                               atomicAdd(&L.hist[(uint32_t)fminf(d2a * scale, kBinTop)], 1u);
+                               dmax = fmaxf(dmax, d2a);
+                           }
+                           if (__builtin_amdgcn_inverse_ballot_w64(bb)) {
+                               atomicAdd(&L.hist[(uint32_t)fminf(d2b * scale, kBinTop)], 1u);
+                               dmax = fmaxf(dmax, d2b);
+                           }
+                       });
+            wave_sync();
+            if (!part || found >= k) break;
+            // fewer than k below the guessed bound: the whole box
+            part = batch = false;
+            hi = hit;
         }
-        bstar = __builtin_amdgcn_readfirstlane(bstar);
-        below = __builtin_amdgcn_readfirstlane(below);
-        nb = __builtin_amdgcn_readfirstlane(nb);
-        wave_sync();  // the histogram is read before the buffer (same LDS) is written
-        if (nb > kWideCap) {
-            if (lane == 0) ovf_list[atomicAdd(ovf_count, 1u)] = q;
-            return;
+        m = found < k ? found : k;
+        if (found > k) {
+            uint32_t bin, c, below;
+            wide_crossing(L, lane, k, bin, c, below);
+            wave_sync();  // the bins are read before they are written again
+            uint32_t sub = 0;
+            const bool split = c > kWideList;
+            if (split) {
+                // the bin's keys by the next eight bits (the difference is
+                // exact, so the order is kept)
+                for (uint32_t e = lane; e < 256; e += 64) L.hist[e] = 0;
+                wave_sync();
+                walk_query(kp0, lane, W, lb, batch, false, hi,
+                           [&](uint64_t am, uint32_t, float d2a, uint64_t bm, uint32_t, float d2b) {
+                               const float fa = fminf(d2a * scale, kBinTop), fb = fminf(d2b * scale, kBinTop);
+                               const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot((uint32_t)fa == bin),
+                                              bb = bm & wballot(__float_as_uint(d2b) < hi) & wballot((uint32_t)fb == bin);
+                               if (__builtin_amdgcn_inverse_ballot_w64(ba))
+                                   atomicAdd(&L.hist[(uint32_t)((fa - (float)bin) * 256.f)], 1u);
+                               if (__builtin_amdgcn_inverse_ballot_w64(bb))
+                                   atomicAdd(&L.hist[(uint32_t)((fb - (float)bin) * 256.f)], 1u);
+                           });
+                wave_sync();
+                uint32_t b2;
+                wide_crossing(L, lane, k - below, sub, c, b2);
+                below += b2;
+                wave_sync();
+                if (c > kWideList) return false;
+            }
+            uint32_t cnt = 0;
+            walk_query(kp0, lane, W, lb, batch, false, hi,
+                       [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
+                           const float fa = fminf(d2a * scale, kBinTop), fb = fminf(d2b * scale, kBinTop);
+                           uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot((uint32_t)fa == bin),
+                                    bb = bm & wballot(__float_as_uint(d2b) < hi) & wballot((uint32_t)fb == bin);
+                           if (split) {
+                               ba &= wballot((uint32_t)((fa - (float)bin) * 256.f) == sub);
+                               bb &= wballot((uint32_t)((fb - (float)bin) * 256.f) == sub);
+                           }
+                           const uint32_t cb = __builtin_amdgcn_readfirstlane(cnt + (uint32_t)__popcll(ba));
+                           if (__builtin_amdgcn_inverse_ballot_w64(ba)) L.list[cnt + mbcnt(ba)] = make_key(d2a, sa);
+                           if (__builtin_amdgcn_inverse_ballot_w64(bb)) L.list[cb + mbcnt(bb)] = make_key(d2b, sb);
+                           cnt = cb + (uint32_t)__popcll(bb);
+                       });
+            wave_sync();
+            const uint64_t kk = lane < c ? L.list[lane] : ~0ull;
+            uint32_t rank = 0;
+            for (uint32_t j = 0; j < c; ++j) {
+                const uint64_t kj = ((uint64_t)__builtin_amdgcn_readlane((uint32_t)(kk >> 32), j) << 32) |
+                                    (uint32_t)__builtin_amdgcn_readlane((uint32_t)kk, j);
+                rank += kj < kk ? 1u : 0u;
+            }
+            const int at = __builtin_ctzll(wballot(lane < c && rank == k - below - 1u));
+            const uint32_t kh = __builtin_amdgcn_readlane((uint32_t)(kk >> 32), at);
+            kstar = ((uint64_t)kh << 32) | (uint32_t)__builtin_amdgcn_readlane((uint32_t)kk, at);
+            rmax2 = __uint_as_float(kh);
+        } else {
+            rmax2 = wave_max_nonneg_f32(dmax);
         }
-        uint32_t cnt = 0;
-        walk2(P, lane, B, qx, qy, qz, T, [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
-            const bool va = __builtin_amdgcn_inverse_ballot_w64(am), vb = __builtin_amdgcn_inverse_ballot_w64(bm);
-            const bool ina = d2a <= (va ? T : -1.0f) && wide_bin(d2a, bT20) == bstar;
-            const bool inb = d2b <= (vb ? T : -1.0f) && wide_bin(d2b, bT20) == bstar;
-            const uint64_t ba = wballot(ina), bb = wballot(inb);
-            const uint32_t na = (uint32_t)__popcll(ba);
-            if (ina) L.buf[cnt + mbcnt(ba)] = make_key(d2a, sa);
-            if (inb) L.buf[cnt + na + mbcnt(bb)] = make_key(d2b, sb);
-            cnt += na + (uint32_t)__popcll(bb);
-        });
-        wave_sync();
-        uint64_t v[kWideCap / 64];
-#pragma unroll
-        for (int j = 0; j < (int)(kWideCap / 64); ++j) {
-            const uint32_t e = (uint32_t)j * 64 + lane;
-            v[j] = e < cnt ? L.buf[e] : ~0ull;
-        }
-        bitonic_sort<kWideCap / 64>(v, lane);
-        const uint32_t r = k - below - 1;  // rank of K* in the bin (< nb)
-        const int jr = (int)(r >> 6);
-        uint64_t pick = 0;
-#pragma unroll
-        for (int j = 0; j < (int)(kWideCap / 64); ++j)
-            if (j == jr) pick = v[j];
-        const uint32_t lo = __shfl((uint32_t)pick, (int)(r & 63), 64);
-        const uint32_t hi = __shfl((uint32_t)(pick >> 32), (int)(r & 63), 64);
-        kstar = ((uint64_t)hi << 32) | lo;
-        rmax2 = __uint_as_float(hi);
-    } else {
-        dmax = wave_max_nonneg_f32(dmax);
-        rmax2 = dmax;
     }
-    if (P.out_count && lane == 0) P.out_count[q] = m;
+    const uint32_t q = __builtin_amdgcn_readlane(W.q, lb);
+    ParamsPtr kp = opaque(kp0);
+    if (kp->out_count && lane == 0) kp->out_count[q] = m;
 
-    // Raytracer.cuh:110-138 over the kept photons. Their keys queue in the
-    // wave's LDS buffer (free again); every 64 queued, one lane per photon
-    // loads its direction and power, and a batch's loads are consumed only
-    // when the next batch is taken (or after the walk), some walk steps
-    // later, so the walk never waits on them.
+    // Raytracer.cuh:110-138 over the kept photons, 64 at a time in walk order,
+    // one lane each, with the weights of radiance_buffer. Their keys queue in
+    // the wave's LDS ring; a batch's direction and power are consumed only when
+    // the next batch is taken, some walk steps later, so the walk does not wait
+    // on them.
     const float alpha = 1.818f, beta = 1.953f;
     const float pi_f = 3.141592654f;
+    const float inv_denom = 1.16529458f, log2e = 1.44269504f;
     float res0 = 0.f, res1 = 0.f, res2 = 0.f;
-    const float rmax = sqrtf(rmax2);
+    const float rmax = __builtin_amdgcn_sqrtf(rmax2);
+    const float filter_r = __fmul_rn(rmax, rmax);
+    const uint32_t nq = kp->nq;
     if (m > 0) {
-        const float filter_r = __fmul_rn(rmax, rmax);
-        const float denom = 1.f - expf(-beta);
-        const float nx = P.nrm[q], ny = P.nrm[P.nq + q], nz = P.nrm[2 * (size_t)P.nq + q];
-        const __amdgpu_buffer_rsrc_t rdx = plane_rsrc(P.dir, P.n), rdy = plane_rsrc(P.dir + P.n, P.n),
-                                     rdz = plane_rsrc(P.dir + 2 * (size_t)P.n, P.n);
-        const __amdgpu_buffer_rsrc_t rpr = plane_rsrc(P.power, P.n), rpg = plane_rsrc(P.power + P.n, P.n),
-                                     rpb = plane_rsrc(P.power + 2 * (size_t)P.n, P.n);
+        const float s = -beta * __builtin_amdgcn_rcpf(2.f * filter_r) * log2e;
+        const float wa = alpha * (1.f - inv_denom), wb = alpha * inv_denom;
+        const float* nrm = kp->nrm;
+        const float nx = nrm[q], ny = nrm[nq + q], nz = nrm[2 * (size_t)nq + q];
         bool bv = false;
         float bd2 = 0.f, bx = 0.f, by = 0.f, bz = 0.f, br = 0.f, bg = 0.f, bb = 0.f;
         auto consume = [&]() {
-            if (bv) {
-                const float cosNL = __fadd_rn(__fadd_rn(__fmul_rn(nx, -bx), __fmul_rn(ny, -by)), __fmul_rn(nz, -bz));
-                if (cosNL > 0.f) {
-                    const float d = sqrtf(bd2);
-                    const float x = __fdiv_rn(__fmul_rn(__fmul_rn(-beta, d), d), __fmul_rn(2.f, filter_r));
-                    const float w = __fmul_rn(alpha, 1.f - __fdiv_rn(1.f - expf(x), denom));
-                    res0 += br * w;
-                    res1 += bg * w;
-                    res2 += bb * w;
-                }
+            const float cosNL = __fadd_rn(__fadd_rn(__fmul_rn(nx, -bx), __fmul_rn(ny, -by)), __fmul_rn(nz, -bz));
+            if (bv && cosNL > 0.f) {
+                const float w = wa + wb * __builtin_amdgcn_exp2f(bd2 * s);
+                res0 += br * w;
+                res1 += bg * w;
+                res2 += bb * w;
             }
         };
-        auto take = [&](uint32_t avail) {  // lanes < avail take queue entries 0..avail-1
+        auto fetch = [&](ParamsPtr kt, uint32_t off) {
+            const uint32_t n = kt->n;
+            const float *dir = kt->dir, *pow = kt->power;
+            bx = bload(plane_rsrc(dir, n), off);
+            by = bload(plane_rsrc(dir + n, n), off);
+            bz = bload(plane_rsrc(dir + 2 * (size_t)n, n), off);
+            br = bload(plane_rsrc(pow, n), off);
+            bg = bload(plane_rsrc(pow + n, n), off);
+            bb = bload(plane_rsrc(pow + 2 * (size_t)n, n), off);
+        };
+        uint32_t head = 0, qn = 0;  // ring: entries head ... head + qn - 1 (mod its size)
+        auto take = [&](uint32_t avail) {  // lanes < avail take the first entries
             bv = lane < avail;
-            const uint64_t key = bv ? L.buf[lane] : 0ull;
-            const uint32_t off = (uint32_t)key * 4u;
-            bd2 = __uint_as_float((uint32_t)(key >> 32));
             if (bv) {
-                bx = bload(rdx, off);
-                by = bload(rdy, off);
-                bz = bload(rdz, off);
-                br = bload(rpr, off);
-                bg = bload(rpg, off);
-                bb = bload(rpb, off);
+                const uint64_t key = L.ring[(head + lane) & (kWideRing - 1u)];
+                bd2 = __uint_as_float((uint32_t)(key >> 32));
+                fetch(opaque(kp0), (uint32_t)key * 4u);
             }
         };
-        uint32_t qn = 0;
-        wave_sync();  // the buffer's previous contents are dead
-        walk2(P, lane, B, qx, qy, qz, T, [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
-            const bool va = __builtin_amdgcn_inverse_ballot_w64(am), vb = __builtin_amdgcn_inverse_ballot_w64(bm);
-            const bool sela = d2a <= (va ? T : -1.0f) && make_key(d2a, sa) <= kstar;
-            const bool selb = d2b <= (vb ? T : -1.0f) && make_key(d2b, sb) <= kstar;
-            const uint64_t ba = wballot(sela), bbal = wballot(selb);
-            const uint32_t na = (uint32_t)__popcll(ba);
-            if (sela) L.buf[qn + mbcnt(ba)] = make_key(d2a, sa);
-            if (selb) L.buf[qn + na + mbcnt(bbal)] = make_key(d2b, sb);
-            qn += na + (uint32_t)__popcll(bbal);  // < 64 + 128: the queue holds < 64 between steps
-            while (qn >= 64) {
-                wave_sync();
-                consume();
-                take(64);
-                // entries 64 .. qn-1 (fewer than 128) move to the front
-                const uint64_t r0 = lane + 64 < qn ? L.buf[64 + lane] : 0ull;
-                const uint64_t r1 = lane + 128 < qn ? L.buf[128 + lane] : 0ull;
-                wave_sync();
-                if (lane + 64 < qn) L.buf[lane] = r0;
-                if (lane + 128 < qn) L.buf[64 + lane] = r1;
-                qn -= 64;
-                wave_sync();
-            }
-        });
+        wave_sync();  // the list is read before the ring is written
+        walk_query(kp0, lane, W, lb, batch, false, hi,
+                   [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
+                       const uint64_t ka = make_key(d2a, sa), kb = make_key(d2b, sb);
+                       const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot(ka <= kstar),
+                                      bbal = bm & wballot(__float_as_uint(d2b) < hi) & wballot(kb <= kstar);
+                       const uint32_t at = __builtin_amdgcn_readfirstlane(head + qn),
+                                      bt = __builtin_amdgcn_readfirstlane(at + (uint32_t)__popcll(ba));
+                       if (__builtin_amdgcn_inverse_ballot_w64(ba))
+                           L.ring[(at + mbcnt(ba)) & (kWideRing - 1u)] = ka;
+                       if (__builtin_amdgcn_inverse_ballot_w64(bbal))
+                           L.ring[(bt + mbcnt(bbal)) & (kWideRing - 1u)] = kb;
+                       // (fewer than 64 + 128: the ring holds fewer than 64 between steps)
+                       qn = bt - head + (uint32_t)__popcll(bbal);
+                       while (qn >= 64) {
+                           wave_sync();
+                           consume();
+                           take(64);
+                           wave_sync();
+                           head = __builtin_amdgcn_readfirstlane(head + 64u);
+                           qn -= 64;
+                       }
+                   });
         wave_sync();
         consume();
         take(qn);
         consume();
     }
-    res0 = wave_sum_f32(res0);
-    res1 = wave_sum_f32(res1);
-    res2 = wave_sum_f32(res2);
-    if (lane == 0) {
-        float coef = 1.f;
-        if (m > 0) coef = __fdiv_rn(1.f, __fmul_rn(__fmul_rn(pi_f, __fmul_rn(rmax, rmax)), 1.f));
-        P.rgb[q] = m > 0 ? res0 * coef : 0.f;
-        P.rgb[P.nq + q] = m > 0 ? res1 * coef : 0.f;
-        P.rgb[2 * (size_t)P.nq + q] = m > 0 ? res2 * coef : 0.f;
+    const float tot = wave_sum3_f32(res0, res1, res2);
+    if ((lane & 15) == 15 && lane < 63) {
+        const float coef = __builtin_amdgcn_rcpf(__fmul_rn(pi_f, __fmul_rn(rmax, rmax)));
+        const uint32_t plane = lane == 15 ? 0u : lane == 31 ? 2u : 1u;
+        kp->rgb[(size_t)plane * nq + q] = m > 0 ? tot * coef : 0.f;
+    }
+    return true;
+}
+
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6))) void k_gather_wide(
+    KnnParams P, uint32_t* __restrict__ ovf_list, uint32_t* __restrict__ ovf_count) {
+    __shared__ WideLds lds[kWaves];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t blk = P.remap == 2 ? xcd_chunked(blockIdx.x, P.xcd_shift)
+                         : P.remap   ? pmd::xcd_remap(blockIdx.x, gridDim.x)
+                                     : blockIdx.x;
+    const uint32_t nq = P.nq_dev ? min(P.nq, *P.nq_dev) : P.nq;
+    const uint32_t u = blk * kWaves + wave;
+    if (u >= nq || u >= P.n_waves) return;  // wave-uniform; no workgroup barriers below
+    ParamsPtr kp0 = (ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    const uint32_t nqw = wave_queries(u, P.n_waves, (uint32_t)P.gq, nq);
+    WaveQueries W;
+    setup_queries(kp0, lane, P.order, u, P.n_waves, 0u, nqw, W);
+    for (uint32_t i = 0; i < nqw; ++i) {
+        const uint32_t lb = i * (uint32_t)opaque(kp0)->nr;
+        if (!wide_query(kp0, W, lb, lane, lds[wave]) && lane == 0)
+            ovf_list[atomicAdd(ovf_count, 1u)] = __builtin_amdgcn_readlane(W.q, lb);
+        wave_sync();
     }
 }
 
@@ -1512,6 +1600,8 @@ void split_waves(KnnParams& P, uint64_t total) {
     P.n_waves = pm::div_up(P.nq, (uint32_t)P.gq);
     // (a single query's wave would only wait for the second look-up of its
     // rows, and the inner box is about the guess already)
+    const float cr = 1.f + 0.6f * P.G.cell / std::max(P.r, 1e-30f);
+    P.within = 1.f / (cr * cr);
     P.guess = P.gq > 1 && P.h == 0 ? 1.2f * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
 }
 
@@ -1571,10 +1661,13 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
     if (wide) {
         pm_status st = pm::fill_u32(ctx, ovf_count, 0u, 1);
         if (st != PM_OK) return st;
-        uint32_t nblk = pm::div_up(P.nq, kWaves);
-        P.xcd_shift = xcd_shift_for(nblk, 1);
+        P.h = 0;  // (the inner box is the k <= 256 gathers')
+        split_waves(P, P.nq);
+        uint32_t nblk = pm::div_up(P.n_waves, kWaves);
+        P.xcd_shift = xcd_shift_for(nblk, (uint32_t)P.gq);
         if (P.remap == 2) nblk = xcd_round(nblk, P.xcd_shift);
-        hipLaunchKernelGGL(k_gather_wide, dim3(nblk), dim3(256), 0, ctx->stream, P, ovf_list, ovf_count);
+        hipLaunchKernelGGL(k_gather_wide, dim3(nblk), dim3(256), 0,
+                           ctx->stream, P, ovf_list, ovf_count);
         PM_CHECK_LAUNCH(ctx, "k_gather_wide");
         const uint32_t lblocks = std::min<uint32_t>(P.nq, (uint32_t)std::max(ctx->cu_count, 1) * 8u);
         if (P.k > 1024)
@@ -1603,7 +1696,9 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
     const bool lists = P.out_idx != nullptr;
     if (two_pass)
         hipLaunchKernelGGL(k_knn_two_pass, grid_dim, block, 0, ctx->stream, P);
-    else if (mid || ((flags & PM_KNN_LARGE_BUFFER) && !lists))
+    else if (mid)
+        hipLaunchKernelGGL((k_knn_stream<768, false>), grid_dim, block, 0, ctx->stream, P);
+    else if ((flags & PM_KNN_LARGE_BUFFER) && !lists)
         hipLaunchKernelGGL((k_knn_stream<1024, false>), grid_dim, block, 0, ctx->stream, P);
     else if (flags & PM_KNN_LARGE_BUFFER)
         hipLaunchKernelGGL((k_knn_stream<1024, true>), grid_dim, block, 0, ctx->stream, P);

@@ -76,3 +76,33 @@ def test_lists_and_estimate(ctx, inputs, cell, layout, flags, nq, k):
         assert np.array_equal(np.isnan(got), nan)
         assert np.all(np.abs(got - want)[~nan] <= 1e-5 * np.abs(want)[~nan])
     g.close()
+
+
+# (the mid kernel up to k = 512, the wide one above: few enough in reach, more
+# than expected, many more; a point's equal distances fill a crossing bin)
+@pytest.mark.parametrize("r,cell,flags,nq,k", [
+    (0.15, 1.0, pm355.KNN_SORT_QUERIES, 2 * FILL + 3, 300),
+    (0.2, 0.5, 0, 3001, 512),
+    (0.15, 1.0, pm355.KNN_SORT_QUERIES, 2 * FILL + 3, 513),
+    (0.2, 0.4, pm355.KNN_INNER_BOX, 3001, 600),
+    (0.25, 1.0, 0, 3001, 700),
+    (0.3, 1.0, pm355.KNN_SORT_QUERIES, 2 * FILL + 1, 2000),
+    (0.3, 0.2, 0, 777, 2048),
+])
+def test_large_k_estimate(ctx, inputs, r, cell, flags, nq, k):
+    ph, q, qn, aabb = inputs
+    q, qn = np.ascontiguousarray(q[:, :nq]), np.ascontiguousarray(qn[:, :nq])
+    g = ctx.grid_build(ph, aabb, cell_size=r * cell)
+    og = O.OracleGrid(ph, aabb, cell_size=r * cell)
+    oi, od, oc = og.knn(q, r, k)
+    _, o64 = O.radiance(oi, od, oc, og.photons, qn, k)
+    rgb, cnt = ctx.gather_radiance(g, q, qn, r, k, flags, want_count=True)
+    few = ctx.gather_radiance(g, q[:, :77].copy(), qn[:, :77].copy(), r, k, flags)
+    ctx.sync()
+    assert np.array_equal(cnt.cpu().numpy().view(np.uint32), oc)
+    assert np.array_equal(few.cpu().numpy().view(np.uint32), rgb[:, :77].cpu().numpy().view(np.uint32))
+    got = rgb.cpu().numpy().astype(np.float64)
+    nan = np.isnan(o64)  # (k photons at the query itself)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.all(np.abs(got - o64)[~nan] <= 1e-5 * np.abs(o64)[~nan])
+    g.close()
