@@ -106,3 +106,29 @@ def test_large_k_estimate(ctx, inputs, r, cell, flags, nq, k):
     assert np.array_equal(np.isnan(got), nan)
     assert np.all(np.abs(got - o64)[~nan] <= 1e-5 * np.abs(o64)[~nan])
     g.close()
+
+
+# Lists on a map with a density step: beside it the first walk's guess from the
+# candidate count falls short, by little (a second bound from the keys it
+# found), by a lot or with no key at all (the radius).
+@pytest.mark.parametrize("sparse,k", [(0, 50), (200, 50), (2000, 50), (20_000, 10), (20_000, 200)])
+def test_lists_beside_a_density_step(ctx, sparse, k):
+    rng = np.random.default_rng(41)
+    nq = 2 * FILL + 1
+    pos = rng.random((3, 60_000 + sparse), dtype=np.float32)
+    pos[0, :60_000] *= 0.5  # crowded below x = 0.5
+    pos[0, 60_000:] = 0.5 + 0.5 * pos[0, 60_000:]
+    pos[1] = 0.0
+    ph = np.concatenate([pos, np.full_like(pos, 1e-6), np.full_like(pos, -0.57)], 0)
+    q = rng.random((3, nq), dtype=np.float32)
+    q[0] = 0.45 + 0.1 * q[0]
+    q[1] = 0.0
+    aabb = (0.0, 0.0, 0.0, 1.0, 1.0, 1.0)
+    g = ctx.grid_build(ph, aabb, cell_size=R)
+    oi, od, oc = O.OracleGrid(ph, aabb, cell_size=R).knn(q, R, k)
+    idx, dist, cnt = ctx.knn(g, q, R, k, pm355.KNN_SORT_QUERIES)
+    ctx.sync()
+    assert np.array_equal(cnt.cpu().numpy().view(np.uint32), oc)
+    assert np.array_equal(idx.cpu().numpy().view(np.uint32), oi)
+    assert np.array_equal(dist.cpu().numpy(), od)
+    g.close()
