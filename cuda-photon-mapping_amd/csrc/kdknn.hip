@@ -184,21 +184,24 @@ __global__ __launch_bounds__(256) void k_kd_knn(KdParams P) {
     }
 
     const uint32_t m = found < k ? found : k;
+    uint32_t hi = __float_as_uint(T) + 1u;
+    khi = min(khi, (uint64_t)hi << 32);
     cnt = buf_select<kCap>(L.sel, lane, cnt, k, 256u, P.bT, khi);
+    hi = (uint32_t)((khi + 0xffffffffull) >> 32);
     wave_sync();
     uint32_t* irow = P.out_idx + (size_t)q * P.k;
     float* drow = P.out_dist + (size_t)q * P.k;
     if (cnt <= 64) {
         uint64_t v[1];
-        sort_keys<1, kCap>(L.sel, lane, cnt, v);
+        sort_keys<1, kCap>(L.sel, lane, cnt, hi, v);
         write_rows<1>(v, lane, m, P.k, irow, drow);
     } else if (cnt <= 128) {
         uint64_t v[2];
-        sort_keys<2, kCap>(L.sel, lane, cnt, v);
+        sort_keys<2, kCap>(L.sel, lane, cnt, hi, v);
         write_rows<2>(v, lane, m, P.k, irow, drow);
     } else {
         uint64_t v[4];
-        sort_keys<4, kCap>(L.sel, lane, cnt, v);
+        sort_keys<4, kCap>(L.sel, lane, cnt, hi, v);
         write_rows<4>(v, lane, m, P.k, irow, drow);
     }
     if (lane == 0) P.out_count[q] = m;

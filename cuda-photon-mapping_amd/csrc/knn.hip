@@ -405,14 +405,9 @@ __device__ __forceinline__ void radiance_epilogue(const KnnParams& P, const uint
 
 template <int R, int CAP>
 __device__ __forceinline__ void sort_and_emit(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, uint32_t q,
-                                              uint32_t cnt, uint32_t m) {
+                                              uint32_t cnt, uint32_t m, uint32_t hi) {
     uint64_t v[R];
-#pragma unroll
-    for (int j = 0; j < R; ++j) {
-        uint32_t e = (uint32_t)j * 64 + lane;
-        v[j] = e < cnt ? L.buf[e] : ~0ull;
-    }
-    bitonic_sort<R>(v, lane);
+    sort_keys<R, CAP>(L, lane, cnt, hi, v);
     if (P.out_idx) {
 #pragma unroll
         for (int j = 0; j < R; ++j) {
@@ -513,16 +508,18 @@ __device__ __forceinline__ void finish(const KnnParams& P, WaveLds<CAP>& L, uint
     const uint32_t k = (uint32_t)P.k;
     const uint32_t m = cnt < k ? cnt : k;
     if (kLists && P.out_idx) {
-        // narrowed to the smallest sort that holds k keys (64, 128 or 256)
-        uint64_t khi = (uint64_t)hi << 32;
-        cnt = buf_select<CAP>(L, lane, cnt, k, k <= 64 ? 64u : k <= 128 ? 128u : 256u, P.bT, khi);
-        wave_sync();
+        if (cnt > 256u) {
+            uint64_t khi = (uint64_t)hi << 32;
+            cnt = buf_select<CAP>(L, lane, cnt, k, 256u, P.bT, khi);
+            hi = (uint32_t)((khi + 0xffffffffull) >> 32);
+            wave_sync();
+        }
         if (cnt <= 64)
-            sort_and_emit<1, CAP>(P, L, lane, q, cnt, m);
+            sort_and_emit<1, CAP>(P, L, lane, q, cnt, m, hi);
         else if (cnt <= 128)
-            sort_and_emit<2, CAP>(P, L, lane, q, cnt, m);
+            sort_and_emit<2, CAP>(P, L, lane, q, cnt, m, hi);
         else
-            sort_and_emit<4, CAP>(P, L, lane, q, cnt, m);
+            sort_and_emit<4, CAP>(P, L, lane, q, cnt, m, hi);
         return;
     }
     // no neighbour lists: narrow to exactly the k smallest and estimate
