@@ -52,13 +52,47 @@ __global__ __launch_bounds__(256) void k_cell_sizes(const uint32_t* __restrict__
         atomicAdd(&sizes[key], i + 1);
 }
 
-// analyze_density_kernel's max (PhotonGrid.cu:70-90), as a reduction.
-__global__ __launch_bounds__(256) void k_max_u32(const uint32_t* __restrict__ a, uint32_t n, uint32_t* __restrict__ out) {
-    uint32_t m = 0;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = max(m, a[i]);
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
+// Whether any cell holds more than `limit` photons (analyze_density_kernel,
+// PhotonGrid.cu:70-141, needs its maximum for this comparison only): photons
+// are counted by atomics until a workgroup finds that a count has passed the
+// limit. The answer does not depend on the order. A workgroup counts its share
+// in LDS first where the cells fit (kLds: 2M photons of the default 1000 a
+// cell are 2k cells, and neighbours in the input fall in the same cell). The
+// flag is read once a share and written where a count passes the limit, not at
+// every photon: one address serves about 0.2 requests a nanosecond (2M photons
+// 168 us with a read each wave, 240 with the counts in memory too).
+constexpr uint32_t kOverThreads = 1024, kOverCells = 16384;
+template <bool kLds>
+__global__ __launch_bounds__(kOverThreads) void k_any_over(const float* __restrict__ in9, uint32_t n, size_t stride,
+                                                          GridGeom G, uint32_t n_cells, uint32_t limit,
+                                                          uint32_t* __restrict__ counts, uint32_t* __restrict__ over) {
+    extern __shared__ uint32_t s_counts[];
+    __shared__ uint32_t s_over;
+    const uint32_t t = threadIdx.x;
+    if (t == 0) s_over = __hip_atomic_load(over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_over) return;  // (workgroup-uniform)
+    if (kLds) {
+        for (uint32_t c = t; c < n_cells; c += kOverThreads) s_counts[c] = 0;
+        __syncthreads();
+    }
+    for (uint32_t i = blockIdx.x * kOverThreads + t; i < n; i += gridDim.x * kOverThreads) {
+        const int x = pmd::cell_coord(in9[i], G.mn[0], G.cell, G.g[0]);
+        const int y = pmd::cell_coord(in9[stride + i], G.mn[1], G.cell, G.g[1]);
+        const int z = pmd::cell_coord(in9[2 * stride + i], G.mn[2], G.cell, G.g[2]);
+        if (atomicAdd((kLds ? s_counts : counts) + pmd::cell_index(G, x, y, z), 1u) == limit)
+            __hip_atomic_store(over, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (kLds) {
+        __syncthreads();
+        for (uint32_t c = t; c < n_cells; c += kOverThreads) {
+            const uint32_t v = s_counts[c];
+            if (v == 0) continue;
+            const uint32_t was = atomicAdd(&counts[c], v);
+            if (was <= limit && was + v > limit)
+                __hip_atomic_store(over, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 // assign_photons_to_cells (PhotonGrid.cu:152-174) with the slot taken from
@@ -187,7 +221,7 @@ size_t grid_bytes(uint32_t n_cells, uint32_t n_cap) {
     return pm::carve_size({(size_t)n_cells * 4, (size_t)n_cells * 4, (size_t)n_cap * 36, (size_t)n_cap * 4});
 }
 
-// scratch of one build: the density counter, keys, sorted keys, sorted
+// scratch of one build: the density flag, keys, sorted keys, sorted
 // order, radix work, records
 size_t build_scratch_bytes(uint32_t n) {
     return pm::carve_size({256, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, pm::radix_sort_scratch_bytes(n),
@@ -283,16 +317,16 @@ pm_status grid_build_strided(pm_ctx* ctx, const float* d_photons9, uint32_t n, s
         return pm::fail(ctx, PM_ERR_UNSUPPORTED, "pm_grid_build: grid too large for cell %g", (double)cell);
 
     pm_status st;
-    uint32_t* dmax = nullptr;
+    uint32_t* over = nullptr;
     {
         void* w = nullptr;
         if ((st = pm::scratch_reserve(ctx, build_scratch_bytes(n), &w)) != PM_OK) return st;
         pm::Carve cv{static_cast<char*>(w)};
-        dmax = cv.take<uint32_t>(64);
+        over = cv.take<uint32_t>(64);
     }
 
-    // One build at dims d into a fresh allocation of capacity n.
-    auto build_once = [&](const HostDims& dd, pm_grid*& out_g) -> pm_status {
+    // a fresh allocation of capacity n at dims dd
+    auto take = [&](const HostDims& dd, pm_grid*& out_g) -> pm_status {
         pm_grid* g = new pm_grid();
         hipError_t e = pm::block_take(ctx, grid_bytes(dd.n_cells, n), &g->mem, &g->mem_bytes);
         if (e != hipSuccess) {
@@ -301,37 +335,56 @@ pm_status grid_build_strided(pm_ctx* ctx, const float* d_photons9, uint32_t n, s
         }
         g->owner = ctx;
         g->n_cap = n;
-        pm_status bs = enqueue_build(ctx, d_photons9, n, stride, aabb, dd, layout, g);
-        if (bs != PM_OK) {
-            pm_grid_destroy(g);
-            return bs;
-        }
         out_g = g;
+        return PM_OK;
+    };
+    // whether a cell at dims d holds more than `limit` photons (the counts are
+    // taken in g's memory, ahead of its build)
+    auto any_over = [&](pm_grid* g, uint32_t limit, bool& yes) -> pm_status {
+        uint32_t* counts = static_cast<uint32_t*>(g->mem);
+        pm_status s;
+        if ((s = pm::fill_u32(ctx, counts, 0u, d.n_cells)) != PM_OK || (s = pm::fill_u32(ctx, over, 0u, 1)) != PM_OK)
+            return s;
+        const dim3 blocks(std::min(pm::div_up(n, 4 * kOverThreads), 512u)), threads(kOverThreads);
+        if (d.n_cells <= kOverCells)
+            hipLaunchKernelGGL(k_any_over<true>, blocks, threads, d.n_cells * 4, ctx->stream, d_photons9, n, stride,
+                               geom_of(aabb, d, layout), d.n_cells, limit, counts, over);
+        else
+            hipLaunchKernelGGL(k_any_over<false>, blocks, threads, 0, ctx->stream, d_photons9, n, stride,
+                               geom_of(aabb, d, layout), d.n_cells, limit, counts, over);
+        PM_CHECK_LAUNCH(ctx, "k_any_over");
+        uint32_t h = 0;
+        PM_HIP(ctx, hipMemcpyAsync(&h, over, 4, hipMemcpyDeviceToHost, ctx->stream));
+        PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        yes = h != 0;
         return PM_OK;
     };
 
     pm_grid* g = nullptr;
-    if ((st = build_once(d, g)) != PM_OK) return st;
+    if ((st = take(d, g)) != PM_OK) return st;
     if (!(cell_size > 0.f)) {
         // analyze_density (PhotonGrid.cu:92-141): at the reference size, the
-        // fullest cell (read from the built grid's sizes) decides whether the
-        // cells shrink to the size for desired / 5; then the grid is built
-        // again at that size.
-        if ((st = pm::fill_u32(ctx, dmax, 0u, 1)) != PM_OK) return st;
-        hipLaunchKernelGGL(k_max_u32, dim3(std::min<uint32_t>(pm::div_up(d.n_cells, 256), 4096)), dim3(256), 0,
-                           ctx->stream, g->desc.d_cell_sizes, d.n_cells, dmax);
-        PM_CHECK_LAUNCH(ctx, "k_max_u32");
-        uint32_t mx = 0;
-        PM_HIP(ctx, hipMemcpyAsync(&mx, dmax, 4, hipMemcpyDeviceToHost, ctx->stream));
-        PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (mx > 5u * (uint32_t)desired) {
+        // fullest cell decides whether the cells shrink to the size for
+        // desired / 5. The count alone decides, so the grid is built once, at
+        // the final size (2M photons: 230 us, 375 with a build at each size; the
+        // count takes 22).
+        bool shrink = false;
+        if ((st = any_over(g, 5u * (uint32_t)desired, shrink)) != PM_OK) {
+            pm_grid_destroy(g);
+            return st;
+        }
+        if (shrink) {
             pm_grid_destroy(g);
             g = nullptr;
             cell = reference_cell(n, aabb, std::max(1, desired / 5));
             if (!(cell > 0.f) || !make_dims(aabb, cell, layout, d))
                 return pm::fail(ctx, PM_ERR_UNSUPPORTED, "pm_grid_build: grid too large for cell %g", (double)cell);
-            if ((st = build_once(d, g)) != PM_OK) return st;
+            if ((st = take(d, g)) != PM_OK) return st;
         }
+    }
+    if ((st = enqueue_build(ctx, d_photons9, n, stride, aabb, d, layout, g)) != PM_OK) {
+        pm_grid_destroy(g);
+        return st;
     }
     *out = g;
     return PM_OK;
