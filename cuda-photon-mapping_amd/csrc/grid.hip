@@ -97,18 +97,21 @@ __global__ __launch_bounds__(kOverThreads) void k_any_over(const float* __restri
 
 // assign_photons_to_cells (PhotonGrid.cu:152-174) with the slot taken from
 // the stable sort instead of an atomic: in-cell order = input order. One
-// 48-byte record gathered per photon, nine coalesced plane writes.
+// 48-byte record gathered per photon, nine coalesced plane writes, past the
+// cache: what it holds is worth more to the gathered records, of which half
+// straddle a 64-byte line (16M photons 560 -> 521 us; records padded to 64
+// bytes 505, but their writing 280 -> 513).
 __global__ __launch_bounds__(256) void k_grid_scatter(const float4* __restrict__ rec, uint32_t n,
                                                      const uint32_t* __restrict__ order, float* __restrict__ out9,
                                                      uint32_t* __restrict__ perm) {
     uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t src = order[j];
-    perm[j] = src;
+    __builtin_nontemporal_store(src, perm + j);
     const float4 a = rec[3 * (size_t)src + 0], b = rec[3 * (size_t)src + 1], c = rec[3 * (size_t)src + 2];
     const float v[9] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, c.x};
 #pragma unroll
-    for (int p = 0; p < 9; ++p) out9[(size_t)p * n + j] = v[p];
+    for (int p = 0; p < 9; ++p) __builtin_nontemporal_store(v[p], out9 + (size_t)p * n + j);
 }
 
 struct HostDims {
