@@ -1,4 +1,4 @@
-// Single-pass u32 prefix scan: wave64 shuffle scan inside a 4096-element
+// Single-pass u32 prefix scan: wave64 shuffle scan inside an 8192-element
 // tile, decoupled look-back across tiles (Merrill & Garland 2016). Tile
 // words carry an epoch held in device memory (read by every tile, advanced
 // by the last), so consecutive launches need no clearing pass and a launch
@@ -6,7 +6,7 @@
 // the reference's 44-block Blelloch scan with its software grid barrier
 // (PrefixScanSum.cuh:12-279, CudaGridSynchronizer.cuh:14-27), which needs all
 // blocks co-resident; here a tile only waits on tiles that took a lower
-// ordered id, so any number of tiles may be in flight. Inputs of 4M
+// ordered id, so any number of tiles may be in flight. Inputs of 6M
 // elements and more take a two-level scan instead (tile sums, a scan of the
 // sums, tiles rescanned from their offsets), whose workgroups never wait on
 // each other.
@@ -14,13 +14,24 @@
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kItems = 16;
-constexpr int kTile = kThreads * kItems;  // 4096
+// The single pass's tiles. Its ordered tile counter hands out one id in about
+// 22 ns (one device-scope atomic a tile, all on one line), which bounds it from
+// some 100 tiles on, while a tile's own latency grows with what one CU reads:
+// 1024 threads of 8 elements take 7.4 us at 1M elements, 9.9 at 2M and 16.2
+// at 4M (tiles of 4096: 8.8, 14.7, 26; of 16384: 8.4, 10.3, 14.5, and 7.5
+// instead of 6.1 at 500k).
+constexpr int kThreads = 1024;
+constexpr int kItems = 8;
+constexpr int kTile = kThreads * kItems;  // 8192
+// The two-level scan's tiles: nothing waits, so they are small.
+constexpr int kThreads2 = 256;
+constexpr int kItems2 = 16;
+constexpr int kTile2 = kThreads2 * kItems2;  // 4096
 
 constexpr uint64_t kStatusAgg = 1, kStatusIncl = 2;
-// inputs of at least this many elements take the two-level scan
-constexpr uint32_t kTwoLevelMin = 1u << 22;
+// inputs of at least this many elements take the two-level scan (4M: 16.2 us in
+// a single pass, 25.6 in two levels; 8M: 28.9 and 25.0)
+constexpr uint32_t kTwoLevelMin = 6u << 20;
 
 __device__ __forceinline__ uint64_t pack_state(uint32_t epoch, uint64_t status, uint32_t value) {
     return ((uint64_t)epoch << 34) | (status << 32) | value;
@@ -173,22 +184,22 @@ __global__ void k_zero_u64(uint64_t* p) { *p = 0; }
 // each tile rescanned from its offset. Three passes and no waiting between
 // workgroups: past a few million elements the single pass is held up by
 // its ordered tile counter, one device-scope atomic per tile.
-__global__ __launch_bounds__(kThreads) void k_tile_sums(const uint32_t* __restrict__ in, uint32_t n,
+__global__ __launch_bounds__(kThreads2) void k_tile_sums(const uint32_t* __restrict__ in, uint32_t n,
                                                        uint32_t* __restrict__ sums) {
-    __shared__ uint32_t s_wave[kThreads / 64];
+    __shared__ uint32_t s_wave[kThreads2 / 64];
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const size_t base = (size_t)blockIdx.x * kTile + (size_t)t * kItems;
+    const size_t base = (size_t)blockIdx.x * kTile2 + (size_t)t * kItems2;
     uint32_t sum = 0;
-    if (base + kItems <= n && ((reinterpret_cast<uintptr_t>(in) & 15) == 0)) {
+    if (base + kItems2 <= n && ((reinterpret_cast<uintptr_t>(in) & 15) == 0)) {
         const uint4* p = reinterpret_cast<const uint4*>(in + base);
 #pragma unroll
-        for (int j = 0; j < kItems / 4; ++j) {
+        for (int j = 0; j < kItems2 / 4; ++j) {
             const uint4 q = p[j];
             sum += q.x + q.y + q.z + q.w;
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < kItems; ++j) sum += (base + j < n) ? in[base + j] : 0u;
+        for (int j = 0; j < kItems2; ++j) sum += (base + j < n) ? in[base + j] : 0u;
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
@@ -197,23 +208,23 @@ __global__ __launch_bounds__(kThreads) void k_tile_sums(const uint32_t* __restri
     if (t == 0) {
         uint32_t a = 0;
 #pragma unroll
-        for (int w = 0; w < kThreads / 64; ++w) a += s_wave[w];
+        for (int w = 0; w < kThreads2 / 64; ++w) a += s_wave[w];
         sums[blockIdx.x] = a;
     }
 }
 
 template <bool kInclusive>
-__global__ __launch_bounds__(kThreads) void k_tile_rescan(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+__global__ __launch_bounds__(kThreads2) void k_tile_rescan(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
                                                          uint32_t n, const uint32_t* __restrict__ offs) {
-    __shared__ uint32_t s_wave[kThreads / 64];
+    __shared__ uint32_t s_wave[kThreads2 / 64];
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const size_t base = (size_t)blockIdx.x * kTile + (size_t)t * kItems;
-    const bool full = base + kItems <= n;
-    uint32_t v[kItems];
+    const size_t base = (size_t)blockIdx.x * kTile2 + (size_t)t * kItems2;
+    const bool full = base + kItems2 <= n;
+    uint32_t v[kItems2];
     if (full && ((reinterpret_cast<uintptr_t>(in) & 15) == 0)) {
         const uint4* p = reinterpret_cast<const uint4*>(in + base);
 #pragma unroll
-        for (int j = 0; j < kItems / 4; ++j) {
+        for (int j = 0; j < kItems2 / 4; ++j) {
             const uint4 q = p[j];
             v[4 * j] = q.x;
             v[4 * j + 1] = q.y;
@@ -222,21 +233,21 @@ __global__ __launch_bounds__(kThreads) void k_tile_rescan(const uint32_t* __rest
         }
     } else {
 #pragma unroll
-        for (int j = 0; j < kItems; ++j) v[j] = (base + j < n) ? in[base + j] : 0u;
+        for (int j = 0; j < kItems2; ++j) v[j] = (base + j < n) ? in[base + j] : 0u;
     }
     uint32_t tsum = 0;
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) tsum += v[j];
+    for (int j = 0; j < kItems2; ++j) tsum += v[j];
     const uint32_t incl = wave_incl_scan(tsum, lane);
     if (lane == 63) s_wave[wave] = incl;
     __syncthreads();
     uint32_t run = offs[blockIdx.x] + (incl - tsum);
 #pragma unroll
-    for (int w = 0; w < kThreads / 64; ++w)
+    for (int w = 0; w < kThreads2 / 64; ++w)
         if ((uint32_t)w < wave) run += s_wave[w];
-    uint32_t o[kItems];
+    uint32_t o[kItems2];
 #pragma unroll
-    for (int j = 0; j < kItems; ++j) {
+    for (int j = 0; j < kItems2; ++j) {
         if (kInclusive) {
             run += v[j];
             o[j] = run;
@@ -248,10 +259,10 @@ __global__ __launch_bounds__(kThreads) void k_tile_rescan(const uint32_t* __rest
     if (full && ((reinterpret_cast<uintptr_t>(out) & 15) == 0)) {
         uint4* p = reinterpret_cast<uint4*>(out + base);
 #pragma unroll
-        for (int j = 0; j < kItems / 4; ++j) p[j] = make_uint4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
+        for (int j = 0; j < kItems2 / 4; ++j) p[j] = make_uint4(o[4 * j], o[4 * j + 1], o[4 * j + 2], o[4 * j + 3]);
     } else {
 #pragma unroll
-        for (int j = 0; j < kItems; ++j)
+        for (int j = 0; j < kItems2; ++j)
             if (base + j < n) out[base + j] = o[j];
     }
 }
@@ -298,8 +309,8 @@ pm_status scan_u32(pm_ctx* ctx, const uint32_t* in, uint32_t* out, uint32_t n, b
         }
         return PM_OK;
     }
-    uint32_t tiles = div_up(n, kTile);
     if (n >= kTwoLevelMin && !ctx->fixed_state) {
+        const uint32_t tiles = div_up(n, kTile2);
         // tile sums and their offsets in the context's own block (callers'
         // scratch carves stay untouched)
         if (2 * (size_t)tiles > ctx->tile_sums_cap) {
@@ -312,17 +323,18 @@ pm_status scan_u32(pm_ctx* ctx, const uint32_t* in, uint32_t* out, uint32_t n, b
         }
         uint32_t* sums = ctx->tile_sums;
         uint32_t* offs = ctx->tile_sums + tiles;
-        hipLaunchKernelGGL(k_tile_sums, dim3(tiles), dim3(kThreads), 0, ctx->stream, in, n, sums);
+        hipLaunchKernelGGL(k_tile_sums, dim3(tiles), dim3(kThreads2), 0, ctx->stream, in, n, sums);
         PM_CHECK_LAUNCH(ctx, "k_tile_sums");
         pm_status st = scan_u32(ctx, sums, offs, tiles, false, total);
         if (st != PM_OK) return st;
         if (inclusive)
-            hipLaunchKernelGGL(k_tile_rescan<true>, dim3(tiles), dim3(kThreads), 0, ctx->stream, in, out, n, offs);
+            hipLaunchKernelGGL(k_tile_rescan<true>, dim3(tiles), dim3(kThreads2), 0, ctx->stream, in, out, n, offs);
         else
-            hipLaunchKernelGGL(k_tile_rescan<false>, dim3(tiles), dim3(kThreads), 0, ctx->stream, in, out, n, offs);
+            hipLaunchKernelGGL(k_tile_rescan<false>, dim3(tiles), dim3(kThreads2), 0, ctx->stream, in, out, n, offs);
         PM_CHECK_LAUNCH(ctx, "k_tile_rescan");
         return PM_OK;
     }
+    const uint32_t tiles = div_up(n, kTile);
     uint64_t* state;
     uint32_t* counter;
     pm_status st = lookback_begin(ctx, tiles, &state, &counter);
