@@ -12,7 +12,7 @@
 //   * at every level each node's segment [from, to) has its median at
 //     mid = from + (to - from)/2 in the order of the node's split axis;
 //     the other two orders are stable-partitioned around that median in one
-//     pass (a segmented scan with decoupled look-back), so every order stays
+//     pass (counts with decoupled look-back), so every order stays
 //     sorted inside every child segment; subtrees of at most 1024 photons
 //     are finished in LDS by one workgroup each;
 //   * a child's split plane is the argmax extent of its points, read from
@@ -60,6 +60,7 @@ __device__ __forceinline__ uint32_t id_at(const Orders& O, int a, uint32_t j) {
 }
 
 constexpr uint32_t kFinal = 0xFFFFFFFFu;
+constexpr uint32_t kTicket = 32;  // words between the axes' tile counters (a line each)
 
 __device__ __forceinline__ uint32_t orderable(float f) {
     f = f + 0.0f;  // -0 -> +0 so that equal coordinates tie on the index
@@ -132,16 +133,18 @@ __device__ __forceinline__ int8_t plane_of(const Orders& O, uint32_t f, uint32_t
 // Per node of a level: its split plane (the argmax extent of its segment,
 // PhotonMap.cuh:252-273: an empty node keeps +-FLT_MAX corners -> plane 0)
 // and, when `medians`, its median, the median's key and the children's
-// segments (med = {the median's rank on the plane, its index}). root_n > 0:
+// segments (med = {the median's rank on the plane, the plane}). root_n > 0:
 // the level is the root's, whose segment is [0, root_n). lookback_counter
 // (nullable): the level partition before this launch has completed, so its
-// look-back epoch is advanced here.
+// look-back epoch is advanced here; the axes' tile counters start at 0 again.
 __global__ __launch_bounds__(256) void k_level_nodes(Orders O, uint32_t first, uint32_t count,
                                                     uint32_t cap, uint32_t root_n, bool medians, uint2* __restrict__ seg,
                                                     int8_t* __restrict__ plane, uint32_t* __restrict__ node_idx,
                                                     int8_t* __restrict__ node_plane, uint2* __restrict__ med,
-                                                    uint32_t* __restrict__ lookback_counter) {
+                                                    uint32_t* __restrict__ lookback_counter,
+                                                    uint32_t* __restrict__ tickets) {
     uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 3) tickets[t * kTicket] = 0;
     if (t == 0 && lookback_counter) pm::lookback_advance(lookback_counter, pm::lookback_epoch(lookback_counter));
     if (t >= count) return;
     uint32_t node = first + t;
@@ -160,7 +163,7 @@ __global__ __launch_bounds__(256) void k_level_nodes(Orders O, uint32_t first, u
     const uint32_t id = id_at(O, p, mid);
     node_idx[node] = id;
     node_plane[node] = p;
-    med[node] = make_uint2(O.rank4[4 * (size_t)id + p], id);
+    med[node] = make_uint2(O.rank4[4 * (size_t)id + p], (uint32_t)p);
     if (s.y - s.x == 1) {
         if (l < cap) seg[l] = make_uint2(0, 0);
         if (r < cap) seg[r] = make_uint2(0, 0);
@@ -179,201 +182,223 @@ __device__ __forceinline__ int side_of(const Rec& e, int p, uint2 m) {
 }
 
 // ---- one level's stable partition in one pass --------------------------------
-// The three axis orders are one stream of 3n positions (axis-major). Each
-// position carries a segmented-scan value: bit 31 = a segment starts here
-// (the node's `from`, or a finished position), bit 30 = the node's median,
-// bits 0-29 = goes left. A tile scans its positions in registers / LDS and
-// takes its prefix from earlier tiles by decoupled look-back (epoch-tagged
-// tile words, as in the u32 scan); within a node's segment the inclusive
-// value then counts the left records (Lb) and the median (Mb) up to each
-// position, which gives the destination directly:
-//   left: from + Lb,   median: mid,   right: mid + 1 + (j - from - Lb - Mb).
-// This replaces flags -> device scan -> scatter (three passes over 3n
-// positions) by one.
-constexpr int kPThreads = 512;                 // (kPItems * kPThreads / 64 wave rows <= 64: one wave scans them)
-constexpr int kPItems = 8;                      // rows of kPThreads positions per tile
-constexpr uint32_t kPTile = kPThreads * kPItems;  // 4096
-static_assert(kPItems * (kPThreads / 64) <= 64, "the wave rows of a tile are scanned by one wave");
-constexpr uint32_t kSegH = 1u << 31, kSegM = 1u << 30, kSegL = (1u << 30) - 1;
+// The three axis orders are three streams of n positions. A record
+// goes left, is its node's median or goes right; with the left records (lb) and
+// the median (mb) counted from its node's `from` up to it, its destination is
+//   left: from + lb,   median: mid,   right: mid + 1 + (j - from - lb - mb).
+// Both counts are differences of plain counts over a stream, whose values at
+// every node's start and end are known without counting: the nodes of a level
+// hold v or v + 1 records, adjacent ones are one finished median apart, and a
+// node of size s has s / 2 left records. So a row of 64 positions takes two
+// ballots, and a tile that holds any node's first or last position knows its
+// place in the stream; only a tile inside one node (the upper levels) takes
+// it from the tiles before it by decoupled look-back (epoch-tagged tile words,
+// as in the u32 scan; kLook), and the lower levels' tiles wait for nothing.
+// The axes' tiles are apart, each axis with its own ordered tile ids (a tile
+// waits for lower ids of its axis only, which have all started): one counter
+// hands out an id in about 22 ns, 16 us a level.
+// 2M photons, a level: 52 us with a segmented scan of flag words over each row
+// (171 VALU instructions for 64 positions, and one tile counter), now 39.6 where
+// tiles wait and 31.6 where they do not (25 is the copying at 5.1 TB/s).
+constexpr int kPThreads = 1024;
+constexpr int kPItems = 8;                        // rows of kPThreads positions per tile
+constexpr uint32_t kPTile = kPThreads * kPItems;  // 8192
+constexpr int kPRows = kPItems * (kPThreads / 64);  // wave rows, two a lane of the wave that scans them
+static_assert(kPRows == 128, "the wave rows of a tile are scanned by one wave, two a lane");
+// counts up to a position inside a tile: left records in bits 0-14, medians
+// from bit 15; and its record's side
+constexpr uint32_t kCntM = 1u << 15, kCnt = (1u << 30) - 1, kIsL = 1u << 30, kIsM = 1u << 31;
+// counts up to a tile: left records mod 2^30, the parity of the medians
+constexpr uint32_t kAbsL = (1u << 30) - 1, kAbsM = 1u << 30;
 constexpr uint64_t kStAgg = 1, kStIncl = 2;
 
-// x then y
-__device__ __forceinline__ uint32_t seg_op(uint32_t x, uint32_t y) {
-    if (y & kSegH) return y;
-    return ((x & kSegL) + (y & kSegL)) | ((x | y) & kSegM) | (x & kSegH);
+// A level's nodes: from `first` on, each of v or v + 1 records.
+struct Level {
+    uint32_t first, v;
+};
+
+__device__ __forceinline__ uint32_t abs_add(uint32_t x, uint32_t y) {
+    return ((x + y) & kAbsL) | ((x ^ y) & kAbsM);
+}
+// a count inside a tile as one up to a tile
+__device__ __forceinline__ uint32_t abs_of(uint32_t cnt) {
+    return (cnt & (kCntM - 1u)) | ((cnt & kCntM) ? kAbsM : 0u);
+}
+// the counts at the start of the level's node i, `from` its first position: c of
+// the nodes before it hold v + 1 records
+__device__ __forceinline__ uint32_t abs_at(const Level& V, uint32_t i, uint32_t from) {
+    const uint32_t c = from - i * (V.v + 1u);
+    const uint32_t l = i * (V.v >> 1) + ((V.v & 1u) ? c : 0u);
+    return (l & kAbsL) | ((i & 1u) ? kAbsM : 0u);
+}
+__device__ __forceinline__ uint32_t abs_sub(uint32_t x, uint32_t y) {
+    return ((x - y) & kAbsL) | ((x ^ y) & kAbsM);
 }
 
 __device__ __forceinline__ uint64_t seg_state(uint32_t epoch, uint64_t status, uint32_t value) {
     return ((uint64_t)epoch << 34) | (status << 32) | value;
 }
 
-__global__ __launch_bounds__(kPThreads) void k_level_partition(
+template <bool kLook>
+__global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(8))) void k_level_partition(
     const Rk* __restrict__ A0, const Rk* __restrict__ A1, const Rk* __restrict__ A2, Rk* __restrict__ B0,
     Rk* __restrict__ B1, Rk* __restrict__ B2, uint32_t n, const uint32_t* __restrict__ node_in,
-    uint32_t* __restrict__ node_out, const uint2* __restrict__ seg, const int8_t* __restrict__ plane,
-    const uint2* __restrict__ med, uint64_t* __restrict__ state, uint32_t* __restrict__ counter, uint32_t n_tiles) {
-    __shared__ uint32_t s_tile, s_epoch;
-    __shared__ uint32_t s_wagg[kPItems * (kPThreads / 64)];
-    __shared__ uint32_t s_wpre[kPItems * (kPThreads / 64)];
-    __shared__ uint32_t s_prefix;
+    uint32_t* __restrict__ node_out, const uint2* __restrict__ seg, const uint2* __restrict__ med, Level V,
+    uint64_t* __restrict__ state, const uint32_t* __restrict__ counter, uint32_t* __restrict__ tickets) {
+    __shared__ uint32_t s_tile, s_epoch, s_known, s_at;
+    __shared__ uint32_t s_row[kPRows];
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint32_t a = blockIdx.x % 3u, n_tiles = gridDim.x / 3u;  // the axis, and its tiles
     if (t == 0) {
-        // the epoch is advanced by k_level_nodes, the next launch: a tile
-        // here may finish its look-back before earlier tiles have read it
-        s_epoch = pm::lookback_epoch(counter);
-        uint32_t id = atomicAdd(counter, 1u);
-        if (id == n_tiles - 1) atomicExch(counter, 0u);  // every tile holds its id: reset for the next launch
-        s_tile = id;
+        s_known = 0;
+        s_tile = blockIdx.x / 3u;
+        if (kLook) {
+            // the epoch is advanced, and the tickets taken back, by
+            // k_level_nodes, the next launch: a tile here may finish its
+            // look-back before earlier tiles have read it
+            s_epoch = pm::lookback_epoch(counter);
+            s_tile = atomicAdd(&tickets[a * kTicket], 1u);
+        }
     }
     __syncthreads();
-    const uint32_t tile = s_tile, epoch = s_epoch;
-    const uint32_t total = 3u * n;  // n <= 2^30
+    const uint32_t tile = s_tile, j0 = tile * kPTile + t;  // n <= 2^30
+    const Rk* __restrict__ A = a == 0 ? A0 : a == 1 ? A1 : A2;
+    Rk* __restrict__ B = a == 0 ? B0 : a == 1 ? B1 : B2;
+    const uint32_t lo = (uint32_t)other_axis((int)a, 0);
 
     // position of item k: tile row k, wave, lane (rows of kPThreads consecutive
     // positions). All loads of the tile's items are issued before any item
-    // is scanned: positions, then their nodes' segments, planes and medians.
-    uint32_t val[kPItems], incl[kPItems], node[kPItems];
-    uint2 sgk[kPItems];
+    // is counted: positions, then their nodes' segments, planes and medians.
+    uint32_t node[kPItems], cnt[kPItems];
     Rk rec[kPItems];
 #pragma unroll
     for (int k = 0; k < kPItems; ++k) {
-        const uint32_t g = tile * kPTile + (uint32_t)k * kPThreads + t;
+        const uint32_t j = j0 + (uint32_t)k * kPThreads;
         node[k] = kFinal;
-        if (g < total) {
-            const uint32_t a = g >= 2 * n ? 2u : (g >= n ? 1u : 0u), j = g - a * n;
+        if (j < n) {
             node[k] = node_in[j];
-            rec[k] = (a == 0 ? A0 : a == 1 ? A1 : A2)[j];
+            rec[k] = A[j];
         }
     }
-    int8_t pl[kPItems];
-    uint2 md[kPItems];
+    // (this thread's latest position that is a node's first or last, and the
+    // counts before it)
+    int mark = -1;
+    uint32_t mark_abs = 0;
 #pragma unroll
     for (int k = 0; k < kPItems; ++k) {
+        const uint32_t j = j0 + (uint32_t)k * kPThreads;
+        bool is_l = false, is_m = false;
         if (node[k] != kFinal) {
-            sgk[k] = seg[node[k]];
-            pl[k] = plane[node[k]];
-            md[k] = med[node[k]];
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < kPItems; ++k) {
-        const uint32_t g = tile * kPTile + (uint32_t)k * kPThreads + t;
-        uint32_t v = kSegH;
-        if (node[k] != kFinal) {
-            const uint32_t a = g >= 2 * n ? 2u : (g >= n ? 1u : 0u), j = g - a * n;
+            const uint2 sg = seg[node[k]], md = med[node[k]];
+            const uint32_t half = (sg.y - sg.x) / 2;
             // the split axis's own order: the position decides; another
             // order: the record's rank on the split axis against the median's
-            int sd;
-            if (pl[k] == (int8_t)a) {
-                const uint32_t mid = sgk[k].x + (sgk[k].y - sgk[k].x) / 2;
-                sd = j < mid ? 0 : (j == mid ? 1 : 2);
-            } else {
-                const uint32_t rr = rec[k].r[pl[k] == other_axis((int)a, 0) ? 0 : 1];
-                sd = rr < md[k].x ? 0 : (rr == md[k].x ? 1 : 2);
+            const bool own = md.y == a;
+            const uint32_t x = own ? j : rec[k].r[md.y == lo ? 0 : 1];
+            const uint32_t m = own ? sg.x + half : md.x;
+            is_l = x < m;
+            is_m = x == m;
+            if (j == sg.x || j + 1u == sg.y) {
+                mark = k;
+                mark_abs = abs_at(V, node[k] - V.first, sg.x);
+                if (j != sg.x)  // (after the last position: all the node's, less its own side)
+                    mark_abs = abs_add(mark_abs, (half - (is_l ? 1u : 0u)) | (is_m ? 0u : kAbsM));
             }
-            v = (j == sgk[k].x ? kSegH : 0u) | (sd == 0 ? 1u : 0u) | (sd == 1 ? kSegM : 0u);
         }
-        val[k] = v;
-        // wave-level inclusive segmented scan over the row
-        uint32_t x = v;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            uint32_t y = __shfl_up(x, d, 64);
-            if (lane >= (uint32_t)d) x = seg_op(y, x);
-        }
-        incl[k] = x;
-        if (lane == 63) s_wagg[k * (kPThreads / 64) + wave] = x;
+        const uint64_t bl = __ballot(is_l), bm = __ballot(is_m);
+        cnt[k] = __builtin_amdgcn_mbcnt_hi((uint32_t)(bl >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bl, 0u)) +
+                 kCntM * __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u)) +
+                 (is_l ? kIsL : 0u) + (is_m ? kIsM : 0u);
+        if (lane == 0) s_row[k * (kPThreads / 64) + wave] = (uint32_t)__popcll(bl) + kCntM * (uint32_t)__popcll(bm);
     }
     __syncthreads();
-    // exclusive prefixes of the 64 wave rows, in tile order (row-major)
+    // exclusive counts of the wave rows, in tile order (row-major)
+    uint32_t agg = 0;
     if (wave == 0) {
-        constexpr uint32_t nw = kPItems * (kPThreads / 64);
-        uint32_t x = lane < nw ? s_wagg[lane] : 0u;
+        const uint32_t a = s_row[2 * lane], b = s_row[2 * lane + 1];
+        uint32_t x = a + b;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
-            uint32_t y = __shfl_up(x, d, 64);
-            if (lane >= (uint32_t)d) x = seg_op(y, x);
+            const uint32_t y = __shfl_up(x, d, 64);
+            if (lane >= (uint32_t)d) x += y;
         }
-        // x = inclusive over rows 0..lane; exclusive = inclusive of lane - 1
-        uint32_t ex = __shfl_up(x, 1, 64);
-        if (lane < nw) s_wpre[lane] = lane == 0 ? 0u : ex;
-        const uint32_t agg = __shfl(x, nw - 1, 64);
-        // decoupled look-back for the tile prefix
-        uint32_t prefix = 0;
-        if (tile == 0) {
-            if (lane == 0)
-                __hip_atomic_store(&state[0], seg_state(epoch, kStIncl, agg), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        } else {
-            if (lane == 0)
-                __hip_atomic_store(&state[tile], seg_state(epoch, kStAgg, agg), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            int64_t jt = (int64_t)tile - 1;
-            bool have = false;  // prefix holds the combination of the tiles after the current window
-            for (;;) {
-                const int64_t idx = jt - (int64_t)lane;
-                uint64_t w;
-                uint32_t status;
-                uint64_t stop_mask, inval_mask, upto;
-                for (;;) {
-                    if (idx >= 0) {
-                        w = __hip_atomic_load(&state[idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        status = ((uint32_t)(w >> 34) == epoch) ? (uint32_t)((w >> 32) & 3) : 0u;
-                    } else {
-                        w = 0;
-                        status = (uint32_t)kStIncl;
-                    }
-                    // a tile whose value holds a segment start ends the walk too
-                    stop_mask = __ballot(status == kStIncl || (status == kStAgg && ((uint32_t)w & kSegH)));
-                    inval_mask = __ballot(status == 0);
-                    const int first = stop_mask ? __builtin_ctzll(stop_mask) : 63;
-                    upto = (first == 63) ? ~0ull : ((2ull << first) - 1);
-                    if ((inval_mask & upto) == 0) break;
-                    __builtin_amdgcn_s_sleep(1);
-                }
-                // combine the window's values from the farthest used lane down to lane 0
-                const int last = (stop_mask & upto) ? __builtin_ctzll(stop_mask) : 63;
-                uint32_t win = 0;
-                for (int l = last; l >= 0; --l) {
-                    const uint32_t wl = (uint32_t)__shfl((uint32_t)w, l, 64);
-                    win = (l == last) ? wl : seg_op(win, wl);
-                }
-                prefix = have ? seg_op(win, prefix) : win;
-                have = true;
-                if (stop_mask & upto) break;
-                jt -= 64;
-            }
-            if (lane == 0)
-                __hip_atomic_store(&state[tile], seg_state(epoch, kStIncl, seg_op(prefix, agg)), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (lane == 0) s_prefix = prefix;
+        s_row[2 * lane] = x - a - b;
+        s_row[2 * lane + 1] = x - b;
+        agg = abs_of(__builtin_amdgcn_readlane(x, 63));
     }
     __syncthreads();
-    const uint32_t tprefix = s_prefix;
 #pragma unroll
     for (int k = 0; k < kPItems; ++k) {
-        const uint32_t g = tile * kPTile + (uint32_t)k * kPThreads + t;
-        if (g >= total) continue;
-        const uint32_t a = g >= 2 * n ? 2u : (g >= n ? 1u : 0u), j = g - a * n;
+        cnt[k] += s_row[k * (kPThreads / 64) + wave];
+        if (mark == k) {  // (every mark of the tile gives the same counts)
+            s_at = abs_sub(mark_abs, abs_of(cnt[k] & kCnt));
+            s_known = 1u;
+        }
+    }
+    __syncthreads();
+    if (kLook) {
+        if (wave == 0) {
+            uint32_t at = s_at;
+            const uint32_t epoch = s_epoch;
+            if (!s_known) {
+                // inside one node: the counts of the tiles before, back to one that knows its own
+                if (lane == 0)
+                    __hip_atomic_store(&state[a * n_tiles + tile], seg_state(epoch, kStAgg, agg), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                at = 0;
+                for (int64_t jt = (int64_t)tile - 1;; jt -= 64) {
+                    const int64_t idx = jt - (int64_t)lane;
+                    uint64_t w, stop_mask, upto;
+                    for (;;) {
+                        uint32_t status = (uint32_t)kStIncl;
+                        w = 0;
+                        if (idx >= 0) {
+                            w = __hip_atomic_load(&state[a * n_tiles + (uint32_t)idx], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            status = ((uint32_t)(w >> 34) == epoch) ? (uint32_t)((w >> 32) & 3) : 0u;
+                        }
+                        stop_mask = __ballot(status == kStIncl);
+                        const uint64_t inval_mask = __ballot(status == 0);
+                        const int first = stop_mask ? __builtin_ctzll(stop_mask) : 63;
+                        upto = (first == 63) ? ~0ull : ((2ull << first) - 1);
+                        if ((inval_mask & upto) == 0) break;
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    uint32_t win = ((upto >> lane) & 1ull) ? (uint32_t)w : 0u;
+#pragma unroll
+                    for (int d = 32; d >= 1; d >>= 1) win = abs_add(win, (uint32_t)__shfl_xor(win, d, 64));
+                    at = abs_add(at, win);
+                    if (stop_mask & upto) break;
+                }
+            }
+            if (lane == 0) {
+                __hip_atomic_store(&state[a * n_tiles + tile], seg_state(epoch, kStIncl, abs_add(at, agg)), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+                s_at = at;
+            }
+        }
+        __syncthreads();
+    }
+    const uint32_t at = s_at;
+#pragma unroll
+    for (int k = 0; k < kPItems; ++k) {
+        const uint32_t j = j0 + (uint32_t)k * kPThreads;
+        if (j >= n) continue;
         const uint32_t s = node[k];
         uint32_t dst = j, nn = kFinal;
         if (s != kFinal) {
-            const uint32_t before = seg_op(seg_op(tprefix, s_wpre[k * (kPThreads / 64) + wave]), incl[k]);
-            const uint2 sg = sgk[k];
-            const uint32_t from = sg.x, mid = sg.x + (sg.y - sg.x) / 2;
-            const uint32_t own = val[k];
-            const uint32_t lb = (before & kSegL) - (own & kSegL), mb = ((before & kSegM) ? 1u : 0u) -
-                                                                       ((own & kSegM) ? 1u : 0u);
-            if (own & 1u)
-                dst = from + lb;
-            else if (own & kSegM)
+            const uint2 sg = seg[s];
+            const uint32_t mid = sg.x + (sg.y - sg.x) / 2;
+            const uint32_t b = abs_sub(abs_add(at, abs_of(cnt[k] & kCnt)), abs_at(V, s - V.first, sg.x));
+            const uint32_t lb = b & kAbsL, mb = b >> 30;
+            if (cnt[k] & kIsL)
+                dst = sg.x + lb;
+            else if (cnt[k] & kIsM)
                 dst = mid;
             else
-                dst = mid + 1 + ((j - from) - lb - mb);
+                dst = mid + 1 + ((j - sg.x) - lb - mb);
             if (!(sg.y - sg.x <= 1 || j == mid)) nn = j < mid ? 2 * s + 1 : 2 * s + 2;
         }
-        if (dst < n) (a == 0 ? B0 : a == 1 ? B1 : B2)[dst] = rec[k];  // always true for a consistent tree
+        if (dst < n) B[dst] = rec[k];  // always true for a consistent tree
         if (a == 0) node_out[j] = nn;
     }
 }
@@ -677,7 +702,8 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
     size_t rs = pm::radix_sort_scratch_bytes(n, 3);
     const size_t rb = (size_t)n * sizeof(Rk), n3 = 3 * (size_t)n;
     size_t need = pm::carve_size({rb, rb, rb, rb, rb, rb, (size_t)n * 4, (size_t)n * 4, (size_t)cap * 8, (size_t)cap,
-                                  (size_t)cap * 8, n3 * 4, n3 * 4, n3 * 4, (size_t)n * 16, rs, (size_t)n * 48});
+                                  (size_t)cap * 8, n3 * 4, n3 * 4, n3 * 4, (size_t)n * 16, rs, (size_t)n * 48,
+                                  3 * kTicket * 4});
     void* work = nullptr;
     pm_status st = pm::scratch_reserve(ctx, need, &work);
     if (st != PM_OK) return bail(st);
@@ -697,6 +723,7 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
     uint32_t* rank4 = cv.take<uint32_t>(4 * (size_t)n);  // each photon's three ranks
     void* rw = cv.take<char>(rs);
     float4* prec = cv.take<float4>((size_t)n * 3);
+    uint32_t* tickets = cv.take<uint32_t>(3 * kTicket);
 
     const uint32_t nb = pm::div_up(n, 256);
     hipStream_t s = ctx->stream;
@@ -734,7 +761,8 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
     if (L - Lg > 11) return bail(pm::fail(ctx, PM_ERR_INVALID, "pm_kdtree_build: internal level split"));
     // the root's plane (and, above the LDS levels, its median)
     hipLaunchKernelGGL(k_level_nodes, dim3(1), dim3(256), 0, s, orders(), 0u, 1u, cap, n, Lg > 0, seg, plane,
-                       T->node_idx, T->node_plane, med, nullptr);
+                       T->node_idx, T->node_plane, med, nullptr, tickets);
+    uint32_t smin = n;  // the smallest node of the level (those above the LDS levels are not empty)
     for (uint32_t lvl = 0; lvl < L; ++lvl) {
         uint32_t first = (1u << lvl) - 1, count = 1u << lvl;
         if (lvl == Lg) {
@@ -745,18 +773,26 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
             break;
         }
         if (lvl + 1 == L) break;  // every segment of the last level has size <= 1
-        const uint32_t tiles = pm::div_up(3ull * n, kPTile);
-        uint64_t* lstate;
-        uint32_t* lcounter;
-        if ((st = pm::lookback_begin(ctx, tiles, &lstate, &lcounter)) != PM_OK) return bail(st);
-        hipLaunchKernelGGL(k_level_partition, dim3(tiles), dim3(kPThreads), 0, s, A[0], A[1], A[2], B[0], B[1], B[2],
-                           n, node_of, node_of2, seg, plane, med, lstate, lcounter, tiles);
+        const uint32_t tiles = 3u * pm::div_up(n, kPTile);
+        uint64_t* lstate = nullptr;
+        uint32_t* lcounter = nullptr;
+        const Level V{first, smin};
+        // (a tile strictly inside a node knows its place from the tiles before)
+        if (smin + 1u >= kPTile + 2u) {
+            if ((st = pm::lookback_begin(ctx, tiles, &lstate, &lcounter)) != PM_OK) return bail(st);
+            hipLaunchKernelGGL(k_level_partition<true>, dim3(tiles), dim3(kPThreads), 0, s, A[0], A[1], A[2], B[0],
+                               B[1], B[2], n, node_of, node_of2, seg, med, V, lstate, lcounter, tickets);
+        } else {
+            hipLaunchKernelGGL(k_level_partition<false>, dim3(tiles), dim3(kPThreads), 0, s, A[0], A[1], A[2], B[0],
+                               B[1], B[2], n, node_of, node_of2, seg, med, V, lstate, lcounter, tickets);
+        }
+        smin = (smin - 1u) / 2u;
         for (int a = 0; a < 3; ++a) std::swap(A[a], B[a]);
         std::swap(node_of, node_of2);
         // the children's planes, and their medians above the LDS levels
         uint32_t cf = (1u << (lvl + 1)) - 1, cc = 1u << (lvl + 1);
         hipLaunchKernelGGL(k_level_nodes, dim3(pm::div_up(cc, 256)), dim3(256), 0, s, orders(), cf, cc, cap, 0u,
-                           lvl + 1 < Lg, seg, plane, T->node_idx, T->node_plane, med, lcounter);
+                           lvl + 1 < Lg, seg, plane, T->node_idx, T->node_plane, med, lcounter, tickets);
     }
     hipLaunchKernelGGL(k_tree_photons, dim3(pm::div_up(cap, 256)), dim3(256), 0, s, prec, T->node_idx,
                        T->node_plane, cap, T->photons, T->nodes);
