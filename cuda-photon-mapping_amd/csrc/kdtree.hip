@@ -26,12 +26,6 @@
 
 namespace {
 
-// a photon in LDS (the subtrees finished by one workgroup)
-struct Rec {
-    float c[3];
-    uint32_t id;
-};
-
 // A photon's record in the order of axis a: its ranks on the two other axes,
 // other_axis(a, 0) < other_axis(a, 1).
 struct Rk {
@@ -171,14 +165,6 @@ __global__ __launch_bounds__(256) void k_level_nodes(Orders O, uint32_t first, u
         if (l < cap) seg[l] = make_uint2(s.x, mid);
         if (r < cap) seg[r] = make_uint2(mid + 1, s.y);
     }
-}
-
-// side of record e relative to node's median on plane p: 0 left, 1 median, 2 right
-__device__ __forceinline__ int side_of(const Rec& e, int p, uint2 m) {
-    if (e.id == m.y) return 1;
-    const float a = p == 0 ? e.c[0] : (p == 1 ? e.c[1] : e.c[2]), b = __uint_as_float(m.x);
-    bool less = a < b || (a == b && e.id < m.y);
-    return less ? 0 : 2;
 }
 
 // ---- one level's stable partition in one pass --------------------------------
@@ -407,81 +393,44 @@ __global__ __launch_bounds__(kPThreads) __attribute__((amdgpu_waves_per_eu(8))) 
 // Once every segment holds at most kLocal records, one workgroup finishes a
 // whole subtree in LDS: the same median / stable-partition / child-plane
 // steps as the level loop above, on the subtree's slice of the three axis
-// orders, with workgroup scans instead of device scans. The subtree's records
-// are loaded once (in axis-0 order); the three orders are permutations of
-// 16-bit local indices, so a partition moves 2 bytes per position and a
-// workgroup needs 46 KB of LDS (three workgroups per CU).
+// orders. The orders are permutations of 16-bit local indices (positions in
+// the axis-0 order); a thread keeps its four positions' nodes and segments in
+// registers (they depend on the positions alone). A depth takes four
+// barriers: each record's side is marked from its node's split axis, all three
+// orders count their left records and medians by ballots from the known node
+// starts (as above), move, and each new segment's first position works out its
+// plane. 31 KB of LDS, five workgroups a CU. The time goes into the barriers and
+// the dependent LDS reads between them: 2M photons 338 us with one axis after
+// the other (fifteen barriers, a scan of 0/1 flags and 46 KB of LDS), now KNEW.
 constexpr int kLocal = 1024;
 constexpr int kLocalThreads = 256;
+constexpr int kLocalPer = kLocal / kLocalThreads;
+constexpr int kLocalRows = kLocal / 64;  // wave rows of an axis
+static_assert(kLocalRows == 16, "an axis's wave rows are one DPP row");
 
 struct LocalLds {
-    Rec rec[kLocal];          // the subtree's records in axis-0 order
-    // per axis: local record index at each position, in buffers ordb[oi[a]];
-    // the fourth buffer receives the next partition and the roles rotate
-    uint16_t ordb[4][kLocal];
-    uint16_t pref[kLocal];
-    uint16_t node[kLocal];    // local node (at the current depth) of each position, 0xFFFF = final
-    ushort2 seg[2][kLocal];   // node segments, current and next depth
-    int8_t plane[2][kLocal];
-    uint2 med[kLocal / 2];
-    uint16_t mpos[kLocal / 2][3];
-    uint8_t flag[kLocal];
-    uint32_t wsum[kLocalThreads / 64];
+    float c[kLocal][3];  // by local index
+    uint32_t id[kLocal];
+    union {
+        uint16_t ord[2][3][kLocal];  // per axis: the local index at each position, this depth's and the next's
+        struct {
+            uint16_t first[3][kLocal];
+            uint32_t r0[kLocal];  // the axis-0 ranks, ascending (while the orders are set up)
+        };
+    };
+    uint8_t side[kLocal];   // by local index: 1 left, 2 median, 0 right
+    uint8_t plane[kLocal];  // by a segment's first position
+    uint32_t row[3 * kLocalRows];
 };
-
-// pos0[id] = position of photon id in the axis-0 order (for the subtrees'
-// index maps).
-// For the LDS levels: ids0[j] = the photon at position j of the axis-0
-// order, and posr0[r] = the position in that order of the photon of axis-0
-// rank r (the order-1 and order-2 records carry that rank).
-__global__ __launch_bounds__(256) void k_pos0(Orders O, uint32_t* __restrict__ ids0, uint32_t* __restrict__ posr0) {
-    uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= O.n) return;
-    const uint32_t id = id_at(O, 0, j);
-    ids0[j] = id;
-    posr0[O.rank4[4 * (size_t)id]] = j;
-}
-
-// Exclusive scan of L.flag[0, m) (0/1) into L.pref.
-__device__ __forceinline__ void local_scan(LocalLds& L, uint32_t m) {
-    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    constexpr uint32_t per = kLocal / kLocalThreads;  // 4 positions per thread
-    uint32_t v[per], sum = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < per; ++i) {
-        uint32_t j = t * per + i;
-        v[i] = j < m ? L.flag[j] : 0u;
-        sum += v[i];
-    }
-    uint32_t inc = sum;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint32_t y = __shfl_up(inc, d, 64);
-        if (lane >= (uint32_t)d) inc += y;
-    }
-    if (lane == 63) L.wsum[wave] = inc;
-    __syncthreads();
-    uint32_t before = 0;
-    for (uint32_t w = 0; w < wave; ++w) before += L.wsum[w];
-    uint32_t run = before + inc - sum;
-#pragma unroll
-    for (uint32_t i = 0; i < per; ++i) {
-        uint32_t j = t * per + i;
-        if (j < m) L.pref[j] = (uint16_t)run;
-        run += v[i];
-    }
-    __syncthreads();
-}
+static_assert(sizeof(uint16_t) * 3 * kLocal >= sizeof(uint32_t) * kLocal, "the ranks fit the next depth's orders");
 
 // find_largest_plane over local segment [f, t) (PhotonMap.cuh:161-178)
-__device__ __forceinline__ int8_t local_plane(const LocalLds& L, const int (&oi)[3], uint32_t f, uint32_t t) {
-    const uint16_t* o0 = L.ordb[oi[0]];
-    const uint16_t* o1 = L.ordb[oi[1]];
-    const uint16_t* o2 = L.ordb[oi[2]];
-    float d0 = fabsf(L.rec[o0[t - 1]].c[0] - L.rec[o0[f]].c[0]);
-    float d1 = fabsf(L.rec[o1[t - 1]].c[1] - L.rec[o1[f]].c[1]);
-    float d2 = fabsf(L.rec[o2[t - 1]].c[2] - L.rec[o2[f]].c[2]);
-    int8_t p = 0;
+__device__ __forceinline__ uint8_t local_plane(const LocalLds& L, const uint16_t (&o)[3][kLocal], uint32_t f,
+                                               uint32_t t) {
+    const float d0 = fabsf(L.c[o[0][t - 1]][0] - L.c[o[0][f]][0]);
+    const float d1 = fabsf(L.c[o[1][t - 1]][1] - L.c[o[1][f]][1]);
+    const float d2 = fabsf(L.c[o[2][t - 1]][2] - L.c[o[2][f]][2]);
+    uint8_t p = 0;
     float mx = d0;
     if (d1 > mx) {
         mx = d1;
@@ -491,114 +440,155 @@ __device__ __forceinline__ int8_t local_plane(const LocalLds& L, const int (&oi)
     return p;
 }
 
+// Inclusive sum over each row of 16 lanes.
+template <int kCtrl>
+__device__ __forceinline__ uint32_t dpp_row_add(uint32_t v) {
+    return v + (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtrl, 0xf, 0xf, false);
+}
+__device__ __forceinline__ uint32_t row_incl_scan(uint32_t v) {
+    v = dpp_row_add<0x111>(v);  // row_shr:1
+    v = dpp_row_add<0x112>(v);
+    v = dpp_row_add<0x114>(v);
+    return dpp_row_add<0x118>(v);
+}
+
 __global__ __launch_bounds__(kLocalThreads) void k_local_subtrees(Orders O, const float4* __restrict__ prec,
-                                                                 const uint32_t* __restrict__ ids0,
-                                                                 const uint32_t* __restrict__ posr0, uint32_t first,
-                                                                 uint32_t depth_left, const uint2* __restrict__ gseg,
+                                                                 uint32_t first, const uint2* __restrict__ gseg,
                                                                  const int8_t* __restrict__ gplane,
                                                                  uint32_t* __restrict__ node_idx,
                                                                  int8_t* __restrict__ node_plane) {
     __shared__ LocalLds L;
-    const uint32_t root = first + blockIdx.x, t = threadIdx.x;
+    const uint32_t root = first + blockIdx.x, t = threadIdx.x, lane = t & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const uint2 rs = gseg[root];
     if (rs.y <= rs.x || rs.y - rs.x > (uint32_t)kLocal) return;  // empty subtree; larger ones never reach here
     const uint32_t m = rs.y - rs.x;
     // the segment holds the same photons in each order: the photons of the
-    // axis-0 order with their coordinates, and axes 1 and 2 mapped to
-    // axis-0 positions by their records' axis-0 ranks
-    for (uint32_t j = t; j < m; j += kLocalThreads) {
-        const uint32_t id = ids0[rs.x + j];
-        const float4 c = prec[3 * (size_t)id];
-        L.rec[j] = Rec{{c.x, c.y, c.z}, id};
-        L.ordb[0][j] = (uint16_t)j;
-        L.ordb[1][j] = (uint16_t)(posr0[O.A[1][rs.x + j].r[0]] - rs.x);
-        L.ordb[2][j] = (uint16_t)(posr0[O.A[2][rs.x + j].r[0]] - rs.x);
-        L.node[j] = 0;
+    // axis-0 order with their coordinates and axis-0 ranks
+    uint32_t id[kLocalPer], a1[kLocalPer], a2[kLocalPer];
+#pragma unroll
+    for (int k = 0; k < kLocalPer; ++k) {
+        const uint32_t j = (uint32_t)k * kLocalThreads + t;
+        if (j < m) {
+            id[k] = id_at(O, 0, rs.x + j);
+            a1[k] = O.A[1][rs.x + j].r[0];
+            a2[k] = O.A[2][rs.x + j].r[0];
+        }
     }
-    if (t == 0) {
-        L.seg[0][0] = make_ushort2(0, (uint16_t)m);
-        L.plane[0][0] = gplane[root];
+#pragma unroll
+    for (int k = 0; k < kLocalPer; ++k) {
+        const uint32_t j = (uint32_t)k * kLocalThreads + t;
+        L.r0[j] = 0xFFFFFFFFu;
+        if (j < m) {
+            const float4 c = prec[3 * (size_t)id[k]];
+            L.r0[j] = O.rank4[4 * (size_t)id[k]];
+            L.id[j] = id[k];
+            L.c[j][0] = c.x;
+            L.c[j][1] = c.y;
+            L.c[j][2] = c.z;
+        }
     }
     __syncthreads();
-    int cur = 0;
-    int oi[3] = {0, 1, 2}, spare = 3;  // (workgroup-uniform)
-    for (uint32_t d = 0; d < depth_left; ++d) {
-        const uint32_t nd = 1u << d;
-        const uint32_t gfirst = (root + 1) * nd - 1;  // global index of local node 0 at this depth
-        const bool last = d + 1 == depth_left;
-        // medians (k_level_nodes) and the children's segments
-        for (uint32_t i = t; i < nd; i += kLocalThreads) {
-            const ushort2 s = L.seg[cur][i];
-            ushort2 cl = make_ushort2(0, 0), cr = make_ushort2(0, 0);
-            if (s.y > s.x) {
-                const int8_t p = L.plane[cur][i];
-                const uint32_t mid = s.x + (s.y - s.x) / 2;
-                const Rec r = L.rec[L.ordb[p == 0 ? oi[0] : p == 1 ? oi[1] : oi[2]][mid]];
-                node_idx[gfirst + i] = r.id;
-                node_plane[gfirst + i] = p;
-                if (!last) L.med[i] = make_uint2(__float_as_uint(r.c[p]), r.id);
-                if (s.y - s.x > 1) {
-                    cl = make_ushort2(s.x, (uint16_t)mid);
-                    cr = make_ushort2((uint16_t)(mid + 1), s.y);
-                }
+    // axes 1 and 2 mapped to axis-0 positions by their records' axis-0 ranks
+#pragma unroll
+    for (int k = 0; k < kLocalPer; ++k) {
+        const uint32_t j = (uint32_t)k * kLocalThreads + t;
+        if (j < m) {
+            uint32_t x = 0, y = 0;
+#pragma unroll
+            for (uint32_t d = kLocal / 2; d > 0; d >>= 1) {
+                if (L.r0[x + d] <= a1[k]) x += d;
+                if (L.r0[y + d] <= a2[k]) y += d;
             }
-            if (!last) {
-                L.seg[cur ^ 1][2 * i] = cl;
-                L.seg[cur ^ 1][2 * i + 1] = cr;
+            L.first[0][j] = (uint16_t)j;
+            L.first[1][j] = (uint16_t)x;
+            L.first[2][j] = (uint16_t)y;
+        }
+    }
+    if (t == 0) L.plane[0] = (uint8_t)gplane[root];
+    __syncthreads();
+
+    // a position's node at this depth and its segment (from | to << 16); to = 0: finished
+    uint32_t node[kLocalPer], sg[kLocalPer];
+#pragma unroll
+    for (int k = 0; k < kLocalPer; ++k) {
+        node[k] = 0;
+        sg[k] = (uint32_t)k * kLocalThreads + t < m ? m << 16 : 0u;
+    }
+    uint32_t smin = m, smax = m;  // the node sizes of the depth
+    for (uint32_t d = 0;; ++d) {
+        const uint16_t(&ord)[3][kLocal] = L.ord[d & 1u];
+        uint16_t(&out)[3][kLocal] = L.ord[(d & 1u) ^ 1u];
+        const uint32_t gfirst = ((root + 1u) << d) - 1u;  // global index of local node 0 at this depth
+#pragma unroll
+        for (int k = 0; k < kLocalPer; ++k) {
+            const uint32_t j = (uint32_t)k * kLocalThreads + t, from = sg[k] & 0xffffu, to = sg[k] >> 16;
+            if (to == 0) continue;
+            const uint32_t mid = (from + to) >> 1;
+            const uint8_t p = L.plane[from];
+            const uint32_t x = ord[p][j];
+            L.side[x] = j < mid ? 1 : j == mid ? 2 : 0;
+            if (j == mid) {
+                node_idx[gfirst + node[k]] = L.id[x];
+                node_plane[gfirst + node[k]] = (int8_t)p;
             }
         }
+        if (smax <= 1) break;
         __syncthreads();
-        if (last) break;
-        // stable partition of each axis order around its node's median
+        // per position and axis: local index, side, counts in its wave row
+        uint32_t e[3][kLocalPer];
+#pragma unroll
         for (int a = 0; a < 3; ++a) {
-            for (uint32_t j = t; j < m; j += kLocalThreads) {
-                const uint32_t i = L.node[j];
-                uint8_t f = 0;
-                if (i != 0xFFFFu) {
-                    const int sd = side_of(L.rec[L.ordb[oi[a]][j]], L.plane[cur][i], L.med[i]);
-                    f = sd == 0;
-                    if (sd == 1) L.mpos[i][a] = (uint16_t)j;
-                }
-                L.flag[j] = f;
+#pragma unroll
+            for (int k = 0; k < kLocalPer; ++k) {
+                const bool on = sg[k] != 0;
+                const uint32_t x = on ? ord[a][(uint32_t)k * kLocalThreads + t] : 0u;
+                const uint32_t s = on ? L.side[x] : 0u;
+                const uint64_t bl = __ballot(s == 1), bm = __ballot(s == 2);
+                e[a][k] = x | s << 10 |
+                          __builtin_amdgcn_mbcnt_hi((uint32_t)(bl >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bl, 0u)) << 12 |
+                          __builtin_amdgcn_mbcnt_hi((uint32_t)(bm >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bm, 0u)) << 20;
+                if (lane == 0)
+                    L.row[a * kLocalRows + k * (kLocalThreads / 64) + wave] =
+                        (uint32_t)__popcll(bl) | (uint32_t)__popcll(bm) << 16;
             }
-            __syncthreads();
-            local_scan(L, m);
-            for (uint32_t j = t; j < m; j += kLocalThreads) {
-                const uint32_t i = L.node[j];
-                uint32_t dst = j;
-                if (i != 0xFFFFu) {
-                    const ushort2 sg = L.seg[cur][i];
-                    const uint32_t from = sg.x, mid = sg.x + (sg.y - sg.x) / 2;
-                    const uint32_t before_l = (uint32_t)L.pref[j] - L.pref[from];
-                    if (L.flag[j]) {
-                        dst = from + before_l;
-                    } else {
-                        const uint32_t mp = L.mpos[i][a];
-                        dst = mp == j ? mid : mid + 1 + ((j - from) - before_l - (mp < j ? 1u : 0u));
-                    }
-                }
-                L.ordb[spare][dst] = L.ordb[oi[a]][j];
-            }
-            __syncthreads();
-            const int was = oi[a];
-            oi[a] = spare;
-            spare = was;
-        }
-        // node of every position at the next depth
-        for (uint32_t j = t; j < m; j += kLocalThreads) {
-            const uint32_t i = L.node[j];
-            if (i == 0xFFFFu) continue;
-            const ushort2 sg = L.seg[cur][i];
-            const uint32_t mid = sg.x + (sg.y - sg.x) / 2;
-            L.node[j] = (sg.y - sg.x <= 1 || j == mid) ? (uint16_t)0xFFFFu : (uint16_t)(j < mid ? 2 * i : 2 * i + 1);
-        }
-        // child planes (as k_level_nodes)
-        for (uint32_t c = t; c < 2 * nd; c += kLocalThreads) {
-            const ushort2 s = L.seg[cur ^ 1][c];
-            L.plane[cur ^ 1][c] = s.y > s.x ? local_plane(L, oi, s.x, s.y) : (int8_t)0;
         }
         __syncthreads();
-        cur ^= 1;
+        const uint32_t rows = lane < 3u * kLocalRows ? L.row[lane] : 0u, before = row_incl_scan(rows) - rows;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+#pragma unroll
+            for (int k = 0; k < kLocalPer; ++k) {
+                const uint32_t b = __builtin_amdgcn_readlane(before, a * kLocalRows + k * (kLocalThreads / 64) + wave);
+                if (sg[k] == 0) continue;
+                const uint32_t j = (uint32_t)k * kLocalThreads + t, from = sg[k] & 0xffffu, to = sg[k] >> 16;
+                const uint32_t mid = (from + to) >> 1, i = node[k];
+                // the left records of the nodes before (abs_at), and their medians
+                const uint32_t bl = i * (smin >> 1) + ((smin & 1u) ? from - i * (smin + 1u) : 0u);
+                const uint32_t lb = (b & 0xffffu) + (e[a][k] >> 12 & 0x7fu) - bl;
+                const uint32_t mb = (b >> 16) + (e[a][k] >> 20) - i, s = e[a][k] >> 10 & 3u;
+                const uint32_t dst = s == 1 ? from + lb : s == 2 ? mid : mid + 1 + ((j - from) - lb - mb);
+                out[a][dst & (kLocal - 1)] = (uint16_t)(e[a][k] & 0x3ffu);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < kLocalPer; ++k) {
+            const uint32_t j = (uint32_t)k * kLocalThreads + t, from = sg[k] & 0xffffu, to = sg[k] >> 16;
+            const uint32_t mid = (from + to) >> 1;
+            if (to == 0) continue;
+            node[k] = 2 * node[k] + (j > mid ? 1u : 0u);
+            sg[k] = j == mid ? 0u : j < mid ? (from | mid << 16) : ((mid + 1u) | to << 16);
+        }
+        smin = (smin - 1u) / 2u;
+        smax /= 2u;
+        __syncthreads();
+        // the new segments' planes (as k_level_nodes), by their first positions
+#pragma unroll
+        for (int k = 0; k < kLocalPer; ++k) {
+            const uint32_t j = (uint32_t)k * kLocalThreads + t, from = sg[k] & 0xffffu, to = sg[k] >> 16;
+            if (to > 0 && j == from) L.plane[from] = local_plane(L, out, from, to);
+        }
+        __syncthreads();
     }
 }
 
@@ -718,7 +708,7 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
     int8_t* plane = cv.take<int8_t>(cap);
     uint2* med = cv.take<uint2>(cap);
     uint32_t* keys = cv.take<uint32_t>(n3);   // sort keys
-    uint32_t* skeys = cv.take<uint32_t>(n3);  // sorted keys, then ids0 and posr0 (the LDS levels)
+    uint32_t* skeys = cv.take<uint32_t>(n3);  // sorted keys
     uint32_t* order = cv.take<uint32_t>(n3);  // each axis's photons in rank order
     uint32_t* rank4 = cv.take<uint32_t>(4 * (size_t)n);  // each photon's three ranks
     void* rw = cv.take<char>(rs);
@@ -766,10 +756,8 @@ extern "C" pm_status pm_kdtree_build(pm_ctx* ctx, const float* d_photons9, uint3
     for (uint32_t lvl = 0; lvl < L; ++lvl) {
         uint32_t first = (1u << lvl) - 1, count = 1u << lvl;
         if (lvl == Lg) {
-            uint32_t *ids0 = skeys, *posr0 = skeys + n;
-            hipLaunchKernelGGL(k_pos0, dim3(nb), dim3(256), 0, s, orders(), ids0, posr0);
-            hipLaunchKernelGGL(k_local_subtrees, dim3(count), dim3(kLocalThreads), 0, s, orders(), prec, ids0, posr0,
-                               first, L - lvl, seg, plane, T->node_idx, T->node_plane);
+            hipLaunchKernelGGL(k_local_subtrees, dim3(count), dim3(kLocalThreads), 0, s, orders(), prec, first, seg,
+                               plane, T->node_idx, T->node_plane);
             break;
         }
         if (lvl + 1 == L) break;  // every segment of the last level has size <= 1
