@@ -1,4 +1,4 @@
-// Stable LSD radix sort of (u32 key, u32 value) pairs, 8-bit digits.
+// Stable LSD radix sort of (u32 key, u32 value) pairs, digits of up to 9 bits.
 //
 // Each pass is count -> scan -> stable scatter: a per-tile digit histogram,
 // the wave64 look-back scan over the digit-major histogram table, and a
@@ -15,12 +15,20 @@
 
 namespace {
 
-constexpr int kThreads = 256;
+// A pass over a million keys is 245 tiles, one a CU, and waits on its own
+// loads, LDS updates and barriers: eight waves of 8 keys a lane take 11.4 us
+// where four of 16 took 17 (2M keys in three segments 32.3 and 37.4, 16M 93
+// and 105; tiles of 2048 or 6144: no faster, or slower from 16M on). Digits of
+// up to 9 bits give a grid of 64k to 256k cells two passes instead of three
+// (29 us of a million queries' 93): a pass of 9 bits takes 14.2 us.
+constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
-constexpr int kItems = 16;                 // keys per lane
-constexpr int kWaveKeys = 64 * kItems;     // 1024 keys per wave
-constexpr int kTile = kThreads * kItems;   // 4096 keys per tile
-constexpr int kBins = 256;
+constexpr int kItems = 8;                 // keys per lane
+constexpr int kWaveKeys = 64 * kItems;    // 512 keys per wave
+constexpr int kTile = kThreads * kItems;  // 4096 keys per tile
+constexpr int kMaxBits = 9;
+constexpr int kMaxBins = 1 << kMaxBits;  // thread t owns digit t
+static_assert(kMaxBins == kThreads, "a digit a thread");
 
 // n: the segment length; n_dev (nullable, one segment only): the element
 // count on the device, at most n (the launch covers n; tiles past the device
@@ -28,22 +36,23 @@ constexpr int kBins = 256;
 __global__ __launch_bounds__(kThreads) void k_rs_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
                                                      uint32_t mask, uint32_t* __restrict__ hist, uint32_t tiles,
                                                      const uint32_t* __restrict__ n_dev) {
-    __shared__ uint32_t s_hist[kBins];
+    __shared__ uint32_t s_hist[kMaxBins];
     const uint32_t t = threadIdx.x, seg = blockIdx.x / tiles, tile = blockIdx.x % tiles;
     const uint32_t* sk = keys + (size_t)seg * n;
     if (n_dev) n = min(n, *n_dev);
     s_hist[t] = 0;
     __syncthreads();
     const size_t base = (size_t)tile * kTile;
-#pragma unroll 4
+#pragma unroll
     for (int i = 0; i < kItems; ++i) {
         size_t idx = base + (size_t)i * kThreads + t;
         if (idx < n) atomicAdd(&s_hist[(sk[idx] >> shift) & mask], 1u);
     }
     __syncthreads();
-    hist[((size_t)seg * kBins + t) * tiles + tile] = s_hist[t];
+    if (t <= mask) hist[((size_t)seg * (mask + 1u) + t) * tiles + tile] = s_hist[t];
 }
 
+template <int kBits>
 __global__ __launch_bounds__(kThreads) void k_rs_scatter(const uint32_t* __restrict__ keys_in,
                                                         const uint32_t* __restrict__ vals_in,
                                                         uint32_t* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
@@ -56,14 +65,14 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const uint32_t* __restr
     if ((size_t)tile * kTile >= n) return;  // (block-uniform, before any barrier)
     __shared__ uint32_t s_keys[kTile];
     __shared__ uint32_t s_vals[kTile];
-    __shared__ uint32_t s_whist[kWaves][kBins];
-    __shared__ uint32_t s_dstart[kBins];
-    __shared__ uint32_t s_goff[kBins];
+    __shared__ uint32_t s_whist[kWaves][kMaxBins];
+    __shared__ uint32_t s_dstart[kMaxBins];
+    __shared__ uint32_t s_goff[kMaxBins];
     __shared__ uint32_t s_scan[kWaves];
 
     const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
     for (int w = 0; w < kWaves; ++w) s_whist[w][t] = 0;
-    s_goff[t] = offsets[((size_t)seg * kBins + t) * tiles + tile];
+    if (t <= mask) s_goff[t] = offsets[((size_t)seg * (mask + 1u) + t) * tiles + tile];
     __syncthreads();
 
     const size_t wbase = (size_t)tile * kTile + (size_t)wave * kWaveKeys;
@@ -78,7 +87,7 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const uint32_t* __restr
         uint32_t d = (key[i] >> shift) & mask;
         uint64_t peers = __ballot(valid);
 #pragma unroll
-        for (int b = 0; b < 8; ++b) {
+        for (int b = 0; b < kBits; ++b) {
             uint64_t bal = __ballot((d >> b) & 1u);
             peers &= ((d >> b) & 1u) ? bal : ~bal;
         }
@@ -95,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const uint32_t* __restr
     __syncthreads();
 
     // Per digit (thread t owns digit t): counts across waves, then the
-    // tile-local start of each digit (exclusive scan over the 256 digits).
+    // tile-local start of each digit (exclusive scan over the digits).
     uint32_t c = 0;
     uint32_t wex[kWaves];
 #pragma unroll
@@ -148,7 +157,7 @@ namespace pm {
 size_t radix_sort_scratch_bytes(uint32_t n, uint32_t segs) {
     const uint32_t tiles = div_up(n ? n : 1, kTile);
     const size_t all = (size_t)n * segs;
-    return carve_size({all * 4, all * 4, (size_t)segs * kBins * tiles * 4, (size_t)segs * kBins * tiles * 4});
+    return carve_size({all * 4, all * 4, (size_t)segs * kMaxBins * tiles * 4, (size_t)segs * kMaxBins * tiles * 4});
 }
 
 pm_status radix_sort_pairs(pm_ctx* ctx, const uint32_t* keys_in, const uint32_t* vals_in, uint32_t* keys_out,
@@ -159,16 +168,19 @@ pm_status radix_sort_pairs(pm_ctx* ctx, const uint32_t* keys_in, const uint32_t*
     if (key_bits < 1) key_bits = 1;
     if (key_bits > 32) key_bits = 32;
     const uint32_t tiles = div_up(n, kTile);
-    const size_t table = (size_t)segs * kBins * tiles;
-    if (table > 0xFFFFFFFFull || (uint64_t)n * segs > 0xFFFFFFFFull)
+    // the fewest passes of at most 9 bits, of digits as alike as they can be
+    const int passes = (key_bits + kMaxBits - 1) / kMaxBits;
+    const int width = (key_bits + passes - 1) / passes;
+    const size_t most = (size_t)segs * tiles << width;
+    if (most > 0xFFFFFFFFull || (uint64_t)n * segs > 0xFFFFFFFFull)
         return fail(ctx, PM_ERR_UNSUPPORTED, "radix sort: %u x %u keys", segs, n);
-    const int passes = (key_bits + 7) / 8;
     const uint32_t* src_k = keys_in;
     const uint32_t* src_v = vals_in;
     for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
-        const int bits = std::min(8, key_bits - shift);
+        const int shift = width * p;
+        const int bits = std::min(width, key_bits - shift);
         const uint32_t mask = (1u << bits) - 1u;
+        const size_t table = (size_t)segs * tiles << bits;
         // ping-pong so that the last pass lands in *_out
         const bool to_out = ((passes - 1 - p) % 2) == 0;
         uint32_t* dk = to_out ? keys_out : keys_tmp;
@@ -178,8 +190,12 @@ pm_status radix_sort_pairs(pm_ctx* ctx, const uint32_t* keys_in, const uint32_t*
         PM_CHECK_LAUNCH(ctx, "k_rs_hist");
         pm_status s = scan_u32(ctx, hist, offs, (uint32_t)table, false, nullptr);
         if (s != PM_OK) return s;
-        hipLaunchKernelGGL(k_rs_scatter, dim3(segs * tiles), dim3(kThreads), 0, ctx->stream, src_k, src_v, dk, dv, n,
-                           shift, mask, offs, tiles, n_dev);
+        if (bits > 8)
+            hipLaunchKernelGGL(k_rs_scatter<9>, dim3(segs * tiles), dim3(kThreads), 0, ctx->stream, src_k, src_v, dk,
+                               dv, n, shift, mask, offs, tiles, n_dev);
+        else
+            hipLaunchKernelGGL(k_rs_scatter<8>, dim3(segs * tiles), dim3(kThreads), 0, ctx->stream, src_k, src_v, dk,
+                               dv, n, shift, mask, offs, tiles, n_dev);
         PM_CHECK_LAUNCH(ctx, "k_rs_scatter");
         src_k = dk;
         src_v = dv;
@@ -196,8 +212,8 @@ pm_status radix_sort_pairs_auto(pm_ctx* ctx, const uint32_t* keys_in, const uint
     Carve cv{static_cast<char*>(work)};
     uint32_t* kt = cv.take<uint32_t>(all);
     uint32_t* vt = cv.take<uint32_t>(all);
-    uint32_t* hist = cv.take<uint32_t>((size_t)segs * kBins * tiles);
-    uint32_t* offs = cv.take<uint32_t>((size_t)segs * kBins * tiles);
+    uint32_t* hist = cv.take<uint32_t>((size_t)segs * kMaxBins * tiles);
+    uint32_t* offs = cv.take<uint32_t>((size_t)segs * kMaxBins * tiles);
     return radix_sort_pairs(ctx, keys_in, vals_in, keys_out, vals_out, kt, vt, n, key_bits, hist, offs, n_dev, segs);
 }
 
