@@ -60,6 +60,19 @@ __global__ void k_fill_u32(uint32_t* __restrict__ p, uint32_t v, size_t count) {
     for (; i < count; i += stride) p[i] = v;
 }
 
+// A chunk of a table as a kernel's own arguments (see put).
+constexpr uint32_t kPutWords = 960;
+struct PutChunk {
+    uint32_t* dst;
+    uint32_t n;
+    uint32_t w[kPutWords];
+};
+__global__ __launch_bounds__(256) void k_put(PutChunk) {
+    typedef const __attribute__((address_space(4))) PutChunk* Ptr;
+    Ptr c = (Ptr)__builtin_amdgcn_kernarg_segment_ptr();
+    for (uint32_t i = threadIdx.x; i < c->n; i += 256) c->dst[i] = c->w[i];
+}
+
 namespace {
 // live contexts (a grid may outlive the context it was built on) and their
 // block caches, under one lock
@@ -120,6 +133,27 @@ pm_status fill_u32(pm_ctx* ctx, uint32_t* p, uint32_t value, size_t count) {
     uint32_t blocks = (uint32_t)std::min<size_t>((count + 255) / 256, 8192);
     hipLaunchKernelGGL(k_fill_u32, dim3(blocks), dim3(256), 0, ctx->stream, p, value, count);
     PM_CHECK_LAUNCH(ctx, "k_fill_u32");
+    return PM_OK;
+}
+
+pm_status put(pm_ctx* ctx, void* dst, const void* src, size_t bytes) {
+    constexpr size_t kMax = 16384;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (bytes <= kMax && bytes % 4 == 0 && hipStreamIsCapturing(ctx->stream, &cap) == hipSuccess &&
+        cap == hipStreamCaptureStatusNone) {
+        PutChunk c;
+        for (size_t at = 0; at < bytes; at += sizeof(c.w)) {
+            const size_t len = std::min(bytes - at, sizeof(c.w));
+            c.dst = reinterpret_cast<uint32_t*>(static_cast<char*>(dst) + at);
+            c.n = (uint32_t)(len / 4);
+            std::memcpy(c.w, static_cast<const char*>(src) + at, len);
+            hipLaunchKernelGGL(k_put, dim3(1), dim3(256), 0, ctx->stream, c);
+            PM_CHECK_LAUNCH(ctx, "k_put");
+        }
+        return PM_OK;
+    }
+    PM_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, ctx->stream));
+    PM_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the source is pageable, and the caller's
     return PM_OK;
 }
 

@@ -1912,12 +1912,16 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     uint32_t* d_cbase = cv.take<uint32_t>(n_jobs);
     uint32_t* d_wbase = cv.take<uint32_t>(n_jobs);
     uint32_t* d_counter = cv.take<uint32_t>(16);
-    PM_HIP(ctx, hipMemcpyAsync(d_jobs, hp.data(), hp.size() * sizeof(KnnParams), hipMemcpyHostToDevice, ctx->stream));
-    PM_HIP(ctx, hipMemcpyAsync(d_qbase, qbase.data(), qbase.size() * 4, hipMemcpyHostToDevice, ctx->stream));
-    PM_HIP(ctx, hipMemcpyAsync(d_cbase, cell_base.data(), cell_base.size() * 4, hipMemcpyHostToDevice, ctx->stream));
-    PM_HIP(ctx, hipMemcpyAsync(d_wbase, wbase.data(), wbase.size() * 4, hipMemcpyHostToDevice, ctx->stream));
-    // the tables are copied from pageable host vectors: wait before they go
-    PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // the four tables lie side by side in the carve
+    std::vector<char> tables(reinterpret_cast<char*>(d_wbase + n_jobs) - reinterpret_cast<char*>(d_jobs));
+    auto place = [&](void* at, const void* src, size_t len) {
+        std::memcpy(tables.data() + (static_cast<char*>(at) - reinterpret_cast<char*>(d_jobs)), src, len);
+    };
+    place(d_jobs, hp.data(), hp.size() * sizeof(KnnParams));
+    place(d_qbase, qbase.data(), qbase.size() * 4);
+    place(d_cbase, cell_base.data(), cell_base.size() * 4);
+    place(d_wbase, wbase.data(), wbase.size() * 4);
+    if ((st = pm::put(ctx, d_jobs, tables.data(), tables.size())) != PM_OK) return st;
     const uint32_t* order = nullptr;
     if (sorted) {
         uint32_t* keys = cv.take<uint32_t>(nt);

@@ -5,6 +5,7 @@
 // Philox4x32-10 stream.
 #pragma once
 #include <cfloat>
+#include <cstring>
 #include <vector>
 
 #include "pm_internal.hpp"
@@ -726,8 +727,10 @@ inline SceneGeo scene_geo(const pm_scene* scene, const DevModel* d_models) {
 // one, else computed on the device over each model's triangles (the live
 // effect of create_kd_tree, KdTree.cu:395-464). d_tmp needs 32 * n_models
 // bytes. On return host_out holds the same records.
+// `tail` (nullable): a further table, at d_tail behind d_models in the same block.
 inline pm_status upload_models(pm_ctx* ctx, const pm_scene* scene, DevModel* d_models, void* d_tmp,
-                               std::vector<DevModel>& host_out) {
+                               std::vector<DevModel>& host_out, void* d_tail = nullptr, const void* tail = nullptr,
+                               size_t tail_bytes = 0) {
     const int nm = scene->n_models;
     const pm_accel* acc = scene->accel;
     std::vector<DevModel>& hm = host_out;
@@ -774,9 +777,12 @@ inline pm_status upload_models(pm_ctx* ctx, const pm_scene* scene, DevModel* d_m
         for (int i = 0; i < nm; ++i)
             for (int c = 0; c < 6; ++c) hm[i].box[c] = boxes[(size_t)i * 6 + c];
     }
-    PM_HIP(ctx, hipMemcpyAsync(d_models, hm.data(), nm * sizeof(DevModel), hipMemcpyHostToDevice, ctx->stream));
-    PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return PM_OK;
+    if (tail_bytes == 0) return pm::put(ctx, d_models, hm.data(), nm * sizeof(DevModel));
+    const size_t at = (size_t)(static_cast<char*>(d_tail) - reinterpret_cast<char*>(d_models));
+    std::vector<char> both(at + tail_bytes);
+    std::memcpy(both.data(), hm.data(), nm * sizeof(DevModel));
+    std::memcpy(both.data() + at, tail, tail_bytes);
+    return pm::put(ctx, d_models, both.data(), both.size());
 }
 
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11); one stream per

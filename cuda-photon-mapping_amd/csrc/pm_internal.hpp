@@ -170,6 +170,15 @@ pm_status radix_sort_pairs_auto(pm_ctx* ctx, const uint32_t* keys_in, const uint
 
 pm_status fill_u32(pm_ctx* ctx, uint32_t* p, uint32_t value, size_t count);
 
+// A host table to device memory, in stream order; the source is free to go on
+// return. Up to 16 KB travel as kernel arguments, 3840 bytes a launch, and the
+// host does not wait; more (and everything under stream capture, which then
+// fails as before) is copied and waited for. Each copy from pageable memory held
+// the stream for 10 to 15 us and the wait kept the host from enqueueing ahead:
+// six jobs of up to 64k queries 188 -> 168 us, a 320x240 frame 518 -> 501, one of
+// 1280x720 1448 -> 1433, a trace of 60k photons 415 -> 400.
+pm_status put(pm_ctx* ctx, void* dst, const void* src, size_t bytes);
+
 // Device blocks for grids and frames: a cached block of this context of at least
 // `bytes` (at most twice as large), else a fresh hipMalloc; *got = its size.
 // A returned block may still be read by work enqueued earlier on this

@@ -705,9 +705,8 @@ extern "C" pm_status pm_trace_photons(pm_ctx* ctx, const pm_scene* scene, uint64
     uint32_t* seg_len = cv.take<uint32_t>(segs);
 
     // model records with their AABBs (the live effect of create_kd_tree)
-    if ((st = upload_models(ctx, scene, d_models, d_tmp, hm)) != PM_OK) return st;
-    if (!ca.empty())
-        PM_HIP(ctx, hipMemcpyAsync(d_ca, ca.data(), ca.size() * sizeof(CaEntry), hipMemcpyHostToDevice, ctx->stream));
+    if ((st = upload_models(ctx, scene, d_models, d_tmp, hm, d_ca, ca.data(), ca.size() * sizeof(CaEntry))) != PM_OK)
+        return st;
 
     trace_params_base(scene, d_models, d_ca, (int)ca.size(), n_global, B, P);
     P.seed = seed;
