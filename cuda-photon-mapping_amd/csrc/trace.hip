@@ -41,11 +41,15 @@ struct TraceParams {
     int max_b;
     uint64_t path_base;
     uint32_t n_paths;
-    float* stage;     // [9][stage_depth][n_paths]
+    // [stage_depth][n_paths][9]: a photon's nine values in one line or two (lanes
+    // are at unrelated paths when they store; as nine planes 2.5M photons took
+    // 98 + 84 us to place, now 76 + 71)
+    float* stage;
     uint8_t* kind;    // [stage_depth][n_paths]: 0 global, 1 caustic
     int stage_depth;  // photon slots per path: max_b, or 1 once the global map is full
     uint32_t* cnt_g;  // [n_paths]
     uint32_t* cnt_c;  // [n_paths]
+    uint32_t* stored;  // caustic-only batches of the host's loop: a bit a path instead of the counts; else null
     int caustic_only;  // the global map is already full: stop a path once it cannot store caustics
     // models whose first event can be specular or refraction (Ks != 0 or
     // opaque < 1), as a bit mask; valid when n_models <= 64
@@ -298,7 +302,7 @@ __device__ __forceinline__ bool bounce_step(const TraceParams& P, Live& L, float
                 if ((caustic || !P.caustic_only) && L.ev < (uint32_t)P.stage_depth) {
                     const float v[9] = {ip.x, ip.y, ip.z, pp.x, pp.y, pp.z, ray.d.x, ray.d.y, ray.d.z};
 #pragma unroll
-                    for (int c = 0; c < 9; ++c) P.stage[((size_t)c * P.stage_depth + L.ev) * P.n_paths + i] = v[c];
+                    for (int c = 0; c < 9; ++c) P.stage[((size_t)L.ev * P.n_paths + i) * 9 + c] = v[c];
                     P.kind[(size_t)L.ev * P.n_paths + i] = caustic ? 1 : 0;
                     ++L.ev;
                     if (caustic)
@@ -360,6 +364,9 @@ __global__ __launch_bounds__(64) void k_trace_emit(TraceParams P, PathState* __r
     const bool all = ph == 0 || !P.spec_mask_valid;
     const uint32_t lo = blockIdx.x * P.seg, hi = min(lo + P.seg, P.n_paths);
     PathState* out = queue + (size_t)blockIdx.x * P.seg;
+    // (segments are multiples of 256 paths)
+    if (P.stored)
+        for (uint32_t w = lo / 32 + threadIdx.x; w < (hi + 31) / 32; w += 64) P.stored[w] = 0;
     uint32_t next = lo, kept = 0;  // (wave-uniform)
     bool have = false;             // a path in trial
     bool full = false;             // a direction found
@@ -370,7 +377,7 @@ __global__ __launch_bounds__(64) void k_trace_emit(TraceParams P, PathState* __r
         // lanes with a direction store their path
         bool keep = false;
         if (full) {
-            if (ph == 1) P.cnt_c[i] = 0;  // (the global counts are not read in this phase)
+            if (ph == 1 && !P.stored) P.cnt_c[i] = 0;  // (the global counts are not read in this phase)
             keep = all || may_store_caustic(P, ray);
             full = false;
         }
@@ -498,8 +505,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k
         int hm = 0;
         const bool hit = find_hit<kRecs>(P.geo, alive, L.ray, th, n, hm, S);
         if (alive && !(hit && bounce_step(P, L, th, n, hm))) {
-            P.cnt_g[L.i] = L.ng;
-            P.cnt_c[L.i] = L.nc;
+            if (P.stored) {
+                if (L.nc) atomicOr(&P.stored[L.i / 32], 1u << (L.i % 32));
+            } else {
+                P.cnt_g[L.i] = L.ng;
+                P.cnt_c[L.i] = L.nc;
+            }
             alive = false;
         }
     }
@@ -536,8 +547,32 @@ __global__ __launch_bounds__(256) void k_trace_compact(const float* __restrict__
         float* out = c ? out_c : out_g;
         if (s < cap) {
 #pragma unroll
-            for (int p = 0; p < 9; ++p) out[(size_t)p * cap + s] = stage[((size_t)p * depth + e) * n_paths + i];
+            for (int p = 0; p < 9; ++p) out[(size_t)p * cap + s] = stage[((size_t)e * n_paths + i) * 9 + p];
         }
+    }
+}
+
+// The caustic-only batches: of all paths, one in twenty stores a photon, and one
+// only. A bit a path instead of words of counts and offsets: 11.4M paths, the
+// offsets and the placing 36 + 71 -> 11 + 22 us. Below kBitPaths the launch more is not worth it (0.3M paths 397 ->
+// 402 us a trace; 2.7M 693 -> 683).
+constexpr uint32_t kBitPaths = 1u << 20;
+__global__ __launch_bounds__(256) void k_trace_words(const uint32_t* __restrict__ stored, uint32_t n_words,
+                                                    uint32_t* __restrict__ cnt) {
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w < n_words) cnt[w] = (uint32_t)__popc(stored[w]);
+}
+__global__ __launch_bounds__(256) void k_trace_place(const float* __restrict__ stage,
+                                                    const uint32_t* __restrict__ stored,
+                                                    const uint32_t* __restrict__ off, uint32_t n_paths,
+                                                    uint64_t base, float* __restrict__ out, uint32_t cap) {
+    const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
+    if (w >= (n_paths + 31) / 32) return;
+    uint64_t s = base + off[w];
+    for (uint32_t m = stored[w]; m && s < cap; m &= m - 1u, ++s) {
+        const uint32_t i = w * 32u + (uint32_t)__builtin_ctz(m);
+#pragma unroll
+        for (int p = 0; p < 9; ++p) out[(size_t)p * cap + s] = stage[(size_t)i * 9 + p];
     }
 }
 
@@ -729,14 +764,25 @@ extern "C" pm_status pm_trace_photons(pm_ctx* ctx, const pm_scene* scene, uint64
         P.path_base = paths;
         P.n_paths = nb;
         P.n_lists = lists;
+        P.stored = P.caustic_only && nb >= kBitPaths ? cnt_c : nullptr;
         if ((st = trace_batch(ctx, P, queue)) != PM_OK) return st;
-        // (in the caustic phase no path stores a global photon)
-        if (!P.caustic_only && (st = pm::scan_u32(ctx, cnt_g, off_g, nb, false, tot)) != PM_OK) return st;
-        if ((st = pm::scan_u32(ctx, cnt_c, off_c, nb, false, tot + 1)) != PM_OK) return st;
-        hipLaunchKernelGGL(k_trace_compact, dim3(pm::div_up(nb, 256)), dim3(256), 0, ctx->stream, stage, kind,
-                           P.caustic_only ? nullptr : cnt_g, cnt_c, off_g, off_c, nb, P.stage_depth, got_g, got_c,
-                           d_global9, n_global, d_caustic9, n_caustic, nullptr);
-        PM_CHECK_LAUNCH(ctx, "k_trace_compact");
+        if (P.stored) {
+            const uint32_t nw = pm::div_up(nb, 32), blocks = pm::div_up(nw, 256);
+            hipLaunchKernelGGL(k_trace_words, dim3(blocks), dim3(256), 0, ctx->stream, P.stored, nw, off_g);
+            PM_CHECK_LAUNCH(ctx, "k_trace_words");
+            if ((st = pm::scan_u32(ctx, off_g, off_c, nw, false, tot + 1)) != PM_OK) return st;
+            hipLaunchKernelGGL(k_trace_place, dim3(blocks), dim3(256), 0, ctx->stream, stage, P.stored, off_c, nb,
+                               got_c, d_caustic9, n_caustic);
+            PM_CHECK_LAUNCH(ctx, "k_trace_place");
+        } else {
+            // (in the caustic phase no path stores a global photon)
+            if (!P.caustic_only && (st = pm::scan_u32(ctx, cnt_g, off_g, nb, false, tot)) != PM_OK) return st;
+            if ((st = pm::scan_u32(ctx, cnt_c, off_c, nb, false, tot + 1)) != PM_OK) return st;
+            hipLaunchKernelGGL(k_trace_compact, dim3(pm::div_up(nb, 256)), dim3(256), 0, ctx->stream, stage, kind,
+                               P.caustic_only ? nullptr : cnt_g, cnt_c, off_g, off_c, nb, P.stage_depth, got_g, got_c, d_global9, n_global,
+                               d_caustic9, n_caustic, nullptr);
+            PM_CHECK_LAUNCH(ctx, "k_trace_compact");
+        }
         uint64_t h[2];
         PM_HIP(ctx, hipMemcpyAsync(h, tot, 16, hipMemcpyDeviceToHost, ctx->stream));
         PM_HIP(ctx, hipStreamSynchronize(ctx->stream));

@@ -80,3 +80,15 @@ def test_path_limits_around_the_segments(ctx, max_paths):
     assert st == ost
     assert np.array_equal(g.cpu().numpy()[:, :st[1]].view(np.uint32), og[:, :st[1]].view(np.uint32))
     assert np.array_equal(c.cpu().numpy()[:, :st[2]].view(np.uint32), oc[:, :st[2]].view(np.uint32))
+
+
+def test_caustic_phase_bits(ctx):
+    """Caustic-phase batches of a million paths and more mark their storing
+    paths by bits, smaller ones by counts: the photons (the first n in path
+    order, whatever the batches) are the same."""
+    scene = ctx.upload_scene(SCENES["cornell"](), accel=True)
+    maps = [ctx.trace_photons(scene, 77, 20_000, nc)[1].cpu().numpy().view(np.uint32)
+            for nc in (1_000, 30_000, 70_000, 160_000)]
+    for few, more in zip(maps, maps[1:]):
+        assert np.array_equal(more[:, :few.shape[1]], few)
+    assert maps[-1][0].max() > 0
