@@ -60,10 +60,11 @@ def native_oracle():
 
 
 def insts_per_query(cs):
-    """Wave instructions per query of the profiled gather launch (SQ_INSTS_*
-    over SQ_WAVES; the launch runs one wave per query)."""
+    """Wave instructions per query of the profiled gather launch: SQ_INSTS_*
+    over the summary's `queries` (a wave takes several), else over SQ_WAVES
+    (one wave per query)."""
     m = (cs or {}).get("per_dispatch_median", {})
-    w = m.get("SQ_WAVES")
+    w = float((cs or {}).get("queries", 0)) or m.get("SQ_WAVES")
     if not w:
         return None
     names = {"valu": "SQ_INSTS_VALU", "salu": "SQ_INSTS_SALU", "lds": "SQ_INSTS_LDS",
@@ -1084,8 +1085,8 @@ def main():
             "l1_hit_rate": cs.get("l1_hit_rate") if cs else None,
             "l2_read_latency_cycles": cs.get("l2_read_latency_cycles") if cs else None,
             "counters_stale": cs["stale"] if cs else None,
-            # the profiled launch's instructions per query (one wave per
-            # query) and the VALU lane utilisation (active lanes per VALU
+            # the profiled launch's instructions per query and the VALU lane
+            # utilisation (active lanes per VALU
             # instruction / 64)
             "insts_per_query": insts_per_query(cs),
             "valu_lane_util": valu_lane_util(cs),

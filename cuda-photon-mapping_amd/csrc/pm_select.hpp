@@ -1,7 +1,8 @@
 // Wave64 selection of the k smallest (d2, index) keys, shared by the grid
 // gather (knn.hip) and the kd-tree gather (kdknn.hip): an LDS key buffer
-// filled with ballot + mbcnt, narrowed by float-bit histograms when it fills,
-// and a register bitonic sort across the wave.
+// filled with ballot + mbcnt, narrowed when it fills (by float-bit histograms,
+// or to exactly k by one histogram linear in d2), and a counting sort over bins
+// linear in d2 for neighbour lists (a bitonic network for crowded bins).
 #pragma once
 #include <cmath>
 
