@@ -61,7 +61,7 @@ __global__ __launch_bounds__(256) void k_cell_sizes(const uint32_t* __restrict__
 // flag is read once a share and written where a count passes the limit, not at
 // every photon: one address serves about 0.2 requests a nanosecond (2M photons
 // 168 us with a read each wave, 240 with the counts in memory too).
-constexpr uint32_t kOverThreads = 1024, kOverCells = 16384;
+constexpr uint32_t kOverThreads = 1024, kOverCells = 16000;  // (under 64 KB)
 template <bool kLds>
 __global__ __launch_bounds__(kOverThreads) void k_any_over(const float* __restrict__ in9, uint32_t n, size_t stride,
                                                           GridGeom G, uint32_t n_cells, uint32_t limit,

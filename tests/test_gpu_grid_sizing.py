@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("where", ["first", "last", "spread"])
-@pytest.mark.parametrize("n,desired", [(5, 5), (3000, 50), (100_000, 5), (60_000, 1000), (300_000, 10)])
+@pytest.mark.parametrize("n,desired", [(5, 5), (3000, 50), (100_000, 5), (60_000, 1000), (78_125, 5), (300_000, 10)])
 def test_density_edge(ctx, n, desired, where):
     rng = np.random.default_rng(n + desired)
     dims = []
