@@ -508,9 +508,10 @@ __device__ __forceinline__ void finish(const KnnParams& P, WaveLds<CAP>& L, uint
     const uint32_t k = (uint32_t)P.k;
     const uint32_t m = cnt < k ? cnt : k;
     if (kLists && P.out_idx) {
-        if (cnt > 256u) {
+        constexpr uint32_t kMost = CAP == 768 ? 512u : 256u;  // (the largest k of the buffer's lists)
+        if (cnt > kMost) {
             uint64_t khi = (uint64_t)hi << 32;
-            cnt = buf_select<CAP>(L, lane, cnt, k, 256u, P.bT, khi);
+            cnt = buf_select<CAP>(L, lane, cnt, k, kMost, P.bT, khi);
             hi = (uint32_t)((khi + 0xffffffffull) >> 32);
             wave_sync();
         }
@@ -518,8 +519,10 @@ __device__ __forceinline__ void finish(const KnnParams& P, WaveLds<CAP>& L, uint
             sort_and_emit<1, CAP>(P, L, lane, q, cnt, m, hi);
         else if (cnt <= 128)
             sort_and_emit<2, CAP>(P, L, lane, q, cnt, m, hi);
-        else
+        else if (CAP != 768 || cnt <= 256)
             sort_and_emit<4, CAP>(P, L, lane, q, cnt, m, hi);
+        else
+            sort_and_emit<8, CAP>(P, L, lane, q, cnt, m, hi);
         return;
     }
     // no neighbour lists: narrow to exactly the k smallest and estimate
@@ -893,11 +896,11 @@ __device__ __forceinline__ uint32_t wave_queries(uint32_t u, uint32_t n_waves, u
 }
 
 // The single-map launch, waves in the XCD-aware order. CAP = 512: 17 KB of
-// LDS per workgroup; CAP = 768 (256 < k <= 512, estimate only): 25 KB, 6 waves
+// LDS per workgroup; CAP = 768 (256 < k <= 512): 25 KB, 6 waves
 // per SIMD; CAP = 1024 (a tuning variant: fewer narrowings) is LDS-limited to
 // 4.
 template <int CAP, bool kLists>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : CAP == 768 ? 6 : 4))) void k_knn_stream(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : CAP == 768 ? (kLists ? 5 : 6) : 4))) void k_knn_stream(
     KnnParams P) {
     __shared__ WaveLds<CAP> lds[kWaves];
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -911,10 +914,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 
                              u, P.n_waves, 0u, wave_queries(u, P.n_waves, (uint32_t)P.gq, nq));
 }
 
-// Large k (257..2048, e.g. the shipped renderer's k = 2000 / 400): one wave
-// per workgroup with a CAP-key LDS buffer (CAP >= 2k). The stream is the same;
-// the final selection narrows the buffer to exactly the k smallest keys,
-// which a bitonic network sorts in LDS.
+// Neighbour lists of k = 513..2048 (and counts alone above k = 256): one wave
+// per workgroup with a CAP-key LDS buffer (CAP >= 2k), 64 candidates a step;
+// the final selection narrows the buffer to exactly the k smallest keys, which
+// a bitonic network sorts in LDS. Up to k = 512 the stream with a 768-key buffer
+// and a register sort took its place: 2482 lists of k = 400 532 -> 194 us, 100k of
+// k = 300 2656 -> 694, of k = 512 4761 -> 1400.
 template <int CAP>
 __device__ __forceinline__ void large_one(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, uint32_t q) {
     Box B;
@@ -1611,20 +1616,27 @@ pm_status setup(pm_ctx* ctx, const pm_grid* grid, const float* d_q, uint32_t nq,
 // The streaming gather's queries per wave, for a launch of `total` queries:
 // as many as their rows fit the wave's 64 lanes, while at least kFillWaves
 // waves remain (16 a SIMD's worth: below that the chip is not full and a
-// wave's queries would only run one after the other).
-constexpr uint32_t kFillWaves = 16384;
+// wave's queries would only run one after the other). Above k = 256 a query's
+// walk dwarfs its set-up and the buffer leaves fewer waves, so the last round
+// of long waves costs more than shared set-ups give: 60k queries, k = 500
+// 920 -> 706 us at 65536 waves instead of 16384, k = 1000 1888 -> 1635, a
+// 1024x768 frame's k = 2000 the same.
+constexpr uint32_t kFillWaves = 16384, kFillWavesLarge = 65536;
 void split_waves(KnnParams& P, uint64_t total) {
     P.w = P.h > 0 ? P.h : P.rc;
     const int64_t side = 2 * (int64_t)P.w + 1, rows = side * side;
     P.nr = P.G.layout == PM_LAYOUT_LINEAR && rows <= 64 ? (int)rows : 0;
     const uint64_t fit = P.nr > 0 ? 64 / (uint64_t)P.nr : 1;
-    P.gq = (int)std::max<uint64_t>(1, std::min<uint64_t>(fit, total / kFillWaves));
+    P.gq = (int)std::max<uint64_t>(1, std::min<uint64_t>(fit, total / (P.k > 256 ? kFillWavesLarge : kFillWaves)));
     P.n_waves = pm::div_up(P.nq, (uint32_t)P.gq);
     // (a single query's wave would only wait for the second look-up of its
-    // rows, and the inner box is about the guess already)
+    // rows, 2000 queries 13 -> 18 us, but for long lists, whose second bound
+    // makes up for a guess that fell short: 2482 lists of k = 400 279 -> 194
+    // us, 10k estimates 304 -> 398; and the inner box is about the guess already)
     const float cr = 1.f + 0.6f * P.G.cell / std::max(P.r, 1e-30f);
     P.within = 1.f / (cr * cr);
-    P.guess = P.gq > 1 && P.h == 0 ? 1.2f * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
+    const bool guess = (P.gq > 1 || (P.k > 256 && P.out_idx)) && P.h == 0;
+    P.guess = guess ? 1.2f * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
 }
 
 pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint32_t* order_out) {
@@ -1649,10 +1661,10 @@ pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint
 
 pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags) {
     if (P.nq == 0) return PM_OK;
-    // radiance (and counts) without neighbour lists for k > 256: the
+    // radiance (and counts) without neighbour lists for k > 512: the
     // three-walk kernel, with an overflow list behind it
-    // (256 < k <= 512 radiance-only: one walk with the 1024-key buffer)
-    const bool mid = P.k > 256 && P.k <= 512 && !P.out_idx && P.rgb;
+    // (256 < k <= 512: one walk with the 768-key buffer)
+    const bool mid = P.k > 256 && P.k <= 512 && (P.out_idx || P.rgb);
     const bool wide = P.k > 512 && !P.out_idx && P.rgb;
     const bool sort = (flags & PM_KNN_SORT_QUERIES) != 0;
     uint32_t* ovf_list = nullptr;
@@ -1718,6 +1730,8 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
     const bool lists = P.out_idx != nullptr;
     if (two_pass)
         hipLaunchKernelGGL(k_knn_two_pass, grid_dim, block, 0, ctx->stream, P);
+    else if (mid && lists)
+        hipLaunchKernelGGL((k_knn_stream<768, true>), grid_dim, block, 0, ctx->stream, P);
     else if (mid)
         hipLaunchKernelGGL((k_knn_stream<768, false>), grid_dim, block, 0, ctx->stream, P);
     else if ((flags & PM_KNN_LARGE_BUFFER) && !lists)

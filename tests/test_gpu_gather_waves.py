@@ -132,3 +132,36 @@ def test_lists_beside_a_density_step(ctx, sparse, k):
     assert np.array_equal(idx.cpu().numpy().view(np.uint32), oi)
     assert np.array_equal(dist.cpu().numpy(), od)
     g.close()
+
+
+# Lists above k = 256: the 768-key buffer's stream, one query a wave (its first
+# walk to a guessed bound), two, a guess off (inner box), and the buffered
+# kernel from k = 513 on.
+@pytest.mark.parametrize("r,cell,flags,nq,k", [
+    (0.15, 1.0, 0, 777, 257),
+    (0.15, 1.0, pm355.KNN_SORT_QUERIES, 3001, 300),
+    (0.2, 0.5, 0, 777, 512),
+    (0.2, 0.4, pm355.KNN_INNER_BOX, 777, 400),
+    (0.1, 1.0, pm355.KNN_SORT_QUERIES, 8 * FILL + 1, 257),
+    (0.3, 0.2, 0, 300, 512),
+    (0.2, 1.0, 0, 777, 513),
+])
+def test_large_k_lists(ctx, inputs, r, cell, flags, nq, k):
+    ph, q, qn, aabb = inputs
+    q, qn = np.tile(q, (1, 2))[:, :nq].copy(), np.tile(qn, (1, 2))[:, :nq].copy()
+    g = ctx.grid_build(ph, aabb, cell_size=r * cell)
+    og = O.OracleGrid(ph, aabb, cell_size=r * cell)
+    oi, od, oc = og.knn(q, r, k)
+    idx, dist, cnt = ctx.knn(g, q, r, k, flags)
+    both = ctx.gather_batch([(g, q, qn, r, k)], flags, want_knn=True)[0]
+    ctx.sync()
+    for i, d, c in ((idx, dist, cnt), (both["idx"], both["dist"], both["count"])):
+        assert np.array_equal(c.cpu().numpy().view(np.uint32), oc)
+        assert np.array_equal(i.cpu().numpy().view(np.uint32), oi)
+        assert np.array_equal(d.cpu().numpy(), od)
+    _, o64 = O.radiance(oi, od, oc, og.photons, qn, k)
+    got = both["rgb"].cpu().numpy().astype(np.float64)
+    nan = np.isnan(o64)  # (k photons at the query itself)
+    assert np.array_equal(np.isnan(got), nan)
+    assert np.all(np.abs(got - o64)[~nan] <= 1e-5 * np.abs(o64)[~nan])
+    g.close()
