@@ -199,7 +199,7 @@ pm_status pm_grid_query_order(pm_ctx* ctx, const pm_grid* grid, const float* d_q
  * and/or pm_grid_gather_radiance (d_rgb3 from d_normals3) on its own.
  * flags: PM_KNN_SORT_QUERIES orders all queries by (job, cell) with one
  * sort. Jobs with k > 256 (the reference frame's k = 2000 / 400) run as
- * their own launches of the large-k gather (one wave per query) ahead of the
+ * their own launches of the large-k gathers ahead of the
  * shared launch. Calls on one context are ordered on its stream; the job
  * table is read before the call returns. */
 typedef struct {
