@@ -333,27 +333,6 @@ __device__ __forceinline__ void walk_runs(__amdgpu_buffer_rsrc_t rx, __amdgpu_bu
     }
 }
 
-// walk_runs over the box B, 64 rows (Morton: cells) at a time; rows and
-// their cells are pruned against Trow (T, or a smaller bound when only keys
-// below it can be kept).
-template <class F>
-__device__ __forceinline__ void walk2(const KnnParams& P, uint32_t lane, const Box& B, float qx, float qy, float qz,
-                                      float Trow, F&& f) {
-    const int nx = B.hi[0] - B.lo[0] + 1, ny = B.hi[1] - B.lo[1] + 1, nz = B.hi[2] - B.lo[2] + 1;
-    const bool linear = P.G.layout == PM_LAYOUT_LINEAR;
-    const int nseg = linear ? ny * nz : nx * ny * nz;
-    const __amdgpu_buffer_rsrc_t rx = plane_rsrc(P.px, P.n), ry = plane_rsrc(P.py, P.n), rz = plane_rsrc(P.pz, P.n);
-    for (int sbase = 0; sbase < nseg; sbase += 64) {
-        const int s = sbase + (int)lane;
-        uint32_t b = 0, len = 0;
-        if (s < nseg) row_span(P.G, P.starts, P.sizes, B, s, qx, qy, qz, Trow, b, len);
-        const uint32_t incl = wave_incl_scan(len, lane);
-        const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
-        if (total == 0) continue;
-        walk_runs(rx, ry, rz, lane, wballot(len > 0), (b + len - incl) * 4u, incl, total, qx, qy, qz, f);
-    }
-}
-
 // Radiance estimate of Raytracer.cuh:110-138 over the m kept photons held in
 // v (sorted); lanes own elements j*64 + lane.
 template <int R>
