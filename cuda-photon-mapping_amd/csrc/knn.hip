@@ -653,7 +653,7 @@ __device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr 
 // radius expected to hold somewhat more than k of them, and the rows and
 // cells are pruned to that: on surfaces the photons within b are about
 // N / (1 + 0.6 cell / sqrt(b))^2 (the walked cells against the disc), evenly
-// in d2; `guess` = 1.2 (k + 3 sqrt(k) + 2) leaves three standard deviations
+// in d2; `guess` = 1.2 (k + 3 sqrt(k) + 2) (split_waves) leaves three standard deviations
 // and a fifth for an uneven map. If the first walk finds at least k keys, the
 // k smallest are the answer; otherwise the query walks the whole box again
 // from an empty buffer, to the radius or, for lists, first to a bound sized
@@ -1615,7 +1615,10 @@ void split_waves(KnnParams& P, uint64_t total) {
     const float cr = 1.f + 0.6f * P.G.cell / std::max(P.r, 1e-30f);
     P.within = 1.f / (cr * cr);
     const bool guess = (P.gq > 1 || (P.k > 256 && P.out_idx)) && P.h == 0;
-    P.guess = guess ? 1.2f * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
+    // (lists, whose next bound is close, do without the fifth: k = 50 959 -> 937
+    // us, k = 100 595 -> 540; from k = 200 on, 794 -> 799, it is worth having)
+    const float spare = P.out_idx && P.k <= 128 ? 1.f : 1.2f;
+    P.guess = guess ? spare * ((float)P.k + 3.f * std::sqrt((float)P.k) + 2.f) : INFINITY;
 }
 
 pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint32_t* order_out) {
