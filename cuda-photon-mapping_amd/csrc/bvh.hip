@@ -57,10 +57,11 @@ __device__ __forceinline__ int delta(const uint32_t* __restrict__ k, int n, int 
 }
 
 // Internal node i of n - 1 (Karras 2012, Algorithm 1). Children: internal
-// nodes as global indices base + g, leaves as ~(t0 + sorted triangle).
+// nodes as global indices base + g, leaves as ~(t0 + sorted triangle). With the
+// children, the node's first record slot and its number of triangles.
 __global__ __launch_bounds__(256) void k_bvh_nodes(const uint32_t* __restrict__ keys, const uint32_t* __restrict__ vals,
-                                                   int n, uint32_t t0, int base, float4* __restrict__ nodes,
-                                                   int* __restrict__ parent_int, int* __restrict__ parent_leaf) {
+                                                   int n, uint32_t t0, uint32_t slot0, int base,
+                                                   float4* __restrict__ nodes, int* __restrict__ parent_int, int* __restrict__ parent_leaf) {
     int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (i >= n - 1) return;
     const int d = (delta(keys, n, i, i + 1) - delta(keys, n, i, i - 1)) >= 0 ? 1 : -1;
@@ -97,7 +98,7 @@ __global__ __launch_bounds__(256) void k_bvh_nodes(const uint32_t* __restrict__ 
     }
     if (i == 0) parent_int[0] = -1;
     nodes[4 * (size_t)(base + i) + 3] =
-        make_float4(__int_as_float(c0), __int_as_float(c1), __int_as_float((int)t0 + lo), __int_as_float(hi - lo + 1));
+        make_float4(__int_as_float(c0), __int_as_float(c1), __int_as_float((int)slot0 + lo), __int_as_float(hi - lo + 1));
 }
 
 // Boxes pass between threads of different blocks (and XCDs): device-scope
@@ -148,14 +149,14 @@ __global__ __launch_bounds__(256) void k_bvh_boxes(const float* __restrict__ t9,
     }
 }
 
-// Triangle records: slot t0 + j holds triangle t0 + (vals ? vals[j] : j). A
-// model with a BVH has its records in the tree's leaf order.
+// A model's triangle records: slot slot0 + j holds triangle t0 + (vals ? vals[j]
+// : j). A model with a BVH has its records in the tree's leaf order.
 __global__ __launch_bounds__(256) void k_tri_recs(const float* __restrict__ t9, const uint32_t* __restrict__ vals,
-                                                 uint32_t t0, uint32_t n, float4* __restrict__ recs) {
+                                                 uint32_t t0, uint32_t n, uint32_t slot0, float4* __restrict__ recs) {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     const uint32_t t = t0 + (vals ? vals[j] : j);
-    pmg::store_rec(recs, t0 + j, t,
+    pmg::store_rec(recs, slot0 + j, t,
                    pmg::make_rec(pmg::load_v(t9, t, 0), pmg::load_v(t9, t, 1), pmg::load_v(t9, t, 2)));
 }
 
@@ -219,7 +220,8 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
     const int nm = scene->n_models;
     std::vector<uint32_t> ranges(2 * (size_t)nm);
     uint32_t max_n = 0;
-    uint64_t n_nodes = 0;
+    uint64_t n_nodes = 0, n_slots = 0;
+    std::vector<uint32_t> slots((size_t)nm);
     for (int i = 0; i < nm; ++i) {
         const pm_model& s = scene->h_models[i];
         if (s.tri_end > scene->n_tris || s.tri_begin > s.tri_end)
@@ -227,6 +229,8 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
         ranges[2 * i] = s.tri_begin;
         ranges[2 * i + 1] = s.tri_end;
         uint32_t c = s.tri_end - s.tri_begin;
+        slots[i] = (uint32_t)n_slots;  // (read where n_slots < 2^29)
+        n_slots += c;
         if (c >= kMinTris) {
             n_nodes += c - 1;
             max_n = std::max(max_n, c);
@@ -270,21 +274,18 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
             return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %llu nodes", (unsigned long long)n_nodes));
         }
     }
-    // (a wide leaf's code holds its first record slot in 29 bits)
-    if (scene->n_tris && scene->n_tris < (1u << 29)) {
-        hipError_t e = hipMalloc(&a->recs, (size_t)scene->n_tris * 80);
-        if (e != hipSuccess) {
-            a->recs = nullptr;
-            return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %u triangles", scene->n_tris));
-        }
-        if (n_nodes && (e = hipMalloc(&a->wide, n_nodes * 128)) != hipSuccess) {
+    // The records and the four-wide trees (a wide leaf's code holds its first
+    // record slot in 29 bits). Overlapping ranges can make them large: where they
+    // do not fit in memory the scene goes without, and is walked model by model.
+    if (n_slots && n_slots < (1ull << 29) && nm <= kRecModels) {
+        if (hipMalloc(&a->recs, (size_t)n_slots * 80) != hipSuccess) a->recs = nullptr;
+        if (a->recs && n_nodes && hipMalloc(&a->wide, n_nodes * 128) != hipSuccess) {
             a->wide = nullptr;
-            return bail(pm::fail(ctx, PM_ERR_NOMEM, "pm_accel_build: %llu nodes", (unsigned long long)n_nodes));
+            (void)hipFree(a->recs);
+            a->recs = nullptr;
         }
-        hipLaunchKernelGGL(k_tri_recs, dim3(pm::div_up(scene->n_tris, 256)), dim3(256), 0, ctx->stream,
-                           scene->d_tris9, (const uint32_t*)nullptr, 0u, scene->n_tris, a->recs);
-        hipError_t le = hipGetLastError();
-        if (le != hipSuccess) return bail(pm::hip_fail(ctx, le, "k_tri_recs"));
+        if (!a->recs) (void)hipGetLastError();
+        a->slots = slots;
     }
     // exact model AABBs (the reference's create_kd_tree result)
     hipError_t e = hipMemcpyAsync(d_tb, ranges.data(), ranges.size() * 4, hipMemcpyHostToDevice, ctx->stream);
@@ -299,7 +300,14 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
     int base = 0;
     for (int i = 0; i < nm; ++i) {
         const uint32_t t0 = ranges[2 * i], n = ranges[2 * i + 1] - t0;
-        if (n < kMinTris) continue;
+        if (n < kMinTris) {
+            if (n && a->recs) {
+                hipLaunchKernelGGL(k_tri_recs, dim3(1), dim3(256), 0, ctx->stream, scene->d_tris9,
+                                   (const uint32_t*)nullptr, t0, n, a->slots[i], a->recs);
+                PM_CHECK_LAUNCH(ctx, "k_tri_recs");
+            }
+            continue;
+        }
         const float* bx = &a->boxes[6 * (size_t)i];
         float sc[3], big = 1.0f;
         for (int c = 0; c < 3; ++c) {
@@ -315,14 +323,14 @@ extern "C" pm_status pm_accel_build(pm_ctx* ctx, const pm_scene* scene, pm_accel
             return bail(st);
         if ((st = pm::fill_u32(ctx, arrive, 0u, n)) != PM_OK) return bail(st);
         hipLaunchKernelGGL(k_bvh_nodes, dim3(pm::div_up(n - 1, 256)), dim3(256), 0, ctx->stream, keys_s, vals_s,
-                           (int)n, t0, base, a->nodes, parent_int, parent_leaf);
+                           (int)n, t0, slots[i], base, a->nodes, parent_int, parent_leaf);
         PM_CHECK_LAUNCH(ctx, "k_bvh_nodes");
         hipLaunchKernelGGL(k_bvh_boxes, dim3(pm::div_up(n, 256)), dim3(256), 0, ctx->stream, scene->d_tris9, vals_s,
                            (int)n, t0, base, margin, a->nodes, parent_int, parent_leaf, arrive);
         PM_CHECK_LAUNCH(ctx, "k_bvh_boxes");
         if (a->recs) {
             hipLaunchKernelGGL(k_tri_recs, dim3(pm::div_up(n, 256)), dim3(256), 0, ctx->stream, scene->d_tris9,
-                               vals_s, t0, n, a->recs);
+                               vals_s, t0, n, a->slots[i], a->recs);
             hipLaunchKernelGGL(k_bvh_wide, dim3(pm::div_up(n - 1, 256)), dim3(256), 0, ctx->stream, a->nodes, base,
                                (int)(n - 1), a->wide);
             PM_CHECK_LAUNCH(ctx, "k_bvh_wide");

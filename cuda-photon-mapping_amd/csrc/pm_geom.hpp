@@ -49,9 +49,10 @@ struct Ray {
 
 // Per-model record on the device (material of Material.cuh:4-31, the
 // triangle range of the model, its AABB and id). bvh is the model's root
-// node in the scene's BVH node array, or -1 to test every triangle.
+// node in the scene's BVH node array, or -1 to test every triangle; rec is its
+// first slot in the scene's triangle records (where there are any).
 struct DevModel {
-    uint32_t t0, t1;
+    uint32_t t0, t1, rec;
     float kd[3], ks[3], ke[3];
     float ior, opaque, shininess;
     int32_t id, bvh;
@@ -59,6 +60,9 @@ struct DevModel {
 };
 
 }  // namespace pmg
+
+// The most models of a scene whose rays take the records (a bit each in a mask).
+constexpr int kRecModels = 32;
 
 // Scene acceleration structure: per-model AABBs and triangle BVHs, built once
 // per geometry and shared by photon tracing and eye-ray rendering.
@@ -70,7 +74,11 @@ struct pm_accel {
     std::vector<int32_t> roots;    // [n_models] root node, -1 = no BVH (every triangle tested)
     uint32_t n_nodes = 0;
     float4* nodes = nullptr;  // [n_nodes][4]
-    float4* recs = nullptr;   // [n_tris][5] (pmg::TriRec), a BVH's triangles in its leaf order
+    // Triangle records (pmg::TriRec, 5 float4 each), for scenes of at most
+    // kRecModels models: every model's own, from slot slots[model] on (ranges may
+    // overlap, and a BVH's are in its leaf order), else in index order.
+    float4* recs = nullptr;
+    std::vector<uint32_t> slots;  // [n_models]
     float4* wide = nullptr;   // [n_nodes][8]: the four-wide trees, by binary node (with recs)
 };
 
@@ -404,7 +412,7 @@ __device__ __forceinline__ bool scene_hit(const DevModel* __restrict__ M, int n_
 }
 
 // The scene as the ray kernels see it. recs (with an acceleration structure,
-// at most 32 models): scene_nearest; brute / tree are the model masks without
+// at most kRecModels models): scene_nearest; brute / tree are the model masks without
 // and with a BVH (models of no triangles in neither).
 struct SceneGeo {
     const DevModel* models;
@@ -649,8 +657,8 @@ __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, con
             if (t == te && pend) {
                 cm = __builtin_ctz(pend);
                 pend &= pend - 1;
-                t = G.models[cm].t0;
-                te = G.models[cm].t1;
+                t = G.models[cm].rec;
+                te = t + (G.models[cm].t1 - G.models[cm].t0);
             }
             if (!__builtin_amdgcn_ballot_w64(t < te)) break;
             if (t < te) {
@@ -661,7 +669,7 @@ __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, con
                 if (rec_hit(G.recs, t, r, pt, pu, tri) && pt < best) {
                     best = pt;
                     bm = cm;
-                    bt = t;
+                    bt = tri;
                     uvw = pu;
                 }
                 ++t;
@@ -712,7 +720,7 @@ inline SceneGeo scene_geo(const pm_scene* scene, const DevModel* d_models) {
     const pm_accel* acc = scene->accel;
     if (!acc || acc->n_models != scene->n_models) return G;  // (upload_models refuses another scene's)
     G.bvh = acc->nodes;
-    if (scene->n_models > 32) return G;
+    if (scene->n_models > kRecModels) return G;
     G.recs = acc->recs;
     G.wide = acc->wide;
     for (int i = 0; i < scene->n_models; ++i) {
@@ -756,6 +764,7 @@ inline pm_status upload_models(pm_ctx* ctx, const pm_scene* scene, DevModel* d_m
         d.shininess = s.shininess;
         d.id = s.id;
         d.bvh = acc ? acc->roots[i] : -1;
+        d.rec = acc && acc->recs ? acc->slots[i] : 0u;
         if (acc)
             for (int c = 0; c < 6; ++c) d.box[c] = acc->boxes[6 * (size_t)i + c];
     }
