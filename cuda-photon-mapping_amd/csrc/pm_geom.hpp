@@ -355,19 +355,22 @@ __device__ __forceinline__ bool bvh_hit(const float4* __restrict__ nodes, int ro
 // the new t is smaller. A model with a BVH finds its nearest triangle by
 // traversal (same result); the others test every triangle, with triangle
 // data read at wave-uniform indices (scalar loads). kTrees = false tests
-// every triangle of every model.
+// every triangle of every model. A lane that is not alive joins the
+// (wave-uniform) triangle loops and hits nothing: it opens no model's box (a
+// null ray in its place opened all boxes behind or above it, and walked their
+// trees: traces of 1000 photons in 45 models took 1958 us instead of 762).
 template <bool kTrees>
 __device__ __forceinline__ bool scene_hit(const DevModel* __restrict__ M, int n_models,
                                           const float* __restrict__ t9, const float* __restrict__ n9,
-                                          const float4* __restrict__ bvh, const Ray& r, float& t_out, V3& n_out,
-                                          int& m_out, BvhStack S) {
+                                          const float4* __restrict__ bvh, bool alive, const Ray& r, float& t_out,
+                                          V3& n_out, int& m_out, BvhStack S) {
     float best = 0.f;
     int bm = -1;
     V3 bn = v3(0, 0, 0);
     V3 inv = v3(0, 0, 0);
     bool have_inv = false;
     for (int m = 0; m < n_models; ++m) {
-        const bool in_box = box_hit(M[m].box, r);
+        const bool in_box = alive && box_hit(M[m].box, r);
         if (!__builtin_amdgcn_ballot_w64(in_box)) continue;
         float mt = FLT_MAX;
         bool found = false;
@@ -690,7 +693,7 @@ __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, con
     const bool again = lost || (found && best == 0.f);
     if (__builtin_amdgcn_ballot_w64(again)) {
         if (again)
-            found = scene_hit<false>(G.models, G.n_models, G.tris, G.nrms, nullptr, r, t_out, n_out, m_out,
+            found = scene_hit<false>(G.models, G.n_models, G.tris, G.nrms, nullptr, true, r, t_out, n_out, m_out,
                                      BvhStack{nullptr});
     }
     return found;
@@ -702,13 +705,8 @@ template <bool kRecs>
 __device__ __forceinline__ bool find_hit(const SceneGeo& G, bool alive, const Ray& r, float& t_out, V3& n_out,
                                          int& m_out, RayLds& L) {
     if constexpr (kRecs) return scene_nearest(G, alive, r, t_out, n_out, m_out, L);
-    // all lanes join the (wave-uniform) triangle loops; a lane without a ray
-    // shoots a null one that hits nothing
-    Ray rr = r;
-    if (!alive) rr.d = v3(0, 0, 0);
-    return scene_hit<true>(G.models, G.n_models, G.tris, G.nrms, G.bvh, rr, t_out, n_out, m_out,
-                           BvhStack{L.stack + __lane_id()}) &&
-           alive;
+    return scene_hit<true>(G.models, G.n_models, G.tris, G.nrms, G.bvh, alive, r, t_out, n_out, m_out,
+                           BvhStack{L.stack + __lane_id()});
 }
 
 inline SceneGeo scene_geo(const pm_scene* scene, const DevModel* d_models) {
