@@ -354,12 +354,10 @@ __device__ __forceinline__ bool bvh_hit(const float4* __restrict__ nodes, int ro
 // normals; a model's hit replaces the current one if the current t is 0 or
 // the new t is smaller. A model with a BVH finds its nearest triangle by
 // traversal (same result); the others test every triangle, with triangle
-// data read at wave-uniform indices (scalar loads). kTrees = false tests
-// every triangle of every model. A lane that is not alive joins the
+// data read at wave-uniform indices (scalar loads). A lane that is not alive joins the
 // (wave-uniform) triangle loops and hits nothing: it opens no model's box (a
 // null ray in its place opened all boxes behind or above it, and walked their
 // trees: traces of 1000 photons in 45 models took 1958 us instead of 762).
-template <bool kTrees>
 __device__ __forceinline__ bool scene_hit(const DevModel* __restrict__ M, int n_models,
                                           const float* __restrict__ t9, const float* __restrict__ n9,
                                           const float4* __restrict__ bvh, bool alive, const Ray& r, float& t_out,
@@ -376,8 +374,8 @@ __device__ __forceinline__ bool scene_hit(const DevModel* __restrict__ M, int n_
         bool found = false;
         V3 uvw = v3(0, 0, 0);
         uint32_t ti = 0;
-        const int root = kTrees ? M[m].bvh : -1;
-        if (kTrees && root >= 0) {
+        const int root = M[m].bvh;
+        if (root >= 0) {
             if (!have_inv) {
                 inv = inv_dir(r.d);
                 have_inv = true;
@@ -626,7 +624,8 @@ __device__ __forceinline__ void tree_nearest(const SceneGeo& G, uint32_t pend, c
 //     alone.
 // That is scene_hit's result unless a hit has t == 0 exactly (its fold lets
 // any later model replace such a hit): those rays, and any whose stack was
-// too small, take scene_hit itself. `alive`: lanes without a ray take part in
+// too small, take scene_hit itself, by the models' trees (a single ray of
+// 65536 paths past every triangle of a scene of 44k cost 3.4 ms). `alive`: lanes without a ray take part in
 // nothing; all 64 lanes call.
 __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, const Ray& r, float& t_out, V3& n_out,
                                               int& m_out, RayLds& L) {
@@ -693,8 +692,8 @@ __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, con
     const bool again = lost || (found && best == 0.f);
     if (__builtin_amdgcn_ballot_w64(again)) {
         if (again)
-            found = scene_hit<false>(G.models, G.n_models, G.tris, G.nrms, nullptr, true, r, t_out, n_out, m_out,
-                                     BvhStack{nullptr});
+            found = scene_hit(G.models, G.n_models, G.tris, G.nrms, G.bvh, true, r, t_out, n_out, m_out,
+                              BvhStack{L.stack + __lane_id()});
     }
     return found;
 }
@@ -705,8 +704,8 @@ template <bool kRecs>
 __device__ __forceinline__ bool find_hit(const SceneGeo& G, bool alive, const Ray& r, float& t_out, V3& n_out,
                                          int& m_out, RayLds& L) {
     if constexpr (kRecs) return scene_nearest(G, alive, r, t_out, n_out, m_out, L);
-    return scene_hit<true>(G.models, G.n_models, G.tris, G.nrms, G.bvh, alive, r, t_out, n_out, m_out,
-                           BvhStack{L.stack + __lane_id()});
+    return scene_hit(G.models, G.n_models, G.tris, G.nrms, G.bvh, alive, r, t_out, n_out, m_out,
+                     BvhStack{L.stack + __lane_id()});
 }
 
 inline SceneGeo scene_geo(const pm_scene* scene, const DevModel* d_models) {

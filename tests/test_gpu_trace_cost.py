@@ -9,7 +9,7 @@ import time
 import numpy as np
 import pytest
 
-from pm355.scenes import PM_MODEL_DTYPE, Scene, _model, cornell_box, uv_sphere
+from pm355.scenes import PM_MODEL_DTYPE, Scene, _model, cornell_box, random_scene, uv_sphere
 
 pytestmark = pytest.mark.gpu
 
@@ -59,3 +59,13 @@ def test_lanes_without_a_path_open_no_box(ctx):
     (rec, by_model), maps = _times(ctx, [scene, _padded(scene, 33)], 1000)
     assert np.array_equal(*maps)
     assert by_model < 3.5 * rec
+
+
+def test_rays_of_the_general_walk_take_the_trees(ctx):
+    """A few rays of this scene of 44k triangles leave the records' walk for the
+    general one (a hit at t == 0): past all triangles a trace took 5.8 times the
+    model-by-model time, by the trees half of it."""
+    scene = random_scene(3)
+    (rec, by_model), maps = _times(ctx, [scene, _padded(scene, 33)], 1000)
+    assert np.array_equal(*maps)
+    assert rec < 1.5 * by_model
