@@ -231,11 +231,15 @@ constexpr int kBvhStack = 64;  // a node's key prefix grows down the tree: depth
 constexpr int kLdsStack = 12;
 constexpr int kRayWaves = 4;  // waves of a block of every kernel that traces rays
 // One wave's LDS: the traversal stacks (a column of [kLdsStack][64] per lane,
-// or of [kWideStack][16] per group of four lanes), and what the groups of
-// tree_nearest pass to and from the rays' own lanes.
+// or of [kWideStack][16] per group of four lanes), and with records what the
+// groups of tree_nearest pass to and from the rays' own lanes.
 constexpr int kWideStack = kLdsStack * 4;
+template <bool kRecs>
 struct RayLds {
     uint2 stack[kLdsStack * 64];
+};
+template <>
+struct RayLds<true> : RayLds<false> {
     float4 hit[64];    // t, u, v, w
     uint2 who[64];     // model, triangle
     uint32_t list[64];
@@ -447,7 +451,7 @@ __device__ __forceinline__ float quadf(float v) {
 // lowest triangle). lost: the ray's stack was too small; its result is not to
 // be used. All 64 lanes take part.
 __device__ __forceinline__ void tree_nearest(const SceneGeo& G, uint32_t pend, const Ray& r, float& best, int& bm,
-                                             uint32_t& bt, V3& uvw, bool& lost, RayLds& L) {
+                                             uint32_t& bt, V3& uvw, bool& lost, RayLds<true>& L) {
     const uint32_t lane = __lane_id(), j = lane & 3u, g = lane >> 2;
     const uint64_t wait = __builtin_amdgcn_ballot_w64(pend != 0);
     const uint32_t n_wait = (uint32_t)__builtin_popcountll(wait);
@@ -628,7 +632,7 @@ __device__ __forceinline__ void tree_nearest(const SceneGeo& G, uint32_t pend, c
 // 65536 paths past every triangle of a scene of 44k cost 3.4 ms). `alive`: lanes without a ray take part in
 // nothing; all 64 lanes call.
 __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, const Ray& r, float& t_out, V3& n_out,
-                                              int& m_out, RayLds& L) {
+                                              int& m_out, RayLds<true>& L) {
     const RayInv R = ray_inv(r);
     uint32_t mask = 0, doubt = 0;
     for (int m = 0; m < G.n_models; ++m) {
@@ -702,10 +706,12 @@ __device__ __forceinline__ bool scene_nearest(const SceneGeo& G, bool alive, con
 // records (G.recs).
 template <bool kRecs>
 __device__ __forceinline__ bool find_hit(const SceneGeo& G, bool alive, const Ray& r, float& t_out, V3& n_out,
-                                         int& m_out, RayLds& L) {
-    if constexpr (kRecs) return scene_nearest(G, alive, r, t_out, n_out, m_out, L);
-    return scene_hit(G.models, G.n_models, G.tris, G.nrms, G.bvh, alive, r, t_out, n_out, m_out,
-                     BvhStack{L.stack + __lane_id()});
+                                         int& m_out, RayLds<kRecs>& L) {
+    if constexpr (kRecs)
+        return scene_nearest(G, alive, r, t_out, n_out, m_out, L);
+    else
+        return scene_hit(G.models, G.n_models, G.tris, G.nrms, G.bvh, alive, r, t_out, n_out, m_out,
+                         BvhStack{L.stack + __lane_id()});
 }
 
 inline SceneGeo scene_geo(const pm_scene* scene, const DevModel* d_models) {

@@ -68,8 +68,8 @@ struct Plan {
 };
 
 __global__ __launch_bounds__(256) void k_render_rays(RaysParams P) {
-    __shared__ RayLds s_ray[kRayWaves];
-    RayLds& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    __shared__ RayLds<false> s_ray[kRayWaves];
+    RayLds<false>& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
     // 8x8 pixel tile per wave: coherent rays share model AABB outcomes
     const uint32_t lane = threadIdx.x & 63, wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
     const int W = P.cam.w, H = P.cam.h;

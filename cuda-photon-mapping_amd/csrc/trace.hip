@@ -445,19 +445,22 @@ __device__ __forceinline__ void take_path(const TraceParams& P, const PathState*
 // VGPRs; at five waves it spills and takes 1.5 times as long) and by the VALU:
 // the Cornell box's 2M + 500k photons take 0.65 + 0.87 ms here and 0.05 + 0.18
 // ms of emission, where the model-by-model walk with emission inside took
-// 1.42 + 1.09 + 0.31 ms.
+// 1.42 + 1.09 + 0.31 ms. Without records (more than 32 models, or no trees)
+// that walk still runs here, at five waves a SIMD: 10 spilled VGPRs cost it less
+// than the fifth wave gives (1M photons among 125 models 3.97 ms at four waves,
+// 3.67 at five).
 constexpr uint32_t kListSegs = 128;  // segments of a list, at most (the host sees to it)
 
 template <bool kRecs>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_trace_pool(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kRecs ? 4 : 5))) void k_trace_pool(
     TraceParams P, const PathState* __restrict__ queue) {
-    __shared__ RayLds s_ray[kRayWaves];
+    __shared__ RayLds<kRecs> s_ray[kRayWaves];
     __shared__ uint32_t s_pre[kListSegs + 1];
     __shared__ uint32_t s_next;
     const int ph = batch_phase(P);
     if (ph == 2) return;  // (a planned batch with both maps full)
     P.caustic_only = ph;
-    RayLds& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
+    RayLds<kRecs>& S = s_ray[__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)];
     const uint32_t mine = blockIdx.x < P.n_segs ? (P.n_segs - blockIdx.x - 1u) / P.n_lists + 1u : 0u;
     if (threadIdx.x < 64) {
         uint32_t sum = 0;
