@@ -6,7 +6,7 @@
 // the reference's 44-block Blelloch scan with its software grid barrier
 // (PrefixScanSum.cuh:12-279, CudaGridSynchronizer.cuh:14-27), which needs all
 // blocks co-resident; here a tile only waits on tiles that took a lower
-// ordered id, so any number of tiles may be in flight. Inputs of 6M
+// ordered id, so any number of tiles may be in flight. Inputs of 4M
 // elements and more take a two-level scan instead (tile sums, a scan of the
 // sums, tiles rescanned from their offsets), whose workgroups never wait on
 // each other.
@@ -29,9 +29,9 @@ constexpr int kItems2 = 16;
 constexpr int kTile2 = kThreads2 * kItems2;  // 4096
 
 constexpr uint64_t kStatusAgg = 1, kStatusIncl = 2;
-// inputs of at least this many elements take the two-level scan (4M: 16.2 us in
-// a single pass, 25.6 in two levels; 8M: 28.9 and 25.0)
-constexpr uint32_t kTwoLevelMin = 6u << 20;
+// inputs of at least this many elements take the two-level scan (4.2M: 17.5 us in
+// a single pass, 15.4 in two levels; 6M: 22.8 and 19.9)
+constexpr uint32_t kTwoLevelMin = 1u << 22;
 
 __device__ __forceinline__ uint64_t pack_state(uint32_t epoch, uint64_t status, uint32_t value) {
     return ((uint64_t)epoch << 34) | (status << 32) | value;
