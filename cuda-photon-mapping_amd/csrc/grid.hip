@@ -53,16 +53,14 @@ __global__ __launch_bounds__(256) void k_cell_sizes(const uint32_t* __restrict__
 }
 
 // Whether any cell holds more than `limit` photons (analyze_density_kernel,
-// PhotonGrid.cu:70-141, needs its maximum for this comparison only): photons
-// are counted by atomics until a workgroup finds that a count has passed the
-// limit. The answer does not depend on the order. A workgroup counts its share
-// in LDS first where the cells fit (kLds: 2M photons of the default 1000 a
-// cell are 2k cells, and neighbours in the input fall in the same cell). The
-// flag is read once a share and written where a count passes the limit, not at
-// every photon: one address serves about 0.2 requests a nanosecond (2M photons
-// 168 us with a read each wave, 240 with the counts in memory too).
+// PhotonGrid.cu:70-141, needs its maximum for this comparison only), for grids
+// of at most kOverCells cells: a workgroup counts its share in LDS (2M photons
+// of the default 1000 a cell are 2k cells, and neighbours in the input fall in
+// the same cell) and adds its counts to the others'. The answer does not depend
+// on the order. The flag is read once a share and written where a count passes
+// the limit, not at every photon: one address serves about 0.2 requests a
+// nanosecond (2M photons 168 us with a read each wave, 16 so).
 constexpr uint32_t kOverThreads = 1024, kOverCells = 16000;  // (under 64 KB)
-template <bool kLds>
 __global__ __launch_bounds__(kOverThreads) void k_any_over(const float* __restrict__ in9, uint32_t n, size_t stride,
                                                           GridGeom G, uint32_t n_cells, uint32_t limit,
                                                           uint32_t* __restrict__ counts, uint32_t* __restrict__ over) {
@@ -72,27 +70,32 @@ __global__ __launch_bounds__(kOverThreads) void k_any_over(const float* __restri
     if (t == 0) s_over = __hip_atomic_load(over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (s_over) return;  // (workgroup-uniform)
-    if (kLds) {
-        for (uint32_t c = t; c < n_cells; c += kOverThreads) s_counts[c] = 0;
-        __syncthreads();
-    }
+    for (uint32_t c = t; c < n_cells; c += kOverThreads) s_counts[c] = 0;
+    __syncthreads();
     for (uint32_t i = blockIdx.x * kOverThreads + t; i < n; i += gridDim.x * kOverThreads) {
         const int x = pmd::cell_coord(in9[i], G.mn[0], G.cell, G.g[0]);
         const int y = pmd::cell_coord(in9[stride + i], G.mn[1], G.cell, G.g[1]);
         const int z = pmd::cell_coord(in9[2 * stride + i], G.mn[2], G.cell, G.g[2]);
-        if (atomicAdd((kLds ? s_counts : counts) + pmd::cell_index(G, x, y, z), 1u) == limit)
+        if (atomicAdd(s_counts + pmd::cell_index(G, x, y, z), 1u) == limit)
             __hip_atomic_store(over, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    if (kLds) {
-        __syncthreads();
-        for (uint32_t c = t; c < n_cells; c += kOverThreads) {
-            const uint32_t v = s_counts[c];
-            if (v == 0) continue;
-            const uint32_t was = atomicAdd(&counts[c], v);
-            if (was <= limit && was + v > limit)
-                __hip_atomic_store(over, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+    __syncthreads();
+    for (uint32_t c = t; c < n_cells; c += kOverThreads) {
+        const uint32_t v = s_counts[c];
+        if (v == 0) continue;
+        const uint32_t was = atomicAdd(&counts[c], v);
+        if (was <= limit && was + v > limit)
+            __hip_atomic_store(over, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+}
+
+// The maximum itself, over the cell sizes of a grid that is built.
+__global__ __launch_bounds__(256) void k_max_u32(const uint32_t* __restrict__ a, uint32_t n, uint32_t* __restrict__ out) {
+    uint32_t m = 0;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) m = max(m, a[i]);
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) m = max(m, (uint32_t)__shfl_xor(m, d, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(out, m);
 }
 
 // assign_photons_to_cells (PhotonGrid.cu:152-174) with the slot taken from
@@ -224,7 +227,7 @@ size_t grid_bytes(uint32_t n_cells, uint32_t n_cap) {
     return pm::carve_size({(size_t)n_cells * 4, (size_t)n_cells * 4, (size_t)n_cap * 36, (size_t)n_cap * 4});
 }
 
-// scratch of one build: the density flag, keys, sorted keys, sorted
+// scratch of one build: the fullest cell (the sizing rule), keys, sorted keys, sorted
 // order, radix work, records
 size_t build_scratch_bytes(uint32_t n) {
     return pm::carve_size({256, (size_t)n * 4, (size_t)n * 4, (size_t)n * 4, pm::radix_sort_scratch_bytes(n),
@@ -320,12 +323,12 @@ pm_status grid_build_strided(pm_ctx* ctx, const float* d_photons9, uint32_t n, s
         return pm::fail(ctx, PM_ERR_UNSUPPORTED, "pm_grid_build: grid too large for cell %g", (double)cell);
 
     pm_status st;
-    uint32_t* over = nullptr;
+    uint32_t* most = nullptr;
     {
         void* w = nullptr;
         if ((st = pm::scratch_reserve(ctx, build_scratch_bytes(n), &w)) != PM_OK) return st;
         pm::Carve cv{static_cast<char*>(w)};
-        over = cv.take<uint32_t>(64);
+        most = cv.take<uint32_t>(64);
     }
 
     // a fresh allocation of capacity n at dims dd
@@ -341,51 +344,75 @@ pm_status grid_build_strided(pm_ctx* ctx, const float* d_photons9, uint32_t n, s
         out_g = g;
         return PM_OK;
     };
-    // whether a cell at dims d holds more than `limit` photons (the counts are
-    // taken in g's memory, ahead of its build)
+    auto read = [&](const uint32_t* word, uint32_t& h) -> pm_status {
+        PM_HIP(ctx, hipMemcpyAsync(&h, word, 4, hipMemcpyDeviceToHost, ctx->stream));
+        PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        return PM_OK;
+    };
+    // whether a cell at dims d holds more than `limit` photons, by a count (taken
+    // in g's memory, ahead of its build)
     auto any_over = [&](pm_grid* g, uint32_t limit, bool& yes) -> pm_status {
-        uint32_t* counts = static_cast<uint32_t*>(g->mem);
+        // (the flag behind the counts: its photons alone take more room)
+        uint32_t *counts = static_cast<uint32_t*>(g->mem), *over = counts + d.n_cells;
         pm_status s;
-        if ((s = pm::fill_u32(ctx, counts, 0u, d.n_cells)) != PM_OK || (s = pm::fill_u32(ctx, over, 0u, 1)) != PM_OK)
-            return s;
-        const dim3 blocks(std::min(pm::div_up(n, 4 * kOverThreads), 512u)), threads(kOverThreads);
-        if (d.n_cells <= kOverCells)
-            hipLaunchKernelGGL(k_any_over<true>, blocks, threads, d.n_cells * 4, ctx->stream, d_photons9, n, stride,
-                               geom_of(aabb, d, layout), d.n_cells, limit, counts, over);
-        else
-            hipLaunchKernelGGL(k_any_over<false>, blocks, threads, 0, ctx->stream, d_photons9, n, stride,
-                               geom_of(aabb, d, layout), d.n_cells, limit, counts, over);
+        if ((s = pm::fill_u32(ctx, counts, 0u, d.n_cells + 1u)) != PM_OK) return s;
+        hipLaunchKernelGGL(k_any_over, dim3(std::min(pm::div_up(n, 4 * kOverThreads), 512u)), dim3(kOverThreads),
+                           d.n_cells * 4, ctx->stream, d_photons9, n, stride, geom_of(aabb, d, layout), d.n_cells,
+                           limit, counts, over);
         PM_CHECK_LAUNCH(ctx, "k_any_over");
         uint32_t h = 0;
-        PM_HIP(ctx, hipMemcpyAsync(&h, over, 4, hipMemcpyDeviceToHost, ctx->stream));
-        PM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        s = read(over, h);
         yes = h != 0;
-        return PM_OK;
+        return s;
+    };
+    // the same of a grid that is built
+    auto max_over = [&](pm_grid* g, uint32_t limit, bool& yes) -> pm_status {
+        pm_status s;
+        if ((s = pm::fill_u32(ctx, most, 0u, 1)) != PM_OK) return s;
+        hipLaunchKernelGGL(k_max_u32, dim3(std::min<uint32_t>(pm::div_up(d.n_cells, 256), 4096)), dim3(256), 0,
+                           ctx->stream, g->desc.d_cell_sizes, d.n_cells, most);
+        PM_CHECK_LAUNCH(ctx, "k_max_u32");
+        uint32_t h = 0;
+        s = read(most, h);
+        yes = h > limit;
+        return s;
     };
 
     pm_grid* g = nullptr;
     if ((st = take(d, g)) != PM_OK) return st;
+    bool built = false;
     if (!(cell_size > 0.f)) {
         // analyze_density (PhotonGrid.cu:92-141): at the reference size, the
         // fullest cell decides whether the cells shrink to the size for
-        // desired / 5. The count alone decides, so the grid is built once, at
-        // the final size (2M photons: 230 us, 375 with a build at each size; the
-        // count takes 22).
+        // desired / 5. The count alone decides, so where it is cheap the grid is
+        // built once, at the final size (2M photons: 206 us, 375 with a build at
+        // each size; the count takes 16). It is not where the cells do not fit
+        // LDS (counts by atomics in memory: 16M photons 5.5 ms, 182 if they lie
+        // in one cell; a build takes 1.1): there the grid is built and its
+        // fullest cell looked up.
+        const bool count = d.n_cells <= kOverCells;
+        const uint32_t limit = 5u * (uint32_t)desired;
         bool shrink = false;
-        if ((st = any_over(g, 5u * (uint32_t)desired, shrink)) != PM_OK) {
+        if (!count) {
+            st = enqueue_build(ctx, d_photons9, n, stride, aabb, d, layout, g);
+            built = true;
+        }
+        if (st == PM_OK) st = count ? any_over(g, limit, shrink) : max_over(g, limit, shrink);
+        if (st != PM_OK) {
             pm_grid_destroy(g);
             return st;
         }
         if (shrink) {
             pm_grid_destroy(g);
             g = nullptr;
+            built = false;
             cell = reference_cell(n, aabb, std::max(1, desired / 5));
             if (!(cell > 0.f) || !make_dims(aabb, cell, layout, d))
                 return pm::fail(ctx, PM_ERR_UNSUPPORTED, "pm_grid_build: grid too large for cell %g", (double)cell);
             if ((st = take(d, g)) != PM_OK) return st;
         }
     }
-    if ((st = enqueue_build(ctx, d_photons9, n, stride, aabb, d, layout, g)) != PM_OK) {
+    if (!built && (st = enqueue_build(ctx, d_photons9, n, stride, aabb, d, layout, g)) != PM_OK) {
         pm_grid_destroy(g);
         return st;
     }
