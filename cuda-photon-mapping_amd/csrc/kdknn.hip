@@ -12,8 +12,10 @@
 // searched from an empty buffer when it is below 0.7 of the full threshold,
 // and the full ball comes last. The first guess is 0.16 of the threshold for
 // a wave's first queries, then a running mean of 1.4 times the squared
-// distances its earlier queries needed, at least 0.01 of the threshold (500k queries, k = 50: 813 -> 740 us;
-// k = 200: 3.6 -> 2.8 ms). The kept set is the k smallest keys whatever balls
+// distances its earlier queries needed, at least 0.01 of the threshold (500k
+// queries, k = 50: 813 -> 740 us; k = 200: 3.6 -> 2.8 ms), and the full ball where
+// that mean is above 0.4 of it (50k queries beside the photons' reach 5.2 -> 3.75
+// ms: nearly all of them walked two balls). The kept set is the k smallest keys whatever balls
 // were tried. A full key buffer keeps its k smallest, and the search goes on
 // below the k-th, photons and half-spaces alike.
 //
@@ -33,6 +35,13 @@
 // within 330 photons' reach 2464 us, now 667; 1000 queries 31 us both ways
 // (the longest query alone). 16 lanes to a query: 808 us instead of 690 (and k = 200
 // 2.5 -> 4.2 ms, LDS for fewer waves).
+//
+// A launch of few queries (kFew) waits for its longest, and 32 lanes take longer
+// over that than 64 do. There a query that has its wave to itself is walked by all
+// lanes, with the idle group's memory for its stack (walk_alone): 1000 queries of
+// k = 200 in 16M photons 151 -> 70 us (79 with 64 lanes to every query), of k = 100
+// in 10k photons 41 -> 23 (26), 20k queries off the surfaces of 16M photons 10.5 ->
+// 3.8 ms (3.6).
 //
 // A subtree is skipped only when the squared distance from the query to its
 // splitting plane exceeds the threshold by a relative 1e-5, so no photon
@@ -149,13 +158,70 @@ __device__ __forceinline__ float finish_query(KdPtr kp, WaveLds<CAP>& L, uint32_
     return m < k ? kp->T : dk;
 }
 
+// A query that the wave has no other beside: the walk of its ball by all 64
+// lanes, with `stk`, the idle group's memory, for its stack (top entries). All
+// else as in k_kd_knn, where a group walks; cnt and T are the query's, wave-uniform.
+template <int CAP>
+__device__ __forceinline__ void walk_alone(KdPtr kp0, WaveLds<CAP>& B, uint32_t* stk, uint32_t lane, uint32_t lev,
+                                           uint32_t via_l, uint32_t via_r, uint64_t bottom, float q0, float q1,
+                                           float q2, uint32_t top, uint32_t& cnt, float& T) {
+    constexpr uint32_t kAll = sizeof(KdLds<CAP>) / 4;
+    const float4* __restrict__ nodes = kp0->nodes;
+    const uint32_t cap = kp0->cap, k = (uint32_t)kp0->k;
+    float prune = T * (1.0f + 1e-5f) + 1e-30f;
+    while (top > 0) {
+        if (cnt > CAP - 64u) {
+            T = lin_select<CAP>(B, lane, cnt, k, __float_as_uint(T) + 1u, opaque(kp0)->bT);
+            wave_sync();
+            cnt = k;
+            prune = T * (1.0f + 1e-5f) + 1e-30f;
+        }
+        uint32_t node = stk[lane < top ? top - 1u - lane : 0u];
+        bool sub = top == 1;
+        if (top > kAll / 2) sub = __builtin_amdgcn_readfirstlane(node) < cap >> 4;
+        const uint32_t n = sub ? 1u : min(min(top, 64u), (uint32_t)max((int)(kAll - kMaxLevels - top), 1));
+        if (sub) node = (__builtin_amdgcn_readfirstlane(node) << lev) + (lane & 31u);
+        const uint64_t has = wballot(lane < (sub ? kGroup - 1u : n)) & wballot(node < cap);
+        wave_sync();  // every pop is read before the pushes reuse the slots
+        top -= n;
+        const float4 rec = nodes[min(node, cap - 1u)];
+        const uint32_t w = __float_as_uint(rec.w);
+        const float d2 = kd_dist2(rec.x, rec.y, rec.z, q0, q1, q2);
+        const bool py = (w >> 30) == 1u, px = (w >> 30) == 0u;
+        const float diff = (px ? q0 : py ? q1 : q2) - (px ? rec.x : py ? rec.y : rec.z);
+        const uint64_t ok = has & wballot(w != 0xFFFFFFFFu), inner = ok & wballot(node < cap >> 1);
+        const uint64_t out = wballot(diff * diff > prune), right = wballot(diff > 0.f);
+        uint64_t go_l = inner & ~(out & right), go_r = inner & ~(out & wballot(diff < 0.f));
+        uint64_t in = ok & wballot(d2 <= T);
+        if (sub) {
+            const float num = q0 + q1 + q2;
+            const uint64_t reached =
+                num == num ? wballot(((via_l & ~(uint32_t)go_l) | (via_r & ~(uint32_t)go_r)) == 0u) : 0ull;
+            in &= reached;
+            go_l &= reached & bottom;
+            go_r &= reached & bottom;
+        }
+        if (__builtin_amdgcn_inverse_ballot_w64(in)) B.buf[cnt + mbcnt(in)] = make_key(d2, w & 0x3FFFFFFFu);
+        cnt += (uint32_t)__popcll(in);
+        const uint64_t both = go_l & go_r, any = go_l | go_r;
+        const uint32_t nf = top + (uint32_t)__popcll(both);
+        const uint64_t nr = (both & right) | (go_r & ~go_l);
+        const uint32_t near = 2u * node + (__builtin_amdgcn_inverse_ballot_w64(nr) ? 2u : 1u);
+        if (__builtin_amdgcn_inverse_ballot_w64(both)) stk[top + mbcnt(both)] = 4u * node + 3u - near;
+        if (__builtin_amdgcn_inverse_ballot_w64(any)) stk[nf + mbcnt(any)] = near;
+        top = nf + (uint32_t)__popcll(any);
+        wave_sync();
+    }
+}
+
 // The half of a wave mask that holds this lane.
 __device__ __forceinline__ uint32_t half_of(uint64_t m, uint32_t lane) {
     return lane >= 32 ? (uint32_t)(m >> 32) : (uint32_t)m;
 }
 
-template <int CAP>
-__global__ __launch_bounds__(64 * kWaves) void k_kd_knn(KdParams P0) {
+template <int CAP, bool kFew>
+__global__ __launch_bounds__(64 * kWaves)
+__attribute__((amdgpu_waves_per_eu(CAP == 128 && !kFew ? 7 : 5))) void k_kd_knn(KdParams P0) {
     __shared__ KdLds<CAP> lds[kWaves][kGroups];
     const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t gl = lane % kGroup, grp = lane / kGroup, below = (1u << gl) - 1u;
@@ -206,68 +272,90 @@ __global__ __launch_bounds__(64 * kWaves) void k_kd_knn(KdParams P0) {
             q0 = kp->qx[q];
             q1 = kp->qy[q];
             q2 = kp->qz[q];
-            start(first);
+            // (a ball of nearly the radius would mostly be walked a second time)
+            start(first < 0.4f * kp->T ? first : kp->T);
         }
     };
     take(next + grp);
     next += kGroups;
     wave_sync();
-    while (wballot(top > 0)) {
-        // a full buffer keeps its k smallest keys, and the search goes on below the k-th
-        for (uint64_t full = wballot(cnt > CAP - kGroup); full;) {
-            const uint32_t l0 = (uint32_t)__builtin_ctzll(full), g = l0 / kGroup;
-            const float d = lin_select<CAP>(W[g].sel, lane, __builtin_amdgcn_readlane(cnt, l0), k,
-                                            __builtin_amdgcn_readlane(__float_as_uint(T), l0) + 1u, opaque(kp0)->bT);
+    uint64_t live = wballot(q < end);  // (kFew; wave-uniform)
+    while (kFew ? live != 0 : wballot(q < end) != 0) {
+        if (kFew && live != ~0ull) {
+            const uint32_t l0 = (uint32_t)__builtin_ctzll(live), g = l0 / kGroup;
+            const auto of = [&](float v) {
+                return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), l0));
+            };
+            const uint32_t n = __builtin_amdgcn_readlane(top, l0);
+            uint32_t* stk = reinterpret_cast<uint32_t*>(&W[1u - g]);
+            for (uint32_t i = lane; i < n; i += 64) stk[i] = W[g].stk[i];
             wave_sync();
-            if (grp == g) {
-                cnt = k;
-                bound(d);
+            uint32_t c = __builtin_amdgcn_readlane(cnt, l0);
+            float t = of(T);
+            walk_alone<CAP>(kp0, W[g].sel, stk, lane, lev, via_l, via_r, bottom, of(q0), of(q1), of(q2), n, c, t);
+            cnt = c;
+            top = 0;
+            T = t;
+        } else {
+            // a full buffer keeps its k smallest keys, and the search goes on below the k-th
+            for (uint64_t full = wballot(cnt > CAP - kGroup); full;) {
+                const uint32_t l0 = (uint32_t)__builtin_ctzll(full), g = l0 / kGroup;
+                const float d = lin_select<CAP>(W[g].sel, lane, __builtin_amdgcn_readlane(cnt, l0), k,
+                                                __builtin_amdgcn_readlane(__float_as_uint(T), l0) + 1u, opaque(kp0)->bT);
+                wave_sync();
+                if (grp == g) {
+                    cnt = k;
+                    bound(d);
+                }
+                full &= ~(0xffffffffull << l0);
             }
-            full &= ~(0xffffffffull << l0);
+            const uint32_t n = min(min(top, kGroup), (uint32_t)max((int)(kStackCap - kMaxLevels - top), 1));
+            const uint64_t sub = wballot(top == 1);
+            const uint32_t e = top - (top == 1 ? 1u : gl + 1u);
+            uint32_t node = L.stk[e < kStackCap ? e : 0u];
+            if (top == 1) node = (node << lev) + gl;
+            const uint64_t has = wballot(gl < (top == 1 ? kGroup - 1u : n)) & wballot(node < cap);
+            wave_sync();  // every pop is read before the pushes reuse the slots
+            top -= n;
+            const float4 rec = nodes[min(node, cap - 1u)];
+            const uint32_t w = __float_as_uint(rec.w);
+            const float d2 = kd_dist2(rec.x, rec.y, rec.z, q0, q1, q2);
+            const bool py = (w >> 30) == 1u, px = (w >> 30) == 0u;
+            const float diff = (px ? q0 : py ? q1 : q2) - (px ? rec.x : py ? rec.y : rec.z);
+            const uint64_t ok = has & wballot(w != 0xFFFFFFFFu), inner = ok & wballot(node < cap >> 1);
+            // left subtree: coordinate <= median; right: >= median
+            const uint64_t out = wballot(diff * diff > prune), right = wballot(diff > 0.f);
+            uint64_t go_l = inner & ~(out & right), go_r = inner & ~(out & wballot(diff < 0.f));
+            uint64_t in = ok & wballot(d2 <= T);
+            if (sub) {
+                // the nodes that the steps above them lead to; the bottom ones' children go on the stack
+                // (every walk begins so: nothing is reached from a position that is not a number)
+                const float num = q0 + q1 + q2;
+                const uint64_t reached =
+                    ~sub | (wballot(((via_l & ~half_of(go_l, lane)) | (via_r & ~half_of(go_r, lane))) == 0u) &
+                            wballot(num == num));
+                in &= reached;
+                go_l &= reached & (bottom | ~sub);
+                go_r &= reached & (bottom | ~sub);
+            }
+            const uint32_t hin = half_of(in, lane);
+            if (__builtin_amdgcn_inverse_ballot_w64(in))
+                L.sel.buf[cnt + __popc(hin & below)] = make_key(d2, w & 0x3FFFFFFFu);
+            cnt += __popc(hin);
+            // far children below the near ones, which are popped first: a full
+            // buffer's k-th key then soon cuts off the rest
+            const uint64_t both = go_l & go_r, any = go_l | go_r;
+            if (any) {
+                const uint32_t hb = half_of(both, lane), ha = half_of(any, lane);
+                const uint32_t nf = top + __popc(hb);
+                const uint64_t nr = (both & right) | (go_r & ~go_l);
+                const uint32_t near = 2u * node + (__builtin_amdgcn_inverse_ballot_w64(nr) ? 2u : 1u);
+                if (__builtin_amdgcn_inverse_ballot_w64(both)) L.stk[top + __popc(hb & below)] = 4u * node + 3u - near;
+                if (__builtin_amdgcn_inverse_ballot_w64(any)) L.stk[nf + __popc(ha & below)] = near;
+                top = nf + __popc(ha);
+            }
+            wave_sync();
         }
-        const uint32_t n = min(min(top, kGroup), (uint32_t)max((int)(kStackCap - kMaxLevels - top), 1));
-        const uint64_t sub = wballot(top == 1);
-        const uint32_t e = top - (top == 1 ? 1u : gl + 1u);
-        uint32_t node = L.stk[e < kStackCap ? e : 0u];
-        if (top == 1) node = (node << lev) + gl;
-        const uint64_t has = wballot(gl < (top == 1 ? kGroup - 1u : n)) & wballot(node < cap);
-        wave_sync();  // every pop is read before the pushes reuse the slots
-        top -= n;
-        const float4 rec = nodes[min(node, cap - 1u)];
-        const uint32_t w = __float_as_uint(rec.w);
-        const float d2 = kd_dist2(rec.x, rec.y, rec.z, q0, q1, q2);
-        const bool py = (w >> 30) == 1u, px = (w >> 30) == 0u;
-        const float diff = (px ? q0 : py ? q1 : q2) - (px ? rec.x : py ? rec.y : rec.z);
-        const uint64_t ok = has & wballot(w != 0xFFFFFFFFu), inner = ok & wballot(node < cap >> 1);
-        // left subtree: coordinate <= median; right: >= median
-        const uint64_t out = wballot(diff * diff > prune), right = wballot(diff > 0.f);
-        uint64_t go_l = inner & ~(out & right), go_r = inner & ~(out & wballot(diff < 0.f));
-        uint64_t in = ok & wballot(d2 <= T);
-        if (sub) {
-            // the nodes that the steps above them lead to; the bottom ones' children go on the stack
-            const uint64_t reached =
-                ~sub | wballot(((via_l & ~half_of(go_l, lane)) | (via_r & ~half_of(go_r, lane))) == 0u);
-            in &= reached;
-            go_l &= reached & (bottom | ~sub);
-            go_r &= reached & (bottom | ~sub);
-        }
-        const uint32_t hin = half_of(in, lane);
-        if (__builtin_amdgcn_inverse_ballot_w64(in))
-            L.sel.buf[cnt + __popc(hin & below)] = make_key(d2, w & 0x3FFFFFFFu);
-        cnt += __popc(hin);
-        // far children below the near ones, which are popped first: a full
-        // buffer's k-th key then soon cuts off the rest
-        const uint64_t both = go_l & go_r, any = go_l | go_r;
-        if (any) {
-            const uint32_t hb = half_of(both, lane), ha = half_of(any, lane);
-            const uint32_t nf = top + __popc(hb);
-            const uint64_t nr = (both & right) | (go_r & ~go_l);
-            const uint32_t near = 2u * node + (__builtin_amdgcn_inverse_ballot_w64(nr) ? 2u : 1u);
-            if (__builtin_amdgcn_inverse_ballot_w64(both)) L.stk[top + __popc(hb & below)] = 4u * node + 3u - near;
-            if (__builtin_amdgcn_inverse_ballot_w64(any)) L.stk[nf + __popc(ha & below)] = near;
-            top = nf + __popc(ha);
-        }
-        wave_sync();
         if (wballot(top == 0) & wballot(q < end)) {
             KdPtr kp = opaque(kp0);
             const float Tr = kp->T;
@@ -292,6 +380,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_kd_knn(KdParams P0) {
                 ++next;
                 done &= ~(0xffffffffull << l0);
             }
+            if (kFew) live = wballot(q < end);
             wave_sync();
         }
     }
@@ -328,14 +417,19 @@ extern "C" pm_status pm_kdtree_knn(pm_ctx* ctx, const pm_kdtree* tree, const flo
     // 12288 waves that way, and up to eight where it has more (the ball learned
     // from the wave's own queries: 500k queries 962 -> 690 us; 100k: 230 us at
     // one, 203 at four, 230 at eight, which leaves 6k waves).
-    P.per_wave = kGroups * std::min(8u, std::max(1u, nq / (kGroups * 12288u)));
-    const dim3 grid(pm::div_up(nq, kWaves * P.per_wave)), block(64 * kWaves);
-    if (k <= 64)
-        hipLaunchKernelGGL(k_kd_knn<128>, grid, block, 0, ctx->stream, P);
-    else if (k <= 128)
-        hipLaunchKernelGGL(k_kd_knn<256>, grid, block, 0, ctx->stream, P);
-    else
-        hipLaunchKernelGGL(k_kd_knn<384>, grid, block, 0, ctx->stream, P);
+    // Few queries: while a wave takes fewer than eight, each with a wave of its own
+    // up to 6144. The buffer then leaves room for 64 keys a step; where that doubles
+    // it, the bound is half (90k queries of k = 64 in 300k photons 312 us with it, 265
+    // with groups alone). 10k to 4M photons, groups alone against it: 20k queries of
+    // k = 200 13 % slower, of k = 64 10 %, 90k of k = 100 9 %; a search of k < 8 is a
+    // few steps long, and from 3072 queries on their number counts (6000 of k = 1:
+    // 17.2 us, with it 18.6).
+    const uint32_t most = (k > 32 && k <= 64 ? 4u : 8u) * 12288u;
+    const bool few = nq < most && (k >= 8 || nq <= 3072u);
+    P.per_wave = few && nq <= 6144u ? 1u : kGroups * std::min(8u, std::max(1u, nq / (kGroups * 12288u)));
+    const auto kernel = few ? (k <= 32 ? k_kd_knn<128, true> : k <= 128 ? k_kd_knn<256, true> : k_kd_knn<384, true>)
+                            : (k <= 64 ? k_kd_knn<128, false> : k <= 128 ? k_kd_knn<256, false> : k_kd_knn<384, false>);
+    hipLaunchKernelGGL(kernel, dim3(pm::div_up(nq, kWaves * P.per_wave)), dim3(64 * kWaves), 0, ctx->stream, P);
     PM_CHECK_LAUNCH(ctx, "k_kd_knn");
     return PM_OK;
 }
