@@ -605,6 +605,12 @@ __device__ __forceinline__ void finish_params(KnnParams& Pf, ParamsPtr kp) {
 template <int CAP>
 constexpr uint32_t kNarrowTo = CAP == 512 ? 256 : 512;
 
+// What a narrowing reads; kOne: held through the walk (two scalar reads at each
+// narrowing, 1 us of 56 where a query's walk has dozens of them).
+struct Narrow {
+    uint32_t k, bT;
+};
+
 // One step of the streaming selection over two candidates per lane (index
 // sa / sb, squared distance d2a / d2b, lanes holding one: masks am / bm):
 // appends the keys whose d2 bits lie below the acceptance bound hi to the
@@ -615,17 +621,21 @@ constexpr uint32_t kNarrowTo = CAP == 512 ? 256 : 512;
 // lets in besides lie above k kept ones, and are dropped by the finish.
 // Every predicate is a ballot of a plain compare combined in SGPRs; the
 // writing lanes come back from their mask.
-template <int CAP>
-__device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr kp0, uint64_t am, uint32_t sa,
-                                      float d2a, uint64_t bm, uint32_t sb, float d2b, uint32_t& cnt, uint32_t& hi) {
+template <int CAP, bool kOne>
+__device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr kp0, Narrow own, uint64_t am,
+                                      uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b, uint32_t& cnt,
+                                      uint32_t& hi) {
     uint64_t bala = am & wballot(__float_as_uint(d2a) < hi), balb = bm & wballot(__float_as_uint(d2b) < hi);
     uint32_t na = (uint32_t)__popcll(bala), nb = (uint32_t)__popcll(balb);
     if (cnt + na + nb > (uint32_t)CAP) {
         // leaves at most kNarrowTo keys, room for this step's 128
         wave_sync();
-        ParamsPtr kp = opaque(kp0);
+        if constexpr (!kOne) {
+            ParamsPtr kp = opaque(kp0);
+            own = Narrow{(uint32_t)kp->k, kp->bT};
+        }
         uint64_t khi = (uint64_t)hi << 32;
-        cnt = buf_select<CAP>(L, lane, cnt, (uint32_t)kp->k, kNarrowTo<CAP>, kp->bT, khi);
+        cnt = buf_select<CAP>(L, lane, cnt, own.k, kNarrowTo<CAP>, own.bT, khi);
         hi = (uint32_t)((khi + 0xffffffffull) >> 32);
         bala = am & wballot(__float_as_uint(d2a) < hi);
         balb = bm & wballot(__float_as_uint(d2b) < hi);
@@ -749,17 +759,73 @@ __device__ __forceinline__ void setup_queries(ParamsPtr kp0, uint32_t lane, cons
     W.rows = rows_all;
 }
 
+// setup_queries for the one query of a wave (at position p0), whose values are
+// then wave-uniform: the three axes' cells and face gaps are worked side by side
+// in lanes 0..2, and there is no guess. 83 VALU instructions fewer of a query's 455;
+// 8000 to 14000 unsorted queries in 200k photons (k = 64 within r = 0.02, the mean
+// of eight maps) 17.2 to 24.0 us with setup_queries, 16.2 to 22.0 so.
+__device__ __forceinline__ void setup_query(ParamsPtr kp0, uint32_t lane, const uint32_t* __restrict__ order,
+                                            uint32_t p0, uint32_t qb, WaveQueries& W) {
+    ParamsPtr kp = opaque(kp0);
+    const GridGeom G = geom_of(kp);
+    const auto uni = [](float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); };
+    const uint32_t q = __builtin_amdgcn_readfirstlane(order ? order[p0] : p0) - qb;
+    const float x = uni(kp->qx[q]), y = uni(kp->qy[q]), z = uni(kp->qz[q]);
+    const float v = lane == 1 ? y : lane == 2 ? z : x, mn = lane == 1 ? G.mn[1] : lane == 2 ? G.mn[2] : G.mn[0];
+    const int g = lane == 1 ? G.g[1] : lane == 2 ? G.g[2] : G.g[0];
+    const int c = pmd::cell_coord(v, mn, G.cell, g);
+    const int cx = __builtin_amdgcn_readlane(c, 0), cy = __builtin_amdgcn_readlane(c, 1),
+              cz = __builtin_amdgcn_readlane(c, 2);
+    const float T = kp->T;
+    uint32_t hib = __float_as_uint(T) + 1u, len = 0, b = 0;
+    float Trow = T;
+    const int h = kp->h, nr = kp->nr;
+    if (h > 0) {
+        const uint32_t gb = __float_as_uint(inner_gap(v, max(0, c - h), min(g - 1, c + h), g, mn, G.cell));
+        const float gap = fminf(fminf(__uint_as_float(__builtin_amdgcn_readlane(gb, 0)),
+                                      __uint_as_float(__builtin_amdgcn_readlane(gb, 1))),
+                                __uint_as_float(__builtin_amdgcn_readlane(gb, 2)));
+        hib = __builtin_amdgcn_readfirstlane(min(__float_as_uint(gap * gap * 0.999f), hib));
+        Trow = fminf(T, __uint_as_float(hib));
+    }
+    W.end = W.d4 = 0;
+    W.rows = 0;
+    if (nr > 0) {
+        const int w = kp->w, side = 2 * w + 1;
+        int zi, yi;
+        small_divmod((int)lane, side, __builtin_amdgcn_rcpf((float)side), zi, yi);
+        const int yy = cy - w + yi, zz = cz - w + zi;
+        if ((int)lane < nr && yy >= 0 && yy < G.g[1] && zz >= 0 && zz < G.g[2])
+            row_cells(G, kp->starts, kp->sizes, yy, zz, max(0, cx - w), min(G.g[0] - 1, cx + w), x, y, z, Trow, b, len);
+        W.end = wave_incl_scan(len, lane);
+        W.d4 = (b + len - W.end) * 4u;
+        W.rows = wballot(len > 0);
+    }
+    W.q = q;
+    W.hib = hib;
+    W.x = x;
+    W.y = y;
+    W.z = z;
+}
+// A value of the wave's queries for the one whose first lane is lb.
+template <bool kOne>
+__device__ __forceinline__ uint32_t of_query(uint32_t v, uint32_t lb) {
+    return kOne ? __builtin_amdgcn_readfirstlane(v) : __builtin_amdgcn_readlane(v, lb);
+}
+template <bool kOne>
+__device__ __forceinline__ float of_query(float v, uint32_t lb) {
+    return __uint_as_float(of_query<kOne>(__float_as_uint(v), lb));
+}
+
 // f (as walk_runs calls it) over the candidates of the query whose first
 // lane is lb: the rows set up for it (batch), or the whole box, or the inner
 // one, looked up now, with rows and cells pruned to the d2 bits below hi.
-template <class F>
+template <bool kOne, class F>
 __device__ __forceinline__ void walk_query(ParamsPtr kp0, uint32_t lane, const WaveQueries& W, uint32_t lb, bool batch,
                                            bool inner, uint32_t hi, F&& f) {
     ParamsPtr kp = opaque(kp0);
     const int nr = kp->nr;
-    const float qx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.x), lb));
-    const float qy = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.y), lb));
-    const float qz = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(W.z), lb));
+    const float qx = of_query<kOne>(W.x, lb), qy = of_query<kOne>(W.y, lb), qz = of_query<kOne>(W.z, lb);
     const uint32_t n = kp->n;
     const __amdgpu_buffer_rsrc_t rx = plane_rsrc(kp->px, n), ry = plane_rsrc(kp->py, n), rz = plane_rsrc(kp->pz, n);
     for (int sbase = 0;; sbase += 64) {
@@ -767,7 +833,7 @@ __device__ __forceinline__ void walk_query(ParamsPtr kp0, uint32_t lane, const W
         uint64_t rows;
         bool last = true;
         if (batch) {
-            rows = W.rows & ((~0ull >> (64 - nr)) << lb);
+            rows = kOne ? W.rows : W.rows & ((~0ull >> (64 - nr)) << lb);
             total = __builtin_amdgcn_readlane(W.end, lb + (uint32_t)nr - 1u);
         } else {
             // 64 rows (Morton: cells) of the box, one per lane
@@ -816,28 +882,32 @@ __device__ __forceinline__ uint32_t next_bound(uint32_t hi, uint32_t cnt, bool f
     return __float_as_uint(T) + 1u;
 }
 
-template <int CAP, bool kLists>
+template <int CAP, bool kLists, bool kOne>
 __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint32_t lane,
                                             const uint32_t* __restrict__ order, uint32_t p0, uint32_t stride,
                                             uint32_t qb, uint32_t nqw) {
     WaveQueries W;
-    setup_queries(kp0, lane, order, p0, stride, qb, nqw, W);
-    for (uint32_t i = 0; i < nqw; ++i) {
+    if constexpr (kOne)
+        setup_query(kp0, lane, order, p0, qb, W);
+    else
+        setup_queries(kp0, lane, order, p0, stride, qb, nqw, W);
+    for (uint32_t i = 0; i < (kOne ? 1u : nqw); ++i) {
         uint32_t cnt, hi, lb;
         {
             ParamsPtr kp = opaque(kp0);
-            lb = i * (uint32_t)kp->nr;
-            hi = __builtin_amdgcn_readlane(W.hib, lb);
+            lb = kOne ? 0u : i * (uint32_t)kp->nr;
+            hi = of_query<kOne>(W.hib, lb);
             // (a first walk below the radius is of the inner box when there
             // is one)
             const uint32_t hit = __float_as_uint(kp->T) + 1u;
             bool batch = kp->nr > 0, inner = kp->h > 0 && kp->nr == 0, part = hi < hit;
             [[maybe_unused]] bool first = true;
+            const Narrow own = kOne ? Narrow{(uint32_t)kp->k, kp->bT} : Narrow{};
             for (;;) {
                 cnt = 0;
-                walk_query(kp0, lane, W, lb, batch, inner, hi,
+                walk_query<kOne>(kp0, lane, W, lb, batch, inner, hi,
                            [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
-                               push2<CAP>(L, lane, kp0, am, sa, d2a, bm, sb, d2b, cnt, hi);
+                               push2<CAP, kOne>(L, lane, kp0, own, am, sa, d2a, bm, sb, d2b, cnt, hi);
                            });
                 wave_sync();
                 // with at least k such keys, the k smallest keys overall are
@@ -864,8 +934,8 @@ __device__ __forceinline__ void stream_wave(ParamsPtr kp0, WaveLds<CAP>& L, uint
         // k (it starts above CAP - 128 >= k keys), so cnt >= k after one.
         KnnParams Pf;
         finish_params(Pf, opaque(kp0));
-        finish<CAP, kLists>(Pf, L, lane, __builtin_amdgcn_readlane(W.q, lb), cnt, hi);
-        wave_sync();  // the buffer is read before the next query's keys
+        finish<CAP, kLists>(Pf, L, lane, of_query<kOne>(W.q, lb), cnt, hi);
+        if (!kOne) wave_sync();  // the buffer is read before the next query's keys
     }
 }
 
@@ -874,14 +944,24 @@ __device__ __forceinline__ uint32_t wave_queries(uint32_t u, uint32_t n_waves, u
     return min(gq, (nq - u - 1u) / n_waves + 1u);  // u < nq
 }
 
+// The argument lines are read one after the other as their values are needed,
+// each a first miss of the XCD's; here all at once (100 queries 9.6 -> 8.8 us).
+__device__ __forceinline__ void touch_args() {
+    typedef const __attribute__((address_space(4))) uint32_t* WordPtr;
+    WordPtr w = (WordPtr)__builtin_amdgcn_kernarg_segment_ptr();
+    static_assert(sizeof(KnnParams) > 3 * 64 && sizeof(KnnParams) <= 4 * 64, "four lines");
+    asm volatile("" ::"s"(w[0]), "s"(w[16]), "s"(w[32]), "s"(w[48]));
+}
+
 // The single-map launch, waves in the XCD-aware order. CAP = 512: 17 KB of
 // LDS per workgroup; CAP = 768 (256 < k <= 512): 25 KB, 6 waves
 // per SIMD; CAP = 1024 (a tuning variant: fewer narrowings) is LDS-limited to
 // 4.
-template <int CAP, bool kLists>
+template <int CAP, bool kLists, bool kOne = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 ? 7 : CAP == 768 ? (kLists ? 5 : 6) : 4))) void k_knn_stream(
     KnnParams P) {
     __shared__ WaveLds<CAP> lds[kWaves];
+    if (kOne) touch_args();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t blk = P.remap == 2 ? xcd_chunked(blockIdx.x, P.xcd_shift)
                          : P.remap   ? pmd::xcd_remap(blockIdx.x, gridDim.x)
@@ -889,8 +969,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 
     const uint32_t nq = P.nq_dev ? min(P.nq, *P.nq_dev) : P.nq;
     const uint32_t u = blk * kWaves + wave;
     if (u >= nq || u >= P.n_waves) return;  // wave-uniform; no workgroup barriers below
-    stream_wave<CAP, kLists>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), lds[wave], threadIdx.x & 63, P.order,
-                             u, P.n_waves, 0u, wave_queries(u, P.n_waves, (uint32_t)P.gq, nq));
+    stream_wave<CAP, kLists, kOne>((ParamsPtr)__builtin_amdgcn_kernarg_segment_ptr(), lds[wave], threadIdx.x & 63,
+                                   P.order, u, P.n_waves, 0u, wave_queries(u, P.n_waves, (uint32_t)P.gq, nq));
 }
 
 // Neighbour lists of k = 513..2048 (and counts alone above k = 256): one wave
@@ -1085,7 +1165,7 @@ __device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, 
             found = 0;
             dmax = 0.f;
             if (!binned) {
-                walk_query(kp0, lane, W, lb, batch, false, hi,
+                walk_query<false>(kp0, lane, W, lb, batch, false, hi,
                            [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
                                const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi),
                                               bb = bm & wballot(__float_as_uint(d2b) < hi);
@@ -1101,7 +1181,7 @@ __device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, 
             wave_sync();
             // (a NaN product, when hi is 0 or denormal, gives bin 255)
             scale = 256.f * __builtin_amdgcn_rcpf(__uint_as_float(hi));
-            walk_query(kp0, lane, W, lb, batch, false, hi,
+            walk_query<false>(kp0, lane, W, lb, batch, false, hi,
                        [&](uint64_t am, uint32_t, float d2a, uint64_t bm, uint32_t, float d2b) {
                            const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi),
                                           bb = bm & wballot(__float_as_uint(d2b) < hi);
@@ -1133,7 +1213,7 @@ __device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, 
                 // exact, so the order is kept)
                 for (uint32_t e = lane; e < 256; e += 64) L.hist[e] = 0;
                 wave_sync();
-                walk_query(kp0, lane, W, lb, batch, false, hi,
+                walk_query<false>(kp0, lane, W, lb, batch, false, hi,
                            [&](uint64_t am, uint32_t, float d2a, uint64_t bm, uint32_t, float d2b) {
                                const float fa = fminf(d2a * scale, kBinTop), fb = fminf(d2b * scale, kBinTop);
                                const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot((uint32_t)fa == bin),
@@ -1151,7 +1231,7 @@ __device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, 
                 if (c > kWideList) return false;
             }
             uint32_t cnt = 0;
-            walk_query(kp0, lane, W, lb, batch, false, hi,
+            walk_query<false>(kp0, lane, W, lb, batch, false, hi,
                        [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
                            const float fa = fminf(d2a * scale, kBinTop), fb = fminf(d2b * scale, kBinTop);
                            uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot((uint32_t)fa == bin),
@@ -1233,7 +1313,7 @@ __device__ __forceinline__ bool wide_query(ParamsPtr kp0, const WaveQueries& W, 
             }
         };
         wave_sync();  // the list is read before the ring is written
-        walk_query(kp0, lane, W, lb, batch, false, hi,
+        walk_query<false>(kp0, lane, W, lb, batch, false, hi,
                    [&](uint64_t am, uint32_t sa, float d2a, uint64_t bm, uint32_t sb, float d2b) {
                        const uint64_t ka = make_key(d2a, sa), kb = make_key(d2b, sb);
                        const uint64_t ba = am & wballot(__float_as_uint(d2a) < hi) & wballot(ka <= kstar),
@@ -1316,7 +1396,7 @@ __device__ __forceinline__ void batch_wave(const KnnParams* __restrict__ jobs, c
     const uint32_t n_waves = kp->n_waves;
     const uint32_t qb = __builtin_amdgcn_readfirstlane(qbase[j]);
     const uint32_t first = __builtin_amdgcn_readfirstlane(u - wbase[j]);
-    stream_wave<512, kLists>(kp, L, threadIdx.x & 63, order, qb + first, n_waves, qb,
+    stream_wave<512, kLists, false>(kp, L, threadIdx.x & 63, order, qb + first, n_waves, qb,
                              wave_queries(first, n_waves, (uint32_t)kp->gq, kp->nq));
 }
 
@@ -1720,10 +1800,12 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
         hipLaunchKernelGGL((k_knn_stream<1024, false>), grid_dim, block, 0, ctx->stream, P);
     else if (flags & PM_KNN_LARGE_BUFFER)
         hipLaunchKernelGGL((k_knn_stream<1024, true>), grid_dim, block, 0, ctx->stream, P);
-    else if (lists)
-        hipLaunchKernelGGL((k_knn_stream<512, true>), grid_dim, block, 0, ctx->stream, P);
+    else if (P.gq == 1)
+        hipLaunchKernelGGL((lists ? k_knn_stream<512, true, true> : k_knn_stream<512, false, true>), grid_dim, block, 0,
+                           ctx->stream, P);
     else
-        hipLaunchKernelGGL((k_knn_stream<512, false>), grid_dim, block, 0, ctx->stream, P);
+        hipLaunchKernelGGL((lists ? k_knn_stream<512, true> : k_knn_stream<512, false>), grid_dim, block, 0,
+                           ctx->stream, P);
     PM_CHECK_LAUNCH(ctx, "k_knn");
     return PM_OK;
 }
