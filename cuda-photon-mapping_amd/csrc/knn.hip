@@ -1675,18 +1675,40 @@ pm_status setup(pm_ctx* ctx, const pm_grid* grid, const float* d_q, uint32_t nq,
 // The streaming gather's queries per wave, for a launch of `total` queries:
 // as many as their rows fit the wave's 64 lanes, while at least kFillWaves
 // waves remain (16 a SIMD's worth: below that the chip is not full and a
-// wave's queries would only run one after the other). Above k = 256 a query's
-// walk dwarfs its set-up and the buffer leaves fewer waves, so the last round
-// of long waves costs more than shared set-ups give: 60k queries, k = 500
-// 920 -> 706 us at 65536 waves instead of 16384, k = 1000 1888 -> 1635, a
+// wave's queries would only run one after the other), and not so that a few waves
+// are left over after two full rounds (8192 waves are resident).
+//
+// Estimates keep kFillUneven waves where several queries a wave give less than the
+// longest wave costs: with the inner box (no guessed bound; 131k queries in 16M
+// photons 376 us at 16384 waves, 318 at 49152, 351 with a set-up each), in
+// sorted launches on crowded maps (thousands of candidates, several such queries
+// end up in one wave: 65k queries in 3.78M photons, r = 0.047, 1107 and 705 us; in
+// 1M, r = 0.05, 315 and 265), and in unsorted ones where the guess saves little
+// (33k in 2M photons, r = 0.01, k = 100, 99 and 87; k = 32 in 16M, r = 0.005, 57 %
+// of the time at 16384). Lists, whose second bound is close, do not lose there.
+//
+// Above k = 256 a query's walk dwarfs its set-up and the buffer leaves fewer waves,
+// so the last round of long waves costs more than shared set-ups give: 60k queries,
+// k = 500 920 -> 706 us at 65536 waves instead of 16384, k = 1000 1888 -> 1635, a
 // 1024x768 frame's k = 2000 the same.
-constexpr uint32_t kFillWaves = 16384, kFillWavesLarge = 65536;
-void split_waves(KnnParams& P, uint64_t total) {
+constexpr uint32_t kFillWaves = 16384, kFillUneven = 49152, kFillWavesLarge = 65536;
+void split_waves(KnnParams& P, uint64_t total, bool sorted) {
     P.w = P.h > 0 ? P.h : P.rc;
     const int64_t side = 2 * (int64_t)P.w + 1, rows = side * side;
     P.nr = P.G.layout == PM_LAYOUT_LINEAR && rows <= 64 ? (int)rows : 0;
     const uint64_t fit = P.nr > 0 ? 64 / (uint64_t)P.nr : 1;
-    P.gq = (int)std::max<uint64_t>(1, std::min<uint64_t>(fit, total / (P.k > 256 ? kFillWavesLarge : kFillWaves)));
+    uint64_t fill = kFillWaves;
+    if (P.k > 256) {
+        fill = kFillWavesLarge;
+    } else if (!P.out_idx) {
+        // photons expected within the radius, were they even on the box's faces
+        const float e[3] = {(float)P.G.g[0] * P.G.cell, (float)P.G.g[1] * P.G.cell, (float)P.G.g[2] * P.G.cell};
+        const float within = 3.14f * P.r * P.r * (float)P.n / (2.f * (e[0] * e[1] + e[1] * e[2] + e[2] * e[0]));
+        if (P.h > 0 || (sorted ? fit > 2 && within > 900.f : within < 6.f * (float)P.k)) fill = kFillUneven;
+    }
+    uint64_t gq = std::min(fit, total / fill);
+    if (P.k <= 256 && total > gq * fill && 16 * total < 17 * gq * fill) gq = gq == 2 ? 1 : gq + 1 == fit ? fit : gq;
+    P.gq = (int)std::max<uint64_t>(1, gq);
     P.n_waves = pm::div_up(P.nq, (uint32_t)P.gq);
     // (a single query's wave would only wait for the second look-up of its
     // rows, 2000 queries 13 -> 18 us, but for long lists, whose second bound
@@ -1758,7 +1780,7 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
         pm_status st = pm::fill_u32(ctx, ovf_count, 0u, 1);
         if (st != PM_OK) return st;
         P.h = 0;  // (the inner box is the k <= 256 gathers')
-        split_waves(P, P.nq);
+        split_waves(P, P.nq, sort);
         uint32_t nblk = pm::div_up(P.n_waves, kWaves);
         P.xcd_shift = xcd_shift_for(nblk, (uint32_t)P.gq);
         if (P.remap == 2) nblk = xcd_round(nblk, P.xcd_shift);
@@ -1784,7 +1806,7 @@ pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags)
         return PM_OK;
     }
     const bool two_pass = !mid && (flags & PM_KNN_TWO_PASS);
-    if (!two_pass) split_waves(P, P.nq);
+    if (!two_pass) split_waves(P, P.nq, sort);
     uint32_t nblk = pm::div_up(two_pass ? P.nq : P.n_waves, kWaves);
     P.xcd_shift = xcd_shift_for(nblk, (uint32_t)P.gq);
     if (P.remap == 2) nblk = xcd_round(nblk, P.xcd_shift);
@@ -1969,7 +1991,7 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     uint64_t waves = 0;
     bool lists = false;
     for (KnnParams& P : hp) {
-        split_waves(P, total);
+        split_waves(P, total, (flags & PM_KNN_SORT_QUERIES) != 0);
         wbase.push_back((uint32_t)waves);
         waves += P.n_waves;
         lists |= P.out_idx != nullptr;
