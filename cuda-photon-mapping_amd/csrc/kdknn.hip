@@ -159,7 +159,9 @@ __device__ __forceinline__ float finish_query(KdPtr kp, WaveLds<CAP>& L, uint32_
 }
 
 // A query that the wave has no other beside: the walk of its ball by all 64
-// lanes, with `stk`, the idle group's memory, for its stack (top entries). All
+// lanes, with `stk`, the idle group's memory, for its stack (top entries). From
+// half the stack on it takes subtrees of five levels off its top, each one entry
+// for up to 32, while these leave the depth-first walk its kMaxLevels. All
 // else as in k_kd_knn, where a group walks; cnt and T are the query's, wave-uniform.
 template <int CAP>
 __device__ __forceinline__ void walk_alone(KdPtr kp0, WaveLds<CAP>& B, uint32_t* stk, uint32_t lane, uint32_t lev,
@@ -178,7 +180,8 @@ __device__ __forceinline__ void walk_alone(KdPtr kp0, WaveLds<CAP>& B, uint32_t*
         }
         uint32_t node = stk[lane < top ? top - 1u - lane : 0u];
         bool sub = top == 1;
-        if (top > kAll / 2) sub = __builtin_amdgcn_readfirstlane(node) < cap >> 4;
+        if (top > kAll / 2 && top + kGroup - 1u <= kAll - kMaxLevels)
+            sub = __builtin_amdgcn_readfirstlane(node) < cap >> 4;
         const uint32_t n = sub ? 1u : min(min(top, 64u), (uint32_t)max((int)(kAll - kMaxLevels - top), 1));
         if (sub) node = (__builtin_amdgcn_readfirstlane(node) << lev) + (lane & 31u);
         const uint64_t has = wballot(lane < (sub ? kGroup - 1u : n)) & wballot(node < cap);

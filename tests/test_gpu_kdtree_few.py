@@ -69,6 +69,24 @@ def test_lists(ctx, n, nq, r, k):
     assert np.array_equal(gd.cpu().numpy().view(np.uint32), od.view(np.uint32))
 
 
+def test_open_search_of_a_deep_tree(ctx):
+    """24 levels with every photon in one place, k for the smallest stack: all
+    nodes are opened. Subtrees of five levels, taken whatever room was left, filled
+    the stack past its end (613 entries of 608, counted on the CPU). The nearest are the first."""
+    import torch
+
+    n, nq, k = 8_400_000, 2, 64
+    ph = torch.full((9, n), 0.25, device="cuda")
+    q = np.array([[0.25, 0.3], [0.25, 0.25], [0.25, 0.25]], np.float32)
+    gi, gd, gc = ctx.kdtree_knn(ctx.kdtree_build(ph), q, 0.5, k)
+    ctx.sync()
+    d = (np.float32(0.25) - q[0]) * (np.float32(0.25) - q[0])
+    assert gc.tolist() == [k] * nq
+    assert gi.tolist() == [list(range(k))] * nq
+    for i in range(nq):
+        assert len(set(gd[i].tolist())) == 1 and abs(float(gd[i, 0]) - np.sqrt(d[i])) <= 1e-6
+
+
 @pytest.mark.parametrize("k", [1, 50])
 def test_queries_that_are_not_numbers_cost_nothing(ctx, k):
     """They walked the whole tree, 300k photons' in 83 ms; the others' walk
