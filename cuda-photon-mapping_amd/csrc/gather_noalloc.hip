@@ -18,7 +18,7 @@ namespace {
 
 constexpr uint32_t kMaxQueries = 1u << 20;  // 1,048,576 queries (a 1280x720 frame's hits fit)
 constexpr size_t kCounterBytes = 256;       // look-back tile counter and epoch word
-constexpr size_t kStateTiles = 256;         // look-back tile words (the sort's scans need 32 at the limit)
+constexpr size_t kStateTiles = 256;         // look-back tile words (the sort's scans need 16 at the limit)
 constexpr size_t kArenaBytes = 26u << 20;   // keys, order, radix passes, overflow list at the limit
 constexpr size_t kScratchBytes = kCounterBytes + kStateTiles * sizeof(uint64_t) + kArenaBytes;
 

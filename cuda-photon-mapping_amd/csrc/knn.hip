@@ -2,7 +2,8 @@
 //
 // Replaces PhotonGrid::find_nearests + PhotonMaxHeap (PhotonGrid.cu:222-284,
 // PhotonMaxHeap.cuh:90-107) and Raytracer::get_color_from_photon_grid
-// (Raytracer.cuh:110-138). One wave64 serves one query:
+// (Raytracer.cuh:110-138). A wave64 walks one query at a time, and a small
+// number of queries one after the other (stream_wave):
 //   1. the candidate box (query cell +- ceil(r/cell), clamped) is split into
 //      contiguous photon runs (one per (y,z) row of cells in the linear
 //      layout, one per cell in the Morton layout), one run per lane;
@@ -15,9 +16,11 @@
 //      float bits of d2 (two bins per octave) finds the smallest bin edge
 //      keeping >= k keys, the buffer is compacted to it and the acceptance
 //      bound tightens (a refinement splits a crowded bin 64 ways);
-//   4. a register bitonic sort across the wave orders the <= 256 survivors;
-//      the first k are the answer — the exact k smallest by (d2, slot);
-//   5. optionally the radiance estimate runs on those k in the same wave.
+//   4. lists: a counting sort over bins linear in d2 orders the survivors (at
+//      most 512 keys; k_knn_large's bitonic network sorts longer ones); the
+//      first k are the answer, the exact k smallest by (d2, slot);
+//   5. estimates: the buffer is narrowed to exactly those k, which the same
+//      wave sums unsorted (k_gather_wide, from k = 513 on, keeps no keys).
 // A two-pass variant (histogram pass, then collect pass) is kept selectable
 // for tuning.
 #include <algorithm>
@@ -518,8 +521,7 @@ __device__ __forceinline__ void finish(const KnnParams& P, WaveLds<CAP>& L, uint
 }
 
 // The candidate box of query q: its cell +- rc, clamped (PhotonGrid.cu:262-272).
-__device__ __forceinline__ void box_of(const KnnParams& P, uint32_t q, Box& B, float& qx, float& qy, float& qz,
-                                       int* cell = nullptr) {
+__device__ __forceinline__ void box_of(const KnnParams& P, uint32_t q, Box& B, float& qx, float& qy, float& qz) {
     // the query is the wave's: its coordinates (and so the box, the row
     // count and the cursor of walk) are wave-uniform, held in SGPRs
     qx = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(P.qx[q])));
@@ -531,7 +533,6 @@ __device__ __forceinline__ void box_of(const KnnParams& P, uint32_t q, Box& B, f
         int c = pmd::cell_coord(qv[a], P.G.mn[a], P.G.cell, P.G.g[a]);
         B.lo[a] = max(0, c - P.rc);
         B.hi[a] = min(P.G.g[a] - 1, c + P.rc);
-        if (cell) cell[a] = c;
     }
 }
 
@@ -664,7 +665,7 @@ __device__ __forceinline__ void push2(WaveLds<CAP>& L, uint32_t lane, ParamsPtr 
 // cells are pruned to that: on surfaces the photons within b are about
 // N / (1 + 0.6 cell / sqrt(b))^2 (the walked cells against the disc), evenly
 // in d2; `guess` = 1.2 (k + 3 sqrt(k) + 2) (split_waves) leaves three standard deviations
-// and a fifth for an uneven map. If the first walk finds at least k keys, the
+// and a fifth for an uneven map (lists of k <= 128 do without the fifth). If the first walk finds at least k keys, the
 // k smallest are the answer; otherwise the query walks the whole box again
 // from an empty buffer, to the radius or, for lists, first to a bound sized
 // from the count so far (next_bound). Every outcome is exact.
@@ -869,7 +870,7 @@ __device__ __forceinline__ void walk_query(ParamsPtr kp0, uint32_t lane, const W
 // hi): a squared radius that should hold half as many again as needed, where
 // that is well below the radius, else the radius. 3 % of the queries come
 // here, but a whole box is several times a guessed walk and the longest of a
-// wave's queries: 1M photons, 500k queries, k = 50, sorted rows of five cells:
+// wave's queries: 1M sorted queries in 4M photons, k = 50, cells of the radius:
 // 1262 -> 1141 us. The estimates' kernels walk the whole box at once: there
 // the loop's extra state costs the compiled walk 4 to 6 % (1480 -> 1537 us at a
 // 1280x720 frame), as much as the shorter walks give.
@@ -978,7 +979,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(CAP == 512 
 // the final selection narrows the buffer to exactly the k smallest keys, which
 // a bitonic network sorts in LDS. Up to k = 512 the stream with a 768-key buffer
 // and a register sort took its place: 2482 lists of k = 400 532 -> 194 us, 100k of
-// k = 300 2656 -> 694, of k = 512 4761 -> 1400.
+// k = 300 2656 -> 650, of k = 512 4761 -> 1185.
 template <int CAP>
 __device__ __forceinline__ void large_one(const KnnParams& P, WaveLds<CAP>& L, uint32_t lane, uint32_t q) {
     Box B;
@@ -1745,8 +1746,8 @@ pm_status query_order(pm_ctx* ctx, const pm_grid* grid, const KnnParams& P, uint
 
 pm_status launch(pm_ctx* ctx, const pm_grid* grid, KnnParams& P, uint32_t flags) {
     if (P.nq == 0) return PM_OK;
-    // radiance (and counts) without neighbour lists for k > 512: the
-    // three-walk kernel, with an overflow list behind it
+    // radiance (and counts) without neighbour lists for k > 512: k_gather_wide
+    // (up to four walks, no key buffer), with an overflow list behind it
     // (256 < k <= 512: one walk with the 768-key buffer)
     const bool mid = P.k > 256 && P.k <= 512 && (P.out_idx || P.rgb);
     const bool wide = P.k > 512 && !P.out_idx && P.rgb;
@@ -1942,9 +1943,9 @@ extern "C" pm_status pm_gather_batch(pm_ctx* ctx, const pm_gather_job* jobs, uin
     if (!ctx) return PM_ERR_INVALID;
     if (n_jobs == 0) return PM_OK;
     if (!jobs) return pm::fail(ctx, PM_ERR_INVALID, "pm_gather_batch: null job table");
-    // Jobs with k <= 256 share one launch of the batch kernel; larger k
-    // (one wave per query over a 2048/4096-entry LDS buffer) run as their own
-    // launches of the single-map kernel, first, on the same stream.
+    // Jobs with k <= 256 share one launch of the batch kernel; those of larger k
+    // run as their own launches of the single-map kernels, first, on the same
+    // stream.
     std::vector<KnnParams> hp;
     std::vector<std::pair<const pm_grid*, KnnParams>> large;
     std::vector<uint32_t> qbase, cell_base, wbase;
