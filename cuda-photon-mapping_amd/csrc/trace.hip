@@ -441,7 +441,7 @@ __device__ __forceinline__ void take_path(const TraceParams& P, const PathState*
 // Each lane traces one path a bounce at a time and, when it ends, takes the
 // list's next path from an LDS counter, so a wave keeps its lanes busy
 // instead of waiting on its longest path. Which lane traces a path does not
-// change the photons it stores. Bound by latency with four waves a SIMD (120
+// change the photons it stores. Bound by latency with four waves a SIMD (123
 // VGPRs; at five waves it spills and takes 1.5 times as long) and by the VALU:
 // the Cornell box's 2M + 500k photons take 0.65 + 0.87 ms here and 0.05 + 0.18
 // ms of emission, where the model-by-model walk with emission inside took
